@@ -313,9 +313,9 @@ void newmark_free(asend_ctx* ctx) {
 
 void ldl_release(asend_ctx* ctx) {
     dfree(ctx->ldl.L);
-    dfree(ctx->ldl.P);
     dfree(ctx->ldl.neg);
     dfree(ctx->ldl.work);
+    dfree(ctx->ldl.tmp);
     dfree(ctx->d_ldl_z);
     ctx->ldl = LdlFactor();
 }
@@ -486,8 +486,9 @@ int ldl_ensure(asend_ctx* ctx) {
                         "LDL^T factor of %lld blocks, band %lld: %.2f GB of device memory needed, %.2f GB free",
                         (long long)d.n_blocks, (long long)W, bytes / 1e9, free_b / 1e9);
         if ((rc = dalloc(ctx, &F.L, (size_t)d.n_blocks * d.stride)) ||
-            (rc = dalloc(ctx, &F.P, (size_t)d.n_blocks * kLdlTileElems)) || (rc = dalloc(ctx, &F.neg, 1)) ||
-            (rc = dalloc(ctx, &F.work, (size_t)ctx->n_dof)) ||
+            (rc = dalloc(ctx, &F.neg, 1)) ||
+            (rc = dalloc(ctx, &F.work, 3 * (size_t)ctx->n_dof)) ||
+            (rc = dalloc(ctx, &F.tmp, (size_t)ldl_tmp_tiles(d) * kLdlTileElems)) ||
             (rc = dalloc(ctx, &ctx->d_ldl_z, (size_t)ctx->n_dof))) {
             ldl_release(ctx);
             return rc;
@@ -499,7 +500,7 @@ int ldl_ensure(asend_ctx* ctx) {
     HIPCHK(hipStreamSynchronize(ctx->st));
     const auto t0 = std::chrono::steady_clock::now();
     ldl_fill(ctx->st, F.d, ctx->fine().n_rows, (int)ctx->n_slices, ctx->d_sptr, ctx->d_scol, ctx->d_K64, F.L);
-    ldl_factor_launch(ctx->st, F.d, F.L, F.P, F.neg);
+    ldl_factor_launch(ctx->st, F.d, F.L, F.tmp, F.neg);
     HIPCHK(hipGetLastError());
     int32_t neg = 0;
     HIPCHK(hipMemcpyAsync(&neg, F.neg, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->st));

@@ -11,22 +11,26 @@ namespace asend {
 
 constexpr int kLdlTile = 64;  // tile edge of the banded storage (DOFs)
 constexpr int kLdlTileElems = kLdlTile * kLdlTile;
-// Most tiles a tile row may hold below the diagonal: the solve keeps the last
-// kLdlMaxWt + 1 solution tiles of its block in LDS (64 doubles each).
+// Most tiles a tile row may hold below the diagonal (bands up to 15,360 DOFs).
 constexpr int kLdlMaxWt = 239;
-// Below this many blocks the solve runs one launch per tile row with the
-// tiles of a row spread over workgroups; from it on, one workgroup streams
-// each block (enough blocks to fill the chip).
-constexpr int kLdlStepBlocks = 64;
+// Super-blocks of the solve: the whole block where it has at most
+// kLdlWholeTiles tiles a side and the band covers it (one launch each way), else kLdlSuperTiles or as
+// many as the band holds.
+constexpr int kLdlWholeTiles = 16;
+constexpr int kLdlSuperTiles = 8;
+// Scratch tiles of the super-block inversion (128 MB; more pairs go in turns)
+constexpr int64_t kLdlTmpTiles = 4096;
 
 // Banded tile storage of the factor.  Block b covers DOFs [b bs, min((b+1) bs,
 // n)); inside a block, tile (I, J) (rows 64 I.., columns 64 J.., I - wt <= J
 // <= I) is 64 x 64 row-major at
 //   L + b stride + (row_off(I) + J - max(0, I - wt)) * 4096,
-// row_off(I) = sum over I' < I of (min(I', wt) + 1).  Diagonal tiles hold
-// D on their diagonal and the unit lower factor below it (the reference's
-// storage of d_i at the end of each row); rows past the block end are padded
-// with identity rows.
+// row_off(I) = sum over I' < I of (min(I', wt) + 1).  During the
+// factorization diagonal tiles take D on their diagonal and the inverse of
+// their unit lower factor below it (the panel multiplies by it); afterwards
+// the tiles (I, J) of every diagonal super-block (I / S = J / S, S =
+// ldl_super) hold the inverse of its unit lower factor, the others the
+// factor.  Rows past the block end are padded with identity rows.
 struct LdlDesc {
     int64_t n = 0;       // DOFs
     int64_t bs = 0;      // DOFs per block (the last block may be shorter)
@@ -55,9 +59,9 @@ struct LdlFactor {
     LdlDesc d;
     int64_t max_bandwidth = 0;  // the reference's maxBandwidth (row span incl. the diagonal)
     double* L = nullptr;        // banded tiles
-    double* P = nullptr;        // per block: D^-1 L_kk^-1 of the current step (panel scratch)
     int32_t* neg = nullptr;     // count of negative pivots (pos_def false when > 0)
-    double* work = nullptr;     // n doubles: the solve's work vector
+    double* work = nullptr;     // 3 n doubles: the solve's work vectors
+    double* tmp = nullptr;      // ldl_tmp_tiles tiles: scratch of the inversion
     int64_t asm_id = -1;        // assembly the factor was computed from
     int64_t bytes = 0;
     double factor_ms = 0.0;
@@ -75,10 +79,14 @@ const char* ldl_plan(LdlDesc* d, int64_t* max_bw, int64_t n_dof, int64_t block_d
 // envelope of each block), then factor them.  Every launch on st.
 void ldl_fill(hipStream_t st, const LdlDesc& d, int n_rows, int n_slices, const int32_t* sptr, const int32_t* scol,
               const double* K, double* L);
-void ldl_factor_launch(hipStream_t st, const LdlDesc& d, double* L, double* P, int32_t* neg);
+void ldl_factor_launch(hipStream_t st, const LdlDesc& d, double* L, double* tmp, int32_t* neg);
+
+// Tiles per super-block side, and the scratch tiles its inversion needs.
+int ldl_super(const LdlDesc& d);
+int64_t ldl_tmp_tiles(const LdlDesc& d);
 
 // x = (L D L^T)^-1 b over every block (ldl_solve).  x may alias b; work is
-// n doubles of scratch (distinct from both).  When done is given and *done
+// 3 n doubles of scratch (distinct from both).  When done is given and *done
 // is set the launches do nothing (solver loops).
 void ldl_solve_launch(hipStream_t st, const LdlDesc& d, const double* L, const double* b, double* x, double* work,
                       const int* done);

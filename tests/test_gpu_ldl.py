@@ -57,6 +57,22 @@ def test_block_factor_solve_matches_oracle(ctx, name, blocks):
         assert rel_err(x, x_ref) <= 1e-10, (info, rel_err(x, x_ref))
 
 
+# super-block edges of the solve: a band of one or two tiles, of seven or more
+# (eight-tile super-blocks, a last one cut short), blocks of exactly 16 tiles
+# (one super-block) and of 17, and a last block of one tile
+@pytest.mark.parametrize("mesh, blocks", [((60, 1, 1), 0), ((40, 3, 4), 0), ((8, 12, 12), 0), ((3, 12, 12), 0),
+                                          ((5, 12, 12), 1024), ((5, 12, 12), 1030), ((5, 12, 12), 1500)])
+def test_super_block_edges(ctx, mesh, blocks):
+    p = problems.heterogeneous(*mesh, seed=21, block_dim=2000000000)
+    gpu_case(f"ldl super-blocks {mesh} blocks={blocks}")
+    K, sf = solid_system(ctx, p)
+    ctx.ldl_factor(blocks)
+    ref = O.LDL(K, p.pen_dofs, sf, blocks if blocks else p.n_dof)
+    for b in (p.f, np.random.default_rng(4).standard_normal(p.n_dof)):
+        x, x_ref = ctx.ldl_solve(b), ref.solve(b)
+        assert rel_err(x, x_ref) <= 1e-10, rel_err(x, x_ref)
+
+
 def test_direct_solve_is_exact(ctx):
     p = solid("het-12x6x6 distorted")
     gpu_case("direct solve het-12x6x6 distorted")
