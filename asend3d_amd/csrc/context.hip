@@ -3178,6 +3178,8 @@ int asend_learned_train(asend_ctx* ctx, int n_steps, float lr, uint64_t seed, in
     // a V-cycle solution of a random load; mode 3 puts a Gaussian sample
     // before every such pair
     const bool solver_samples = (mode == 1 || mode == 3);
+    if (mode != 2 && n_steps > 0 && (rc0 = learned_train_begin(ctx->learned, ctx->st, g)))
+        return fail(ctx, rc0, "%s", learned_error(ctx->learned));
     double ema = 0.0;  // running level of the accepted mode-2 losses
     for (int k = 0; k < n_steps; ++k) {
         const uint64_t s = seed * 1000003ull + (uint64_t)k;

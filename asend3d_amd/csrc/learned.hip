@@ -45,7 +45,8 @@ __device__ __forceinline__ bf16 f2bf(float f) {
 }
 
 constexpr int kNodesPerWave = 32;
-constexpr int kWgChunk = 1024;  // nodes per block of the weight-gradient kernel
+constexpr int kWgChunk = 256;   // nodes per block of the weight-gradient kernel
+constexpr int kOuterBlocks = 256;  // most blocks of the small weight gradients
 constexpr int kHeadPad = 32;    // head rows padded to one MFMA tile
 constexpr float kExpClamp = 10.f;
 constexpr int kMaxPairs = 2 * kMaxUses;  // outer-product pairs of one gradient
@@ -209,7 +210,8 @@ __global__ __launch_bounds__(256) void k_aggregate(int n, const int32_t* __restr
 // Node GEMM on MFMA: out[node][col] = sum_k Arow[node][k] W[col][k] (+ epilogue)
 //   Arow = [A1[node][0..K1) | A2[node][0..KA-K1)], BF16; W is BF16 [N][KA].
 //   MODE 0: out BF16 [n][N] = relu(acc + bias)
-//   MODE 1: out FP32 [n][N] = acc
+//   MODE 1: out FP32 [n][N] = acc, columns >= N / 2 divided by the node's neighbour count
+//     (rp): the mean's factor, once per value instead of in every gather of it
 //   MODE 2: out FP32 [n][kHead] = acc + bias, columns < kHead only
 // One wavefront owns 32 nodes and all N columns (N/32 accumulator tiles of
 // v_mfma_f32_32x32x16_bf16); its A fragments stay in registers across tiles.
@@ -218,7 +220,7 @@ __global__ __launch_bounds__(256) void k_aggregate(int n, const int32_t* __restr
 template <int KA, int K1, int N, int MODE>
 __global__ __launch_bounds__(256) void k_node_gemm(int n, const bf16* __restrict__ A1, const bf16* __restrict__ A2,
                                                    const bf16* __restrict__ W, const float* __restrict__ bias,
-                                                   void* __restrict__ out) {
+                                                   const int32_t* __restrict__ rp, void* __restrict__ out) {
     const int lane = threadIdx.x % 64;
     const int node0 = (blockIdx.x * 4 + threadIdx.x / 64) * kNodesPerWave;
     if (node0 >= n) return;
@@ -252,7 +254,12 @@ __global__ __launch_bounds__(256) void k_node_gemm(int n, const bf16* __restrict
             if (MODE == 0) {
                 ((bf16*)out)[(int64_t)N * row + col] = f2bf(fmaxf(acc[v] + bcol, 0.f));
             } else if (MODE == 1) {
-                ((float*)out)[(int64_t)N * row + col] = acc[v];
+                float o = acc[v];
+                if (col >= N / 2) {
+                    const int deg = rp[row + 1] - rp[row] - 1;
+                    o = deg > 0 ? o / (float)deg : 0.f;
+                }
+                ((float*)out)[(int64_t)N * row + col] = o;
             } else if (col < kHead) {
                 ((float*)out)[(int64_t)kHead * row + col] = acc[v] + bcol;
             }
@@ -575,40 +582,107 @@ __global__ __launch_bounds__(256) void k_head_back(int n, const float* __restric
     dH[(int64_t)kHid * node + c] = s;
 }
 
-// Per-block partial sums over node chunks of
-//   g[row * ncol + col] = sum_node U[node][row] * V[node][col]   and
-//   g[nrow * ncol + row] = sum_node U[node][row]                 (bias rows)
-// U is FP32 [n][nrow]; V is FP32 (vkind 0) or BF16 (vkind 1) [n][ncol].
-__global__ __launch_bounds__(256) void k_small_wgrad(int n, int nrow, int ncol, const float* __restrict__ U,
-                                                     const void* __restrict__ V, int vkind,
-                                                     float* __restrict__ partials) {
-    const int np = nrow * ncol + nrow;
+// Per-block column sums of a [n][81] array over the block's nodes: 243 threads
+// take three whole rows a step, so thread t always holds column t % 81 and the
+// loads are contiguous.
+__global__ __launch_bounds__(256) void k_col_sums81(int n, const float* __restrict__ U, float* __restrict__ partials) {
+    __shared__ float sh[243];
     const int chunk = (n + gridDim.x - 1) / gridDim.x;
-    const int n0 = blockIdx.x * chunk, n1 = min(n, n0 + chunk);
-    for (int p = threadIdx.x; p < np; p += blockDim.x) {
-        float s = 0.f;
-        if (p < nrow * ncol) {
-            const int row = p / ncol, col = p % ncol;
-            for (int i = n0; i < n1; ++i) {
-                float v = vkind ? bf2f(((const bf16*)V)[(int64_t)ncol * i + col])
-                                : ((const float*)V)[(int64_t)ncol * i + col];
-                s += U[(int64_t)nrow * i + row] * v;
-            }
-        } else {
-            const int row = p - nrow * ncol;
-            for (int i = n0; i < n1; ++i) s += U[(int64_t)nrow * i + row];
-        }
-        partials[(int64_t)np * blockIdx.x + p] = s;
+    const int64_t e0 = 81 * (int64_t)min(n, (int)blockIdx.x * chunk);
+    const int64_t e1 = 81 * (int64_t)min(n, ((int)blockIdx.x + 1) * chunk);
+    const int t = threadIdx.x;
+    float s = 0.f;
+    if (t < 243) {
+#pragma unroll 4
+        for (int64_t e = e0 + t; e < e1; e += 243) s += U[e];
+        sh[t] = s;
     }
+    __syncthreads();
+    if (t < 81) partials[81 * (int64_t)blockIdx.x + t] = sh[t] + sh[t + 81] + sh[t + 162];
 }
 
-// g[p] = sum_b partials[b][p]  (fixed order: deterministic)
-__global__ void k_reduce_partials(int nparts, int np, const float* __restrict__ partials, float* __restrict__ g) {
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= np) return;
+// Per-block partial sums over the block's nodes of the outer products of a
+// 64-wide array (one lane per entry) and an NR-wide one (entries broadcast
+// from LDS), NR / 4 of the latter per wavefront:
+//   HEAD: g[r][c] = sum dO[node][r] H[node][c], r < NR = 24, c < 64, bias sum dO
+//   else: g[r][c] = sum dz0[node][r] X[node][c], r < 64, c < NR = 8, bias sum dz0
+// Slabs of 32 nodes go through LDS.  One output per thread and the nodes read
+// straight from memory by 64 blocks took 686 us a launch over 58,719 nodes,
+// with every thread on a chain of single loads; 256 blocks of this: 36 us (HEAD)
+// and 26 us.
+template <int NR, bool HEAD>
+__global__ __launch_bounds__(256) void k_outer_wgrad(int n, const float* __restrict__ U, const void* __restrict__ V,
+                                                     float* __restrict__ partials) {
+    constexpr int kSlab = 32, R = NR / 4;
+    constexpr int np = NR * kHid + (HEAD ? NR : kHid);
+    __shared__ float sw[kSlab][kHid];
+    __shared__ float sn[kSlab][NR];
+    const int chunk = (n + gridDim.x - 1) / gridDim.x;
+    const int n0 = min(n, (int)blockIdx.x * chunk), n1 = min(n, n0 + chunk);
+    const int t = threadIdx.x, c = t & 63, w = t >> 6;
+    float acc[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[r] = 0.f;
+    float bias = 0.f;
+    for (int base = n0; base < n1; base += kSlab) {
+        const int m = min(kSlab, n1 - base);
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < kSlab * kHid / 256; ++h) {
+            const int e = t + 256 * h;
+            float v = 0.f;
+            if (e < m * kHid)
+                v = HEAD ? bf2f(((const bf16*)V)[(int64_t)kHid * base + e]) : U[(int64_t)kHid * base + e];
+            sw[e / kHid][e % kHid] = v;
+        }
+#pragma unroll
+        for (int h = 0; h < (kSlab * NR + 255) / 256; ++h) {
+            const int e = t + 256 * h;
+            if (e < kSlab * NR) {
+                float v = 0.f;
+                if (e < m * NR) v = HEAD ? U[(int64_t)NR * base + e] : ((const float*)V)[(int64_t)NR * base + e];
+                sn[e / NR][e % NR] = v;
+            }
+        }
+        __syncthreads();
+#pragma unroll 8
+        for (int i = 0; i < kSlab; ++i) {
+            const float x = sw[i][c];
+#pragma unroll
+            for (int r = 0; r < R; ++r) acc[r] += sn[i][R * w + r] * x;
+        }
+        if (t < (HEAD ? NR : kHid))
+#pragma unroll 8
+            for (int i = 0; i < kSlab; ++i) bias += HEAD ? sn[i][t] : sw[i][t];
+    }
+    float* P = partials + (int64_t)np * blockIdx.x;
+#pragma unroll
+    for (int r = 0; r < R; ++r) P[HEAD ? (R * w + r) * kHid + c : c * NR + R * w + r] = acc[r];
+    if (t < (HEAD ? NR : kHid)) P[NR * kHid + t] = bias;
+}
+
+// g[p] = sum_b partials[b][p]: 64 parameters per block, four wavefronts over
+// the partials, added in a fixed order (deterministic)
+__global__ __launch_bounds__(256) void k_reduce_partials(int nparts, int np, const float* __restrict__ partials,
+                                                         float* __restrict__ g) {
+    __shared__ float sh[4][64];
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + l;
     float s = 0.f;
-    for (int b = 0; b < nparts; ++b) s += partials[(int64_t)np * b + p];
-    g[p] = s;
+    if (p < np) {
+        int b = w;
+        for (; b + 28 < nparts; b += 32) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = partials[(int64_t)np * (b + 4 * u) + p];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s += v[u];
+        }
+        for (; b < nparts; b += 4) s += partials[(int64_t)np * b + p];
+    }
+    sh[w][l] = s;
+    __syncthreads();
+    if (w == 0 && p < np) g[p] = sh[0][l] + sh[1][l] + sh[2][l] + sh[3][l];
 }
 
 // dz = bf16(dH * [h_out > 0])
@@ -627,42 +701,61 @@ __global__ void k_relu_back_f32(int64_t m, const float* __restrict__ dH, const b
 
 // Weight gradient on MFMA: dW[o][i] (64 x 128) = sum_node dz[node][o] * X[node][i],
 // X = [Hin | Ain]; db[o] = sum_node dz[node][o].  Each block reduces one chunk
-// of nodes, staging 16-node slabs of dz and X in LDS; its 8 output tiles are
-// split over the 4 wavefronts (wave w: rows 32 (w/2).., columns 64 (w%2)..).
-// Per-block partials are summed afterwards in a fixed order.
+// of nodes in slabs of 64, transposed into LDS (feature rows, two nodes to a
+// word) so that a lane's eight consecutive nodes of one feature, its operand of a
+// 16-node step, are one 16-byte read; its 8 output tiles are split over the 4
+// wavefronts (wave w: rows 32 (w/2).., columns 64 (w%2)..).  Per-block partials
+// are summed afterwards in a fixed order.
+//
+// Reads 22 MB on 58,719 nodes.  16-node slabs staged two bytes at a time by 58
+// blocks took 296 us; 230 blocks of 16-byte loads: 10 us.
+constexpr int kWgSlab = 64;
+constexpr int kWgRow = kWgSlab + 8;  // LDS row of a feature: 16-byte aligned, 8 lanes of a read in different banks
 __global__ __launch_bounds__(256) void k_wgrad_mfma(int n, const bf16* __restrict__ dz, const bf16* __restrict__ Hin,
                                                     const bf16* __restrict__ Ain, float* __restrict__ partials) {
-    __shared__ bf16 sdz[16][kHid];
-    __shared__ bf16 sx[16][2 * kHid];
+    __shared__ __align__(16) bf16 sT[3 * kHid][kWgRow];  // dz, Hin, Ain features
     __shared__ float sdb[4][kHid];
-    const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
+    const int t = threadIdx.x, lane = t % 64, w = t / 64;
     const int n0 = blockIdx.x * kWgChunk, n1 = min(n, n0 + kWgChunk);
     const int to = w / 2;
     const int kq = 8 * (lane / 32);
     f32x16 acc0 = {0}, acc1 = {0};
     float dbp = 0.f;
-    for (int base = n0; base < n1; base += 16) {
+    for (int base = n0; base < n1; base += kWgSlab) {
+        // thread: 8 features (oct) of nodes 2 pair, 2 pair + 1 of each array
+        const int oct = t & 7, pair = t >> 3;
+        const int node = base + 2 * pair;
+        bf16x8 v[3][2];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const bf16* src = (q == 0 ? dz : (q == 1 ? Hin : Ain)) + 8 * oct;
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                v[q][u] = node + u < n1 ? *(const bf16x8*)(src + (int64_t)kHid * (node + u))
+                                        : bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+        }
         __syncthreads();
-        for (int t = threadIdx.x; t < 16 * kHid; t += 256) {
-            int rr = t / kHid, c = t % kHid, node = base + rr;
-            sdz[rr][c] = node < n1 ? dz[(int64_t)kHid * node + c] : (bf16)0;
-        }
-        for (int t = threadIdx.x; t < 16 * 2 * kHid; t += 256) {
-            int rr = t / (2 * kHid), c = t % (2 * kHid), node = base + rr;
-            bf16 v = 0;
-            if (node < n1) v = c < kHid ? Hin[(int64_t)kHid * node + c] : Ain[(int64_t)kHid * node + (c - kHid)];
-            sx[rr][c] = v;
-        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                *reinterpret_cast<uint32_t*>(&sT[kHid * q + 8 * oct + i][2 * pair]) =
+                    (uint32_t)(uint16_t)v[q][0][i] | ((uint32_t)(uint16_t)v[q][1][i] << 16);
         __syncthreads();
-        for (int rr = 4 * w; rr < 4 * w + 4; ++rr) dbp += bf2f(sdz[rr][lane]);
-        bf16x8 a, b0, b1;
-        for (int i = 0; i < 8; ++i) {
-            a[i] = (short)sdz[kq + i][32 * to + lane % 32];
-            b0[i] = (short)sx[kq + i][64 * (w % 2) + lane % 32];
-            b1[i] = (short)sx[kq + i][64 * (w % 2) + 32 + lane % 32];
+        {
+            const bf16x8 d0 = *(const bf16x8*)&sT[lane][16 * w], d1 = *(const bf16x8*)&sT[lane][16 * w + 8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) dbp += bf2f((bf16)d0[i]) + bf2f((bf16)d1[i]);
         }
-        acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b0, acc0, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b1, acc1, 0, 0, 0);
+#pragma unroll
+        for (int s = 0; s < kWgSlab / 16; ++s) {
+            const int k = 16 * s + kq;
+            const bf16x8 a = *(const bf16x8*)&sT[32 * to + lane % 32][k];
+            const bf16x8 b0 = *(const bf16x8*)&sT[kHid + 64 * (w % 2) + lane % 32][k];
+            const bf16x8 b1 = *(const bf16x8*)&sT[kHid + 64 * (w % 2) + 32 + lane % 32][k];
+            acc0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b0, acc0, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b1, acc1, 0, 0, 0);
+        }
     }
     float* P = partials + (int64_t)kLayerSize * blockIdx.x;
     const int i0 = 64 * (w % 2) + lane % 32;
@@ -678,19 +771,42 @@ __global__ __launch_bounds__(256) void k_wgrad_mfma(int n, const bf16* __restric
             sdb[0][threadIdx.x] + sdb[1][threadIdx.x] + sdb[2][threadIdx.x] + sdb[3][threadIdx.x];
 }
 
-// dHin = dX[:, :64] + aggregation^T(dX[:, 64:])
+// dHin = dX[:, :64] + aggregation^T(dX[:, 64:]), the latter already over the
+// neighbour counts.  16 lanes per node and 16 bytes per lane (a wavefront
+// gathers a 256 B row for each of its 4 nodes per load), four neighbour rows
+// in flight, added in row order; one float per lane and one row at a time took
+// 137 us on 58,719 nodes, this 27 us.
 __global__ __launch_bounds__(256) void k_agg_back(int n, const int32_t* __restrict__ rp, const int32_t* __restrict__ bc,
                                                   const float* __restrict__ dX, float* __restrict__ dH) {
-    int node = blockIdx.x * 4 + threadIdx.x / 64, c = threadIdx.x % 64;
+    const int node = blockIdx.x * (256 / kAggLanes) + threadIdx.x / kAggLanes;
+    const int c = 4 * (threadIdx.x % kAggLanes);
     if (node >= n) return;
-    float s = dX[(int64_t)2 * kHid * node + c];
-    for (int k = rp[node]; k < rp[node + 1]; ++k) {
-        int i = bc[k];
-        if (i == node) continue;
-        int deg = rp[i + 1] - rp[i] - 1;
-        s += dX[(int64_t)2 * kHid * i + kHid + c] / (float)deg;
+    auto row = [&](int i) { return *reinterpret_cast<const float4*>(dX + (int64_t)2 * kHid * i + kHid + c); };
+    float4 s = *reinterpret_cast<const float4*>(dX + (int64_t)2 * kHid * node + c);
+    auto add = [&](float4 v) {
+        s.x += v.x;
+        s.y += v.y;
+        s.z += v.z;
+        s.w += v.w;
+    };
+    int k = rp[node];
+    const int end = rp[node + 1];
+    for (; k + 4 <= end; k += 4) {
+        int j[4];
+        float4 h[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) j[u] = bc[k + u];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) h[u] = row(j[u]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (j[u] != node) add(h[u]);
     }
-    dH[(int64_t)kHid * node + c] = s;
+    for (; k < end; ++k) {
+        const int j = bc[k];
+        if (j != node) add(row(j));
+    }
+    *reinterpret_cast<float4*>(dH + (int64_t)kHid * node + c) = s;
 }
 
 // Adam on the FP32 master parameters
@@ -854,8 +970,9 @@ int ensure_cap(Learned* lp, int n, int W) {
     LCHK(hipMalloc((void**)&lp->Gea, c * 81 * sizeof(float)));
     for (float** q : {&lp->e, &lp->r, &lp->t, &lp->y, &lp->w, &lp->u})
         LCHK(hipMalloc((void**)q, c * 3 * sizeof(float)));
-    const int nwg = std::max(blocks_for(n, kWgChunk), 64);
-    LCHK(hipMalloc((void**)&lp->wpart, (size_t)nwg * kLayerSize * sizeof(float)));
+    const size_t n_wpart = std::max((size_t)blocks_for(n, kWgChunk) * kLayerSize,
+                                    (size_t)kOuterBlocks * (kHead * kHid + kHead));
+    LCHK(hipMalloc((void**)&lp->wpart, n_wpart * sizeof(float)));
     LCHK(hipMalloc((void**)&lp->pairbuf, (size_t)2 * kMaxUses * c * 3 * sizeof(float)));
     lp->cap = n;
     lp->cap_w = W;
@@ -877,7 +994,9 @@ Factor factor_of(const Learned* lp, const LearnedGraph& g) {
     return F;
 }
 
-void forward(Learned* lp, hipStream_t st, const LearnedGraph& g) {
+// The graph's own data: node features, inverse Cholesky factors of the
+// diagonal blocks and scaled couplings (no parameter enters).
+void forward_graph(Learned* lp, hipStream_t st, const LearnedGraph& g) {
     const int n = g.n_nodes, W = g.n_edge;
     const int nb = blocks_for(n, 256);
     hipLaunchKernelGGL(k_features, dim3(nb), dim3(256), 0, st, n, g.rp, g.n2e_ptr, g.n2e, g.E, g.mean_log_e,
@@ -885,6 +1004,13 @@ void forward(Learned* lp, hipStream_t st, const LearnedGraph& g) {
     hipLaunchKernelGGL(k_prep_ci, dim3(nb), dim3(256), 0, st, n, g.op.sptr, g.K32, g.kdiag, lp->Ci);
     hipLaunchKernelGGL(k_prep_ahat, dim3(nb), dim3(256), 0, st, n, W, g.enb, g.eslot, g.op.sptr, g.K32, lp->Ci,
                        lp->Ahat);
+}
+
+// Network and factor over forward_graph's data; smoother: also the FP16 copies
+// the smoother reads (training needs none).
+void forward(Learned* lp, hipStream_t st, const LearnedGraph& g, bool smoother) {
+    const int n = g.n_nodes, W = g.n_edge;
+    const int nb = blocks_for(n, 256);
     hipLaunchKernelGGL(k_layer0, dim3(blocks_for(n, 4)), dim3(256), 0, st, n, lp->X, lp->wbf + kOffW0,
                        lp->p + kOffB0, lp->H[0]);
     const int gb = blocks_for(n, 4 * kNodesPerWave);
@@ -893,13 +1019,14 @@ void forward(Learned* lp, hipStream_t st, const LearnedGraph& g) {
                            lp->H[l], lp->A[l]);
         const int off = kOffL1 + l * kLayerSize;
         hipLaunchKernelGGL((k_node_gemm<2 * kHid, kHid, kHid, 0>), dim3(gb), dim3(256), 0, st, n, lp->H[l], lp->A[l],
-                           lp->wbf + off, lp->p + off + kHid * 2 * kHid, (void*)lp->H[l + 1]);
+                           lp->wbf + off, lp->p + off + kHid * 2 * kHid, (const int32_t*)nullptr, (void*)lp->H[l + 1]);
     }
     hipLaunchKernelGGL((k_node_gemm<kHid, kHid, kHeadPad, 2>), dim3(gb), dim3(256), 0, st, n, lp->H[kLayers],
-                       lp->H[kLayers], lp->whp, lp->p + kOffBh, (void*)lp->O);
+                       lp->H[kLayers], lp->whp, lp->p + kOffBh, (const int32_t*)nullptr, (void*)lp->O);
     hipLaunchKernelGGL(k_factor, dim3(nb), dim3(256), 0, st, n, W, lp->O, lp->Ci, lp->Ahat, g.enb, lp->wbf + kOffWa,
                        lp->Ls);
     hipLaunchKernelGGL(k_factor_transpose, dim3(nb), dim3(256), 0, st, n, W, lp->Ls, g.enb, g.erev, lp->LsT);
+    if (!smoother) return;
     hipLaunchKernelGGL(k_factor_to16, dim3(nb), dim3(256), 0, st, n, W, lp->Ls, lp->Ls16, lp->sc16);
     hipLaunchKernelGGL(k_factor_to16, dim3(nb), dim3(256), 0, st, n, W, lp->LsT, lp->LsT16, lp->scT16);
 }
@@ -943,15 +1070,16 @@ void backward_from_pairs(Learned* lp, hipStream_t st, const LearnedGraph& g, con
                        lp->DOE, lp->Gea);
     hipLaunchKernelGGL(k_grad_to, dim3(nb), dim3(256), 0, st, n, W, g.enb, g.erev, lp->DOE, lp->dO);
     // edge map Wa: column sums of Gea
-    const int nsb = 64;
-    hipLaunchKernelGGL(k_small_wgrad, dim3(nsb), dim3(256), 0, st, n, 81, 0, lp->Gea, (const void*)nullptr, 0,
-                       lp->wpart);
-    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(128), 0, st, nsb, 81, lp->wpart, lp->g + kOffWa);
+    const int nsb = std::min(kOuterBlocks, blocks_for(n, 32));
+    auto reduce = [&](int nparts, int np, float* gout) {
+        hipLaunchKernelGGL(k_reduce_partials, dim3(blocks_for(np, 64)), dim3(256), 0, st, nparts, np, lp->wpart, gout);
+    };
+    hipLaunchKernelGGL(k_col_sums81, dim3(nsb), dim3(256), 0, st, n, lp->Gea, lp->wpart);
+    reduce(nsb, 81, lp->g + kOffWa);
     // head
-    hipLaunchKernelGGL(k_small_wgrad, dim3(nsb), dim3(256), 0, st, n, kHead, kHid, lp->dO,
-                       (const void*)lp->H[kLayers], 1, lp->wpart);
-    hipLaunchKernelGGL(k_reduce_partials, dim3(blocks_for(kHead * kHid + kHead, 256)), dim3(256), 0, st, nsb,
-                       kHead * kHid + kHead, lp->wpart, lp->g + kOffWh);
+    hipLaunchKernelGGL((k_outer_wgrad<kHead, true>), dim3(nsb), dim3(256), 0, st, n, lp->dO,
+                       (const void*)lp->H[kLayers], lp->wpart);
+    reduce(nsb, kHead * kHid + kHead, lp->g + kOffWh);
     hipLaunchKernelGGL(k_head_back, dim3(blocks_for(n, 4)), dim3(256), 0, st, n, lp->dO, lp->wbf + kOffWh, lp->dH);
     // message-passing layers
     const int gb = blocks_for(n, 4 * kNodesPerWave);
@@ -961,19 +1089,18 @@ void backward_from_pairs(Learned* lp, hipStream_t st, const LearnedGraph& g, con
                            (int64_t)n * kHid, lp->dH, lp->H[l + 1], lp->dz);
         hipLaunchKernelGGL(k_wgrad_mfma, dim3(nwg), dim3(256), 0, st, n, lp->dz, lp->H[l], lp->A[l], lp->wpart);
         const int off = kOffL1 + l * kLayerSize;
-        hipLaunchKernelGGL(k_reduce_partials, dim3(blocks_for(kLayerSize, 256)), dim3(256), 0, st, nwg, kLayerSize,
-                           lp->wpart, lp->g + off);
+        reduce(nwg, kLayerSize, lp->g + off);
         hipLaunchKernelGGL((k_node_gemm<kHid, kHid, 2 * kHid, 1>), dim3(gb), dim3(256), 0, st, n, lp->dz, lp->dz,
-                           lp->wcatT + (int64_t)l * 2 * kHid * kHid, (const float*)nullptr, (void*)lp->dX);
-        hipLaunchKernelGGL(k_agg_back, dim3(blocks_for(n, 4)), dim3(256), 0, st, n, g.rp, g.bc, lp->dX, lp->dH);
+                           lp->wcatT + (int64_t)l * 2 * kHid * kHid, (const float*)nullptr, g.rp, (void*)lp->dX);
+        hipLaunchKernelGGL(k_agg_back, dim3(blocks_for(n, 256 / kAggLanes)), dim3(256), 0, st, n, g.rp, g.bc, lp->dX,
+                           lp->dH);
     }
     // layer 0
     hipLaunchKernelGGL(k_relu_back_f32, dim3(blocks_for((int64_t)n * kHid, 256)), dim3(256), 0, st,
                        (int64_t)n * kHid, lp->dH, lp->H[0], lp->dz0);
-    hipLaunchKernelGGL(k_small_wgrad, dim3(nsb), dim3(256), 0, st, n, kHid, kFeat, lp->dz0, (const void*)lp->X, 0,
+    hipLaunchKernelGGL((k_outer_wgrad<kFeat, false>), dim3(nsb), dim3(256), 0, st, n, lp->dz0, (const void*)lp->X,
                        lp->wpart);
-    hipLaunchKernelGGL(k_reduce_partials, dim3(blocks_for(kHid * kFeat + kHid, 256)), dim3(256), 0, st, nsb,
-                       kHid * kFeat + kHid, lp->wpart, lp->g + kOffW0);
+    reduce(nsb, kHid * kFeat + kHid, lp->g + kOffW0);
 }
 
 void adam_step(Learned* lp, hipStream_t st, float lr) {
@@ -1071,7 +1198,8 @@ int learned_set_params(Learned* lp, const float* host, int n) {
 int learned_infer(Learned* lp, hipStream_t st, const LearnedGraph& g, Factor* F) {
     int rc = check_graph(lp, g);
     if (rc || (rc = ensure_cap(lp, g.n_nodes, g.n_edge))) return rc;
-    forward(lp, st, g);
+    forward_graph(lp, st, g);
+    forward(lp, st, g, true);
     LCHK(hipGetLastError());
     *F = factor_of(lp, g);
     return ASEND_OK;
@@ -1081,11 +1209,17 @@ void learned_sample(hipStream_t st, const LearnedGraph& g, uint64_t seed, float*
     hipLaunchKernelGGL(k_randn, dim3(kVecBlocks), dim3(256), 0, st, g.n_nodes, seed, g.clamped, d_e);
 }
 
-int learned_train_step(Learned* lp, hipStream_t st, const LearnedGraph& g, const float* d_e, uint64_t sample_seed,
-                       float lr, double* loss_out) {
+int learned_train_begin(Learned* lp, hipStream_t st, const LearnedGraph& g) {
     int rc = check_graph(lp, g);
     if (rc || (rc = ensure_cap(lp, g.n_nodes, g.n_edge))) return rc;
-    forward(lp, st, g);
+    forward_graph(lp, st, g);
+    LCHK(hipGetLastError());
+    return ASEND_OK;
+}
+
+int learned_train_step(Learned* lp, hipStream_t st, const LearnedGraph& g, const float* d_e, uint64_t sample_seed,
+                       float lr, double* loss_out) {
+    forward(lp, st, g, false);
     if (d_e) LCHK(hipMemcpyAsync(lp->e, d_e, 3 * (size_t)g.n_nodes * sizeof(float), hipMemcpyDeviceToDevice, st));
     else learned_sample(st, g, sample_seed, lp->e);
     loss_and_backward(lp, st, g);
@@ -1145,7 +1279,8 @@ int learned_eval(Learned* lp, hipStream_t st, const LearnedGraph& g, const float
                  float* h_feat, float* h_out) {
     int rc = check_graph(lp, g);
     if (rc || (rc = ensure_cap(lp, g.n_nodes, g.n_edge))) return rc;
-    forward(lp, st, g);
+    forward_graph(lp, st, g);
+    forward(lp, st, g, false);
     LCHK(hipMemcpyAsync(lp->e, d_e, 3 * (size_t)g.n_nodes * sizeof(float), hipMemcpyDeviceToDevice, st));
     loss_and_backward(lp, st, g);
     LCHK(hipGetLastError());

@@ -94,6 +94,9 @@ int learned_set_params(Learned* lp, const float* host, int n);
 // Forward pass on graph g; *F describes the factor (owned by the Learned
 // object, valid until its next call).
 int learned_infer(Learned* lp, hipStream_t st, const LearnedGraph& g, Factor* F);
+// Once before the learned_train_step calls on a graph: buffers and the
+// graph's own data.
+int learned_train_begin(Learned* lp, hipStream_t st, const LearnedGraph& g);
 // One training step on the pair (r = A e, e): forward, loss
 // min_w ||e - w L L^T r||_A^2 / ||e||_A^2 (scale-free in P), backward, Adam.
 // d_e = null draws e from a seeded Gaussian (zero on penalised nodes).

@@ -58,6 +58,29 @@ def test_network_parity_with_oracle(ctx):
     assert np.linalg.norm(z_d - z_o) <= 1e-5 * np.linalg.norm(z_o)
 
 
+# several blocks of the gradient kernels with a short last one (1,440 nodes), and
+# fewer nodes than one block takes
+@pytest.mark.parametrize("dims", [(17, 9, 7), (4, 2, 1)])
+def test_gradient_blocks_match_oracle(ctx, dims):
+    gpu_case(f"learned gradient {dims}")
+    p = small_problem(dims, seed=9)
+    problems.upload(ctx, p)
+    ctx.assemble()
+    ctx.learned_init(1)
+    prm = mpnn.random_params(12).astype(np.float32)
+    ctx.learned_set_params(prm)
+    g, _ = oracle_learned_graph(p)
+    e = np.random.default_rng(2).standard_normal(p.n_dof)
+    e[np.repeat(g.X[:, 4] > 0, 3)] = 0.0
+    loss_d, grad_d, _, _ = ctx.learned_eval(e, p.n_dof // 3)
+    loss_o, grad_o = mpnn.loss_and_grad(g, prm.astype(np.float64), e)
+    # BF16 activations on both sides, as in test_network_parity_with_oracle
+    assert abs(loss_d - loss_o) <= 1e-4 * abs(loss_o)
+    for name, a, b in GROUPS:
+        err = np.linalg.norm(grad_d[a:b] - grad_o[a:b]) / np.linalg.norm(grad_o[a:b])
+        assert err < 1e-2, (name, err)
+
+
 def test_untrained_network_is_block_jacobi(ctx):
     gpu_case("learned untrained = block Jacobi")
     p = small_problem((8, 3, 3), seed=2)
