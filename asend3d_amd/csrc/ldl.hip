@@ -192,15 +192,13 @@ __device__ __forceinline__ void diag_factor(double* A, double* Li, DiagLds& S, d
         for (int q = w; q < nb * (nb + 1) / 2; q += 4) {
             const int pi = q == 0 ? 0 : (q < 3 ? 1 : 2), pj = q - pi * (pi + 1) / 2;
             const int ib = kb + 1 + pi, jb = kb + 1 + pj;
-            d4v acc;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[r] = A[(kPivot * ib + 4 * r + q4) * kLm + kPivot * jb + c16];
+            d4v acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
             for (int s = 0; s < 4; ++s)
-                acc = mfma64(-A[(kPivot * ib + c16) * kLm + o + 4 * s + q4],
+                acc = mfma64(A[(kPivot * ib + c16) * kLm + o + 4 * s + q4],
                              S.U[(kPivot * pj + c16) * kUs + 4 * s + q4], acc);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) A[(kPivot * ib + 4 * r + q4) * kLm + kPivot * jb + c16] = acc[r];
+            for (int r = 0; r < 4; ++r) A[(kPivot * ib + 4 * r + q4) * kLm + kPivot * jb + c16] -= acc[r];
         }
     }
     if (t == 0 && n_neg > 0) atomicAdd(neg, n_neg);
@@ -323,18 +321,20 @@ __global__ __launch_bounds__(kBlock) void k_ldl_update(LdlDesc d, int k, double*
     const double* Dk = L + ldl_tile(d, blk, k, k);
     double* C = L + ldl_tile(d, blk, I, J);
     const int l = threadIdx.x & 63, r0 = 16 * (threadIdx.x >> 6) + (l >> 4), c = l & 15;
-    d4v acc[4];
+    // the product is summed by itself and subtracted once: added to C term by
+    // term it would be rounded at C's magnitude 16 times a step
+    d4v acc[4] = {}, old[4];
     {
         d2t va[8], vb[8];
         load_tile(L + ldl_tile(d, blk, I, k), va);
         load_tile(L + ldl_tile(d, blk, J, k), vb);
         // the thread's two columns are the same in all of its rows
         const int m = 2 * (threadIdx.x & 31);
-        const double d0 = -Dk[m * (kLdlTile + 1)], d1 = -Dk[(m + 1) * (kLdlTile + 1)];
+        const double d0 = Dk[m * (kLdlTile + 1)], d1 = Dk[(m + 1) * (kLdlTile + 1)];
 #pragma unroll
         for (int b = 0; b < 4; ++b)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[b][r] = C[(r0 + 4 * r) * kLdlTile + 16 * b + c];
+            for (int r = 0; r < 4; ++r) old[b][r] = C[(r0 + 4 * r) * kLdlTile + 16 * b + c];
         store_tile(sA, va);
 #pragma unroll
         for (int h = 0; h < 8; ++h) {
@@ -345,6 +345,8 @@ __global__ __launch_bounds__(kBlock) void k_ldl_update(LdlDesc d, int k, double*
     }
     __syncthreads();
     tile_rows_abt(sA, sB, acc);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) acc[b] = old[b] - acc[b];
     if (q == 0) {
         __syncthreads();  // every wavefront is done with sA
 #pragma unroll
