@@ -45,7 +45,7 @@ struct asend_ctx {
     int64_t n_slices = 0, n_slots = 0;
     std::vector<int32_t> h_sptr;
     int32_t *d_sptr = nullptr, *d_scol = nullptr;
-    Sell3 fine() const {
+    Sell3 sell() const {
         Sell3 A;
         A.n_rows = (int)n_nodes;
         A.n_slices = (int)n_slices;
@@ -53,6 +53,13 @@ struct asend_ctx {
         A.scol = d_scol;
         A.waves_per_block = spmv_wpb;
         A.n_slots = n_slots;
+        return A;
+    }
+    // the same with the reference-block operators (uni) for the solves
+    Sell3 fine() const {
+        Sell3 A = sell();
+        A.uni = uni;
+        A.n_uni = 2;
         return A;
     }
     int64_t nval() const { return 9 * 64 * n_slots; }
@@ -66,6 +73,23 @@ struct asend_ctx {
     // ratio: reference blocks Khat (E = 1) and Mhat (rho = 1) of that element
     bool uniform_hex = false;
     double *d_khat = nullptr, *d_mhat = nullptr;
+    // such a mesh whose nodes are one lattice (every element finds the same
+    // node at the same offset): the solves' products come from the reference
+    // blocks (k_uni3); uni[0] stands for the current operator, uni[1] for the
+    // Newmark mass, each while its value array is set
+    bool uni_tables = false;
+    int32_t *d_uni_nbr = nullptr, *d_uni_el = nullptr, *d_uni_pslot = nullptr;
+    struct UniBufs {
+        double *w64 = nullptr, *kh64 = nullptr;
+        float *w32 = nullptr, *kh32 = nullptr;
+    } uni_bufs[2];
+    double* d_uni_pen64 = nullptr;
+    float* d_uni_pen32 = nullptr;
+    int n_uni_pslots = 0;
+    UniOp uni[2];
+    // one modulus, one density over all elements, and their values
+    bool e_const = false, rho_const = false;
+    double e_first = 0.0, rho_first = 0.0;
     double* d_K64 = nullptr;
     float* d_K32 = nullptr;
     // FP16 row-scaled copy read by the multigrid cycle (allocated with the
@@ -209,6 +233,7 @@ struct asend_ctx {
         // workgroup geometry as launch arguments
         double graph_ru = -1.0;
         int graph_wpb = -1;
+        int graph_uni = -1;  // whether K_eff's products come from the reference blocks
     } nm;
 };
 
@@ -308,6 +333,8 @@ void newmark_free(asend_ctx* ctx) {
     nm.graph_iters = nm.graph_watch = -1;
     nm.graph_ru = -1.0;
     nm.graph_wpb = -1;
+    nm.graph_uni = -1;
+    ctx->uni[1] = UniOp();
     nm.ready = false;
 }
 
@@ -355,6 +382,20 @@ void free_mesh(asend_ctx* ctx) {
     dfree(ctx->d_khat);
     dfree(ctx->d_mhat);
     ctx->uniform_hex = false;
+    ctx->uni_tables = false;
+    ctx->uni[0] = ctx->uni[1] = UniOp();
+    dfree(ctx->d_uni_nbr);
+    dfree(ctx->d_uni_el);
+    dfree(ctx->d_uni_pslot);
+    for (auto& b : ctx->uni_bufs) {
+        dfree(b.w64);
+        dfree(b.kh64);
+        dfree(b.w32);
+        dfree(b.kh32);
+    }
+    dfree(ctx->d_uni_pen64);
+    dfree(ctx->d_uni_pen32);
+    ctx->n_uni_pslots = 0;
     dfree(ctx->d_K64);
     dfree(ctx->d_K32);
     dfree(ctx->d_K16);
@@ -1006,6 +1047,11 @@ int solve_device(asend_ctx* ctx, const asend_solve_opts* o, asend_solve_stats* s
     return ASEND_OK;
 }
 
+// whether an assembly goes through the mesh's reference blocks
+bool uniform_path(const asend_ctx* ctx, double c_damp) {
+    return ctx->uniform_hex && c_damp == 0.0 && !ctx->d_kcond && ctx->n_smat == 0;
+}
+
 // Element integration into K: k_scale K_e(E) + c_mass M_e of every element.
 // Translated-element meshes (brick8, brickIM): one row-wise launch scaling the
 // reference blocks.  Other brick8 meshes: each element integrated once into
@@ -1017,7 +1063,7 @@ int integrate_elements(asend_ctx* ctx, const double* E, double k_scale, double c
         return fail(ctx, ASEND_ERR_UNSUPPORTED, "material damping is implemented for brick8 meshes");
     if (ctx->d_kcond && c_damp != 0.0)
         return fail(ctx, ASEND_ERR_UNSUPPORTED, "the conduction operator has no damping term");
-    if (ctx->uniform_hex && c_damp == 0.0 && !ctx->d_kcond && ctx->n_smat == 0) {
+    if (uniform_path(ctx, c_damp)) {
         launch_hex8_assemble_uniform(ctx->st, (int)ctx->n_nodes, (int)ctx->n_slices, ctx->d_sptr, ctx->d_scol,
                                      ctx->d_rp, ctx->d_n2e_ptr, ctx->d_n2e, ctx->d_conn_r, ctx->d_khat, ctx->d_mhat, E,
                                      ctx->d_rho, k_scale, c_mass, K);
@@ -1062,19 +1108,100 @@ void launch_sens(asend_ctx* ctx, const double* u, const double* lam) {
                          ctx->d_sens);
 }
 
+// Reference-block operator i for the values (val64, val32) = k_scale K +
+// c_mass M of the current mesh: weights k_scale E_e over Khat; with a mass
+// term only where modulus and density are the same in all elements (then
+// both go into one set of blocks with weights 1).  Else none stands for them.
+void uni_set(asend_ctx* ctx, int i, double k_scale, double c_mass, const double* val64, const float* val32) {
+    UniOp& U = ctx->uni[i];
+    U = UniOp();
+    if (!ctx->uni_tables) return;
+    const auto& b = ctx->uni_bufs[i];
+    const int ns = (int)ctx->n_slices;
+    if (c_mass == 0.0) {
+        launch_uni_coef(ctx->st, ctx->d_khat, ctx->d_mhat, 1.0, 0.0, b.kh64, b.kh32);
+        launch_uni_weights(ctx->st, ns, ctx->d_uni_el, ctx->d_E, k_scale, b.w64, b.w32);
+    } else if (k_scale == 0.0) {
+        launch_uni_coef(ctx->st, ctx->d_khat, ctx->d_mhat, 0.0, 1.0, b.kh64, b.kh32);
+        launch_uni_weights(ctx->st, ns, ctx->d_uni_el, ctx->d_rho, c_mass, b.w64, b.w32);
+    } else if (ctx->e_const && ctx->rho_const) {
+        launch_uni_coef(ctx->st, ctx->d_khat, ctx->d_mhat, k_scale * ctx->e_first, c_mass * ctx->rho_first, b.kh64,
+                        b.kh32);
+        launch_uni_weights(ctx->st, ns, ctx->d_uni_el, nullptr, 1.0, b.w64, b.w32);
+    } else {
+        return;
+    }
+    U.val64 = val64;
+    U.val32 = val32;
+    U.nbr = ctx->d_uni_nbr;
+    U.w64 = b.w64;
+    U.kh64 = b.kh64;
+    U.w32 = b.w32;
+    U.kh32 = b.kh32;
+    if (i == 0) {  // the mass carries no penalty
+        U.pslot = ctx->d_uni_pslot;
+        U.pen64 = ctx->d_uni_pen64;
+        U.pen32 = ctx->d_uni_pen32;
+    }
+}
+
+// Tables of the reference-block products for the slices of a mesh (conn_r:
+// block-row ranks), if its nodes are one lattice: at most one element per
+// local position of a node, and the same node at the same offset of a node
+// from all of its elements.
+bool uni_tables(int64_t n_nodes, int64_t n_el, const std::vector<int32_t>& conn_r, std::vector<int32_t>& nbr,
+                std::vector<int32_t>& el) {
+    static const int pos[8][3] = {{0, 0, 0}, {1, 0, 0}, {1, 1, 0}, {0, 1, 0}, {0, 0, 1}, {1, 0, 1}, {1, 1, 1}, {0, 1, 1}};
+    const int64_t ns = (n_nodes + 63) / 64;
+    nbr.assign(27 * 64 * ns, -1);
+    el.assign(8 * 64 * ns, -1);
+    for (int64_t e = 0; e < n_el; ++e)
+        for (int a = 0; a < 8; ++a) {
+            const int64_t r = conn_r[8 * e + a], s = r >> 6, l = r & 63;
+            int32_t& slot = el[64 * (8 * s + a) + l];
+            if (slot >= 0) return false;
+            slot = (int32_t)e;
+            for (int b = 0; b < 8; ++b) {
+                const int o = (pos[b][0] - pos[a][0] + 1) + 3 * (pos[b][1] - pos[a][1] + 1) +
+                              9 * (pos[b][2] - pos[a][2] + 1);
+                int32_t& c = nbr[64 * (27 * s + o) + l];
+                const int32_t v = conn_r[8 * e + b];
+                if (c >= 0 && c != v) return false;
+                c = v;
+            }
+        }
+    for (int64_t s = 0; s < ns; ++s)
+        for (int o = 0; o < 27; ++o)
+            for (int64_t l = 0; l < 64; ++l) {
+                int32_t& c = nbr[64 * (27 * s + o) + l];
+                if (c < 0) c = (int32_t)std::min(64 * s + l, n_nodes - 1);
+            }
+    return true;
+}
+
+bool all_equal(const double* v, int64_t n) {
+    for (int64_t i = 1; i < n; ++i)
+        if (v[i] != v[0]) return false;
+    return true;
+}
+
 // FP16 row-scaled copy of the current operator for the multigrid cycle,
-// when the hierarchy exists (after the Jacobi diagonal).
+// when the hierarchy exists (after the Jacobi diagonal) and the cycle's
+// products do not come from the reference blocks.
 void refresh_f16(asend_ctx* ctx) {
-    if (ctx->d_K16)
+    if (ctx->d_K16 && !ctx->uni[0].val32)
         launch_to_f16_rowscaled(ctx->st, (int)ctx->n_nodes, (int)ctx->n_slices, ctx->d_sptr, ctx->d_K64,
                                 ctx->d_dinv64, ctx->d_K16);
 }
 
 // Penalty scale (fixed on the first assembly), penalty diagonal, Jacobi
-// diagonal and FP32 copy of the element operator held in d_K64
-int finish_assembly(asend_ctx* ctx, double k_scale, double c_mass) {
+// diagonal and FP32 copy of the element operator held in d_K64; uniform: it
+// was assembled from the reference blocks
+int finish_assembly(asend_ctx* ctx, double k_scale, double c_mass, bool uniform) {
     const int64_t nval = ctx->nval();
     int rc;
+    ctx->uni[0] = UniOp();
+    if (uniform) uni_set(ctx, 0, k_scale, c_mass, ctx->d_K64, ctx->d_K32);
     if (ctx->n_pen > 0) {
         if (ctx->h_pen.back() >= ctx->n_dof) return fail(ctx, ASEND_ERR_STATE, "penalty DOF beyond the mesh");
         if (!ctx->sf_fixed) {
@@ -1093,6 +1220,9 @@ int finish_assembly(asend_ctx* ctx, double k_scale, double c_mass) {
         if ((rc = write_scalars(ctx, 2))) return rc;
         launch_penalty_diag(ctx->st, ctx->d_pen, ctx->d_pen_mult, ctx->n_pen, ctx->d_sptr, ctx->d_kdiag,
                             ctx->d_K64, ctx->d_sc + 2);
+        if (ctx->uni[0].val64)
+            launch_uni_penalty(ctx->st, ctx->d_pen, ctx->d_pen_mult, ctx->n_pen, ctx->sf, ctx->d_uni_pslot,
+                               ctx->n_uni_pslots, ctx->d_uni_pen64, ctx->d_uni_pen32);
     }
     launch_diag_inv(ctx->st, (int)ctx->n_nodes, ctx->d_sptr, ctx->d_kdiag, ctx->d_K64, ctx->d_dinv64,
                     ctx->d_dinv32);
@@ -1112,7 +1242,7 @@ int assemble_device(asend_ctx* ctx, double k_scale, double c_mass, double c_damp
     if (ctx->etype == ASEND_SHELL4 && !ctx->thk_set)
         return fail(ctx, ASEND_ERR_STATE, "shell4 mesh without thickness (asend_set_thickness)");
     int rc = integrate_elements(ctx, ctx->d_E, k_scale, c_mass, ctx->d_K64, c_damp);
-    if (rc || (rc = finish_assembly(ctx, k_scale, c_mass))) return rc;
+    if (rc || (rc = finish_assembly(ctx, k_scale, c_mass, uniform_path(ctx, c_damp)))) return rc;
     ctx->asm_cdamp = c_damp;
     return ASEND_OK;
 }
@@ -1159,7 +1289,7 @@ int nl_assemble(asend_ctx* ctx, double fact, double* rhs) {
     launch_rec_gather(ctx->st, (int)ctx->n_nodes, (int)ctx->n_slices, ctx->d_sptr, ctx->d_n2e_ptr, ctx->d_n2rec,
                       ctx->d_slot, ctx->d_kb, ctx->d_nl_re, fact, ctx->d_nl_f, ctx->d_K64, ctx->d_nl_r, rhs);
     HIPCHK(hipGetLastError());
-    if ((rc = finish_assembly(ctx, 1.0, 0.0))) return rc;
+    if ((rc = finish_assembly(ctx, 1.0, 0.0, false))) return rc;
     if (rhs) {
         launch_nl_penalty_load(ctx->st, ctx->d_pen, ctx->d_pen_mult, ctx->n_pen, ctx->d_sc + 2, ctx->d_nl_u, rhs);
         HIPCHK(hipGetLastError());
@@ -1271,7 +1401,7 @@ int asend_ctx_create(int device, asend_ctx** out) {
     if (hipStreamCreateWithFlags(&ctx->st, hipStreamNonBlocking) != hipSuccess ||
         hipMalloc((void**)&ctx->d_sc, 4 * sizeof(Scalars)) != hipSuccess ||
         hipHostMalloc((void**)&ctx->h_sc, 4 * sizeof(Scalars), hipHostMallocDefault) != hipSuccess ||
-        hipMalloc((void**)&ctx->d_partials, kMaxPartials * 2 * sizeof(double)) != hipSuccess ||
+        hipMalloc((void**)&ctx->d_partials, kMaxPartials * 3 * sizeof(double)) != hipSuccess ||
         hipMalloc((void**)&ctx->d_counter, 16 * sizeof(unsigned)) != hipSuccess ||
         hipEventCreate(&ctx->ev0) != hipSuccess || hipEventCreate(&ctx->ev1) != hipSuccess ||
         hipStreamCreateWithFlags(&ctx->st2, hipStreamNonBlocking) != hipSuccess ||
@@ -1522,7 +1652,7 @@ int asend_upload_mesh(asend_ctx* ctx, int elem_type, int64_t n_mesh_nodes, const
     ctx->n_slots = ctx->h_sptr[ctx->n_slices];
     // the SpMV with one slice per workgroup writes one partial per slice
     if (ctx->n_slices > ctx->partials_cap) {
-        int rc0 = dalloc(ctx, &ctx->d_partials, 2 * (size_t)ctx->n_slices);
+        int rc0 = dalloc(ctx, &ctx->d_partials, 3 * (size_t)ctx->n_slices);
         if (rc0) return rc0;
         ctx->partials_cap = ctx->n_slices;
     }
@@ -1614,6 +1744,25 @@ int asend_upload_mesh(asend_ctx* ctx, int elem_type, int64_t n_mesh_nodes, const
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(ctx->st));
         ctx->uniform_hex = true;
+        std::vector<int32_t> nbr, el;
+        if (uni_tables(n_nodes, n_el, conn_r, nbr, el)) {
+            const size_t ns = (size_t)ctx->n_slices;
+            if ((rc = dalloc(ctx, &ctx->d_uni_nbr, nbr.size())) || (rc = dalloc(ctx, &ctx->d_uni_el, el.size())) ||
+                (rc = dalloc(ctx, &ctx->d_uni_pslot, ns)))
+                return rc;
+            for (auto& b : ctx->uni_bufs)
+                if ((rc = dalloc(ctx, &b.w64, 512 * ns)) || (rc = dalloc(ctx, &b.w32, 512 * ns)) ||
+                    (rc = dalloc(ctx, &b.kh64, kUniCoefs)) || (rc = dalloc(ctx, &b.kh32, kUniCoefs)))
+                    return rc;
+            HIPCHK(hipMemcpy(ctx->d_uni_nbr, nbr.data(), nbr.size() * 4, hipMemcpyHostToDevice));
+            HIPCHK(hipMemcpy(ctx->d_uni_el, el.data(), el.size() * 4, hipMemcpyHostToDevice));
+            HIPCHK(hipMemset(ctx->d_uni_pslot, 0xff, ns * 4));  // no penalties
+            ctx->e_const = all_equal(E, n_el);
+            ctx->e_first = E[0];
+            ctx->rho_const = !rho || all_equal(rho, n_el);
+            ctx->rho_first = rho ? rho[0] : 0.0;
+            ctx->uni_tables = true;
+        }
     }
     if ((rc = ensure_work(ctx))) return rc;
     return ASEND_OK;
@@ -1707,6 +1856,8 @@ int asend_update_moduli(asend_ctx* ctx, const double* E) {
     double s = 0.0;
     for (int64_t e = 0; e < ctx->n_el; ++e) s += std::log(E[e]);
     ctx->mean_log_e = s / (double)ctx->n_el;
+    ctx->e_const = all_equal(E, ctx->n_el);
+    ctx->e_first = E[0];
     ctx->assembled = false;
     return ASEND_OK;
 }
@@ -1737,6 +1888,19 @@ int asend_set_penalty(asend_ctx* ctx, int64_t n, const int64_t* dofs, double sf)
         std::vector<uint8_t> cl(ctx->n_nodes, 0);
         for (int64_t d : u) cl[d / 3] = 1;
         HIPCHK(hipMemcpy(ctx->d_clamped, cl.data(), cl.size(), hipMemcpyHostToDevice));
+    }
+    if (ctx->uni_tables) {
+        // penalty terms of the reference-block products: 64 x 3 per slice that holds any
+        std::vector<int32_t> ps(ctx->n_slices, -1);
+        int n_ps = 0;
+        for (int64_t d : u)
+            if (ps[d / 192] < 0) ps[d / 192] = n_ps++;
+        ctx->uni[0] = UniOp();
+        if ((rc = dalloc(ctx, &ctx->d_uni_pen64, 192 * (size_t)n_ps)) ||
+            (rc = dalloc(ctx, &ctx->d_uni_pen32, 192 * (size_t)n_ps)))
+            return rc;
+        HIPCHK(hipMemcpy(ctx->d_uni_pslot, ps.data(), ps.size() * 4, hipMemcpyHostToDevice));
+        ctx->n_uni_pslots = n_ps;
     }
     ctx->n_pen = (int)u.size();
     ctx->h_pen = u;
@@ -1806,14 +1970,14 @@ int asend_spmv(asend_ctx* ctx, int precision, const double* x, double* y) {
     const int64_t n = ctx->n_dof;
     if (precision == 64) {
         HIPCHK(hipMemcpy(ctx->d_p, x, n * 8, hipMemcpyHostToDevice));
-        launch_sell3<double>(ctx->st, 0, ctx->fine(), ctx->d_K64, ctx->d_p, ctx->d_q, nullptr, nullptr, nullptr);
+        launch_sell3<double>(ctx->st, 0, ctx->sell(), ctx->d_K64, ctx->d_p, ctx->d_q, nullptr, nullptr, nullptr);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(ctx->st));
         HIPCHK(hipMemcpy(y, ctx->d_q, n * 8, hipMemcpyDeviceToHost));
     } else if (precision == 32) {
         std::vector<float> xf(x, x + n), yf(n);
         HIPCHK(hipMemcpy(ctx->d_p32, xf.data(), n * 4, hipMemcpyHostToDevice));
-        launch_sell3<float>(ctx->st, 0, ctx->fine(), ctx->d_K32, ctx->d_p32, ctx->d_q32, nullptr, nullptr, nullptr);
+        launch_sell3<float>(ctx->st, 0, ctx->sell(), ctx->d_K32, ctx->d_p32, ctx->d_q32, nullptr, nullptr, nullptr);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(ctx->st));
         HIPCHK(hipMemcpy(yf.data(), ctx->d_q32, n * 4, hipMemcpyDeviceToHost));
@@ -2217,10 +2381,10 @@ int asend_bench_spmv(asend_ctx* ctx, int precision, int n_iter, double* avg_ms) 
         if (pass == 1) HIPCHK(hipEventRecord(ctx->ev0, ctx->st));
         for (int i = 0; i < cnt; ++i) {
             if (precision == 64)
-                launch_sell3<double>(ctx->st, 0, ctx->fine(), ctx->d_K64, ctx->d_u, ctx->d_q, nullptr, nullptr,
+                launch_sell3<double>(ctx->st, 0, ctx->sell(), ctx->d_K64, ctx->d_u, ctx->d_q, nullptr, nullptr,
                                      nullptr);
             else
-                launch_sell3<float>(ctx->st, 0, ctx->fine(), ctx->d_K32, ctx->d_x32, ctx->d_q32, nullptr, nullptr,
+                launch_sell3<float>(ctx->st, 0, ctx->sell(), ctx->d_K32, ctx->d_x32, ctx->d_q32, nullptr, nullptr,
                                     nullptr);
         }
     }
@@ -2494,6 +2658,7 @@ int asend_newmark_setup(asend_ctx* ctx, double dt, double beta, double gamma) {
         dfree(zeroE);
         if (rc) return rc;
     }
+    if (uniform_path(ctx, 0.0)) uni_set(ctx, 1, 0.0, 1.0, nm.M64, nullptr);
     // D = cm M + ck K (+ the material damping matrices), the damped load's
     // work vector
     if (nm.damped()) {
@@ -2668,7 +2833,7 @@ int asend_newmark_run(asend_ctx* ctx, int64_t n_steps, const double* f_shape, co
     const bool graph = ctx->use_graphs;
     if (graph && (!nm.exec_head || nm.graph_iters != blk || nm.graph_watch != nw || nm.graph_save != nm.save_u ||
                   nm.graph_save_y != nm.save_y || nm.graph_mixed != (int)mixed || nm.graph_ru != mx.ru_factor ||
-                  nm.graph_wpb != A.waves_per_block)) {
+                  nm.graph_wpb != A.waves_per_block || nm.graph_uni != (ctx->uni[0].val64 ? 1 : 0))) {
         if ((rc = capture(&nm.exec_head, head)) || (rc = capture(&nm.exec_more, iterations)) ||
             (rc = capture(&nm.exec_tail, tail)))
             return rc;
@@ -2679,6 +2844,7 @@ int asend_newmark_run(asend_ctx* ctx, int64_t n_steps, const double* f_shape, co
         nm.graph_mixed = (int)mixed;
         nm.graph_ru = mx.ru_factor;
         nm.graph_wpb = A.waves_per_block;
+        nm.graph_uni = ctx->uni[0].val64 ? 1 : 0;
     }
     HIPCHK(hipEventRecord(ctx->ev0, ctx->st));
     for (int64_t s = 0; s < n_steps; ++s) {
@@ -2960,6 +3126,7 @@ static int modal_impl(asend_ctx* ctx, int kind, const double* u, int n_modes, do
         launch_diag_inv(ctx->st, (int)ctx->n_nodes, ctx->d_sptr, ctx->d_kdiag, ctx->d_K64, ctx->d_dinv64,
                         ctx->d_dinv32);
         launch_to_f32(ctx->st, ctx->d_K64, ctx->d_K32, nval);
+        ctx->uni[0] = UniOp();  // the shift is not in the reference blocks
         refresh_f16(ctx);
         HIPCHK(hipGetLastError());
     }

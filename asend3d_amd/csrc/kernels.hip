@@ -743,20 +743,78 @@ __device__ __forceinline__ T sell_load(const T* p) {
     else return *p;
 }
 
+// Row epilogue of the operator products (modes at the block-row SpMV below):
+// (a0, a1, a2) = row r of K x; writes y and adds to the row's partial sums.
+template <typename T, int MODE>
+__device__ __forceinline__ void row_epilogue(int r, T a0, T a1, T a2, const T* __restrict__ x, T* __restrict__ y,
+                                             const T* __restrict__ f, double (&part)[3]) {
+    const int64_t d = 3 * (int64_t)r;
+    if (MODE == 2 || MODE == 3 || MODE == 5) {
+        const T y0 = f[d] - a0, y1 = f[d + 1] - a1, y2 = f[d + 2] - a2;
+        y[d] = y0;
+        y[d + 1] = y1;
+        y[d + 2] = y2;
+        part[0] = (double)y0 * y0 + (double)y1 * y1 + (double)y2 * y2;
+        return;
+    }
+    y[d] = a0;
+    y[d + 1] = a1;
+    y[d + 2] = a2;
+    if (MODE == 0) return;
+    const double x0 = x[d], x1 = x[d + 1], x2 = x[d + 2];
+    const double kx = (double)a0 * x0 + (double)a1 * x1 + (double)a2 * x2;
+    if (MODE == 1) part[0] = kx;
+    if (MODE == 7) {
+        // x = p, f = r: partials p.(K p) and p.r
+        part[0] = kx;
+        part[1] = x0 * f[d] + x1 * f[d + 1] + x2 * f[d + 2];
+    }
+    if (MODE == 4 || MODE == 6) {
+        // x = u (preconditioned residual), f = r: partials r.u, (K u).u, r.r
+        const double r0 = f[d], r1 = f[d + 1], r2 = f[d + 2];
+        part[0] = r0 * x0 + r1 * x1 + r2 * x2;
+        part[1] = kx;
+        part[2] = r0 * r0 + r1 * r1 + r2 * r2;
+    }
+}
+
+// the block's partial sums of a mode, stored for its finalize kernel
+template <int MODE>
+__device__ __forceinline__ void mode_partials(const double (&part)[3], double* partials) {
+    if (MODE == 0 || MODE == 3) return;
+    if (MODE == 4 || MODE == 6) {
+        double t[3] = {part[0], part[1], part[2]};
+        block_partials<3>(t, partials);
+    } else if (MODE == 7) {
+        double t[2] = {part[0], part[1]};
+        block_partials<2>(t, partials);
+    } else {
+        double t[1] = {part[0]};
+        block_partials<1>(t, partials);
+    }
+}
+
+// whether a mode's launch has nothing to do (converged, or paused)
+template <int MODE>
+__device__ __forceinline__ bool mode_idle(const Scalars* sc) {
+    if (MODE == 1 || MODE == 4 || MODE == 7) return sc->done;
+    if (MODE == 6) return sc->done || sc->gate;
+    if (MODE == 5) return !sc->gate;
+    return false;
+}
+
 template <typename T, int MODE, bool NT>
 __global__ __launch_bounds__(kSellMaxWaves * kWave) void k_sell3(int n_rows, int n_slices,
                                                                  const int32_t* __restrict__ sptr,
                                                   const int32_t* __restrict__ scol, const T* __restrict__ val,
                                                   const T* __restrict__ x, T* __restrict__ y,
                                                   const T* __restrict__ f, double* partials, const Scalars* sc) {
-    if ((MODE == 1 || MODE == 4 || MODE == 7) && sc->done) return;
-    if (MODE == 6 && (sc->done || sc->gate)) return;
-    if (MODE == 5 && !sc->gate) return;
+    if (mode_idle<MODE>(sc)) return;
     const int lb = xcd_block(blockIdx.x, gridDim.x);
     const int slice = lb * (int)(blockDim.x / kWave) + threadIdx.x / kWave;
     const int lane = threadIdx.x % kWave;
     const int r = slice * kWave + lane;
-    double part = 0.0, part1 = 0.0, part2 = 0.0;
+    double part[3] = {0.0, 0.0, 0.0};
     if (slice < n_slices) {
         const int k0 = sptr[slice], k1 = sptr[slice + 1];
         const int32_t* cp = scol + (int64_t)k0 * kWave + lane;
@@ -778,104 +836,287 @@ __global__ __launch_bounds__(kSellMaxWaves * kWave) void k_sell3(int n_rows, int
             cp += kWave;
             vp += 9 * kWave;
         }
-        if (r < n_rows) {
-            if (MODE == 2 || MODE == 3 || MODE == 5) {
-                T y0 = f[3 * (int64_t)r] - a0, y1 = f[3 * (int64_t)r + 1] - a1, y2 = f[3 * (int64_t)r + 2] - a2;
-                y[3 * (int64_t)r] = y0;
-                y[3 * (int64_t)r + 1] = y1;
-                y[3 * (int64_t)r + 2] = y2;
-                part = (double)y0 * y0 + (double)y1 * y1 + (double)y2 * y2;
-            } else if (MODE == 7) {
-                // x = p, f = r: partials p.(K p) and p.r
-                y[3 * (int64_t)r] = a0;
-                y[3 * (int64_t)r + 1] = a1;
-                y[3 * (int64_t)r + 2] = a2;
-                const double p0 = x[3 * (int64_t)r], p1 = x[3 * (int64_t)r + 1], p2 = x[3 * (int64_t)r + 2];
-                part = (double)a0 * p0 + (double)a1 * p1 + (double)a2 * p2;
-                part1 = p0 * f[3 * (int64_t)r] + p1 * f[3 * (int64_t)r + 1] + p2 * f[3 * (int64_t)r + 2];
-            } else if (MODE == 4 || MODE == 6) {
-                // x = u (preconditioned residual), f = r: partials r.u, (K u).u, r.r
-                y[3 * (int64_t)r] = a0;
-                y[3 * (int64_t)r + 1] = a1;
-                y[3 * (int64_t)r + 2] = a2;
-                const double u0 = x[3 * (int64_t)r], u1 = x[3 * (int64_t)r + 1], u2 = x[3 * (int64_t)r + 2];
-                const double r0 = f[3 * (int64_t)r], r1 = f[3 * (int64_t)r + 1], r2 = f[3 * (int64_t)r + 2];
-                part = r0 * u0 + r1 * u1 + r2 * u2;
-                part1 = (double)a0 * u0 + (double)a1 * u1 + (double)a2 * u2;
-                part2 = r0 * r0 + r1 * r1 + r2 * r2;
-            } else {
-                y[3 * (int64_t)r] = a0;
-                y[3 * (int64_t)r + 1] = a1;
-                y[3 * (int64_t)r + 2] = a2;
-                if (MODE == 1)
-                    part = (double)a0 * x[3 * (int64_t)r] + (double)a1 * x[3 * (int64_t)r + 1] +
-                           (double)a2 * x[3 * (int64_t)r + 2];
+        if (r < n_rows) row_epilogue<T, MODE>(r, a0, a1, a2, x, y, f, part);
+    }
+    mode_partials<MODE>(part, partials);
+}
+
+// ---------------------------------------------------------------------------
+// Operator products on meshes of translated copies of one element (brick8,
+// brickIM), without the assembled values:
+//   (K x)_r = sum over a of w_a(r) [sum over b != a of Kh_ab (x_b(r, a) - x_r)
+//             + s_a x_r] + pen_r x_r,
+// a the local position of node r in its (at most one per position) element,
+// w_a that element's weight (its modulus; 0 where there is none), b(r, a) the
+// element's node b, s_a the row sum of the blocks (a mass term's; a stiffness
+// has none: translations carry no force).  As the elements are translates, node
+// b of the element at position a is the neighbour of r at lattice offset
+// pos(b) - pos(a), one of 27 (checked at upload), so a row reads 27 neighbours, 27
+// indices and 8 weights instead of 27 blocks of 9 values: 220 B (FP64) against
+// 2.1 kB, for 610 operations against 243 multiply-adds.  The 576 block entries
+// are the same for every row: they are read through the scalar cache as the
+// scalar operand of each multiply-add.
+//
+// The differences keep translations in the null space whatever the rounding.
+// With Kh_aa x_r in the sum instead, an FP32 Kh is off by the same rounding in
+// every element, which adds up over the mesh to a spurious stiffness of its
+// translations: the multigrid FCG on 200x40x40 took 40 iterations instead of 24
+// although each product was closer to the FP64 one.
+//
+// A workgroup's four wavefronts take one 64-row slice, two positions (11
+// neighbours, 14 of the 56 blocks) each, and add up in LDS.  One wavefront per
+// slice reads each neighbour once instead of 1.6 times but holds all 81
+// values at once (256 registers, one wavefront per SIMD): 52 us against 30 us
+// on 200x40x40 in FP64.  Assembled values against this, p.Kp included:
+//   525 nodes FP64 12.9 / 5.0 us, 44,541 nodes FP64 14.8 / 7.7 us,
+//   337,881 nodes FP64 136 / 29.6 us, FP32 65 / 18 us, cycle (FP16) 38 / 17.7 us,
+// so it is taken wherever the tables exist.  The large ones are bound by the
+// 26 gathers of 24 (12) scattered bytes per lane.
+// ---------------------------------------------------------------------------
+constexpr int kUniWaves = 4;  // wavefronts per slice
+
+// lattice position of brick8 node t
+__host__ __device__ constexpr int uni_px(int t) { return ((t ^ (t >> 1)) & 1); }
+__host__ __device__ constexpr int uni_py(int t) { return (t >> 1) & 1; }
+__host__ __device__ constexpr int uni_pz(int t) { return t >> 2; }
+// node at lattice position (x, y, z), -1 outside the element
+__host__ __device__ constexpr int uni_node(int x, int y, int z) {
+    return (x < 0 || x > 1 || y < 0 || y > 1 || z < 0 || z > 1) ? -1 : 4 * z + 2 * y + (x ^ y);
+}
+
+// rows' products over the positions A0 and A0 + 1; xr: the row's own values,
+// kh: blocks 9 (8 a + b) + c, then the 8 row sums
+template <typename T, int A0>
+__device__ __forceinline__ void uni_rows(const int32_t* __restrict__ nb, const T* __restrict__ w,
+                                         const T* __restrict__ kh, const T* __restrict__ x, const T (&xr)[3],
+                                         T (&y)[3]) {
+    constexpr int NA = 2;
+    T t[NA][3], wa[NA];
+#pragma unroll
+    for (int a = 0; a < NA; ++a) {
+        wa[a] = w[64 * (A0 + a)];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) t[a][i] = kh[576 + A0 + a] * xr[i];
+    }
+#pragma unroll
+    for (int dz = -1; dz <= 1; ++dz) {
+        T xs[9][3];
+#pragma unroll
+        for (int j = 0; j < 9; ++j) {
+            const int dx = j % 3 - 1, dy = j / 3 - 1;
+            bool used = false;
+#pragma unroll
+            for (int a = A0; a < A0 + NA; ++a)
+                used = used || uni_node(uni_px(a) + dx, uni_py(a) + dy, uni_pz(a) + dz) >= 0;
+            if (!used || (dz == 0 && j == 4)) continue;
+            const int64_t c = 3 * (int64_t)nb[64 * (9 * (dz + 1) + j)];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) xs[j][i] = x[c + i];
+        }
+#pragma unroll
+        for (int j = 0; j < 9; ++j) {
+            const int dx = j % 3 - 1, dy = j / 3 - 1;
+            if (dz == 0 && j == 4) continue;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) xs[j][i] -= xr[i];
+#pragma unroll
+            for (int a = 0; a < NA; ++a) {
+                const int b = uni_node(uni_px(A0 + a) + dx, uni_py(A0 + a) + dy, uni_pz(A0 + a) + dz);
+                if (b < 0) continue;
+                const T* k = kh + 9 * (8 * (A0 + a) + b);
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+                    t[a][i] += k[3 * i] * xs[j][0] + k[3 * i + 1] * xs[j][1] + k[3 * i + 2] * xs[j][2];
             }
         }
     }
-    if (MODE == 0 || MODE == 3) return;
-    if (MODE == 4 || MODE == 6) {
-        double t[3] = {part, part1, part2};
-        block_partials<3>(t, partials);
-        return;
-    }
-    if (MODE == 7) {
-        double t[2] = {part, part1};
-        block_partials<2>(t, partials);
-        return;
-    }
-    double t[1] = {part};
-    block_partials<1>(t, partials);
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) y[i] += wa[a] * t[a][i];
 }
 
 template <typename T, int MODE>
-static void sell3_go(hipStream_t st, bool nt, int nblk, int nthr, const Sell3& A, const T* val, const T* x, T* y,
-                     const T* f, double* partials, Scalars* sc) {
+__global__ __launch_bounds__(kUniWaves * kWave) void k_uni3(int n_rows, const int32_t* __restrict__ nbr,
+                                                            const T* __restrict__ w, const T* __restrict__ kh,
+                                                            const int32_t* __restrict__ pslot,
+                                                            const T* __restrict__ pen, const T* __restrict__ x,
+                                                            T* __restrict__ y, const T* __restrict__ f,
+                                                            double* partials, const Scalars* sc) {
+    if (mode_idle<MODE>(sc)) return;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int slice = xcd_block(blockIdx.x, gridDim.x);
+    const int r = 64 * slice + lane;
+    const int32_t* nb = nbr + (int64_t)27 * 64 * slice + lane;
+    const T* wl = w + (int64_t)8 * 64 * slice + lane;
+    const T* xp = x + 3 * (int64_t)min(r, n_rows - 1);
+    const T xr[3] = {xp[0], xp[1], xp[2]};
+    T a[3] = {0, 0, 0};
+    if (wv == 0) uni_rows<T, 0>(nb, wl, kh, x, xr, a);
+    else if (wv == 1) uni_rows<T, 2>(nb, wl, kh, x, xr, a);
+    else if (wv == 2) uni_rows<T, 4>(nb, wl, kh, x, xr, a);
+    else uni_rows<T, 6>(nb, wl, kh, x, xr, a);
+    __shared__ T sh[3][kUniWaves - 1][kWave];
+    if (wv > 0) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) sh[i][wv - 1][lane] = a[i];
+    }
+    __syncthreads();
+    double part[3] = {0.0, 0.0, 0.0};
+    if (wv == 0 && r < n_rows) {
+#pragma unroll
+        for (int v = 0; v < kUniWaves - 1; ++v)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) a[i] += sh[i][v][lane];
+        const int ps = pslot ? pslot[slice] : -1;
+        if (ps >= 0) {
+            const T* pp = pen + 192 * (int64_t)ps + 3 * lane;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) a[i] += pp[i] * xr[i];
+        }
+        row_epilogue<T, MODE>(r, a[0], a[1], a[2], x, y, f, part);
+    }
+    mode_partials<MODE>(part, partials);
+}
+
+__global__ void k_uni_weights(int n, const int32_t* __restrict__ el, const double* __restrict__ E, double scale,
+                              double* __restrict__ w64, float* __restrict__ w32) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int e = el[i];
+    const double v = e >= 0 ? scale * (E ? E[e] : 1.0) : 0.0;
+    w64[i] = v;
+    w32[i] = (float)v;
+}
+
+void launch_uni_weights(hipStream_t st, int n_slices, const int32_t* el, const double* E, double scale, double* w64,
+                        float* w32) {
+    const int n = 512 * n_slices;
+    hipLaunchKernelGGL(k_uni_weights, dim3((n + 255) / 256), dim3(256), 0, st, n, el, E, scale, w64, w32);
+}
+
+__global__ void k_uni_coef(const double* __restrict__ Khat, const double* __restrict__ Mhat, double sK, double sM,
+                           double* __restrict__ kh64, float* __restrict__ kh32) {
+    const int i = threadIdx.x;
+    double v;
+    if (i < 576) {
+        v = sK * Khat[i] + (i % 9 % 4 == 0 ? sM * Mhat[i / 9] : 0.0);
+    } else {
+        v = 0.0;
+        for (int b = 0; b < 8; ++b) v += sM * Mhat[8 * (i - 576) + b];
+    }
+    kh64[i] = v;
+    kh32[i] = (float)v;
+}
+
+void launch_uni_coef(hipStream_t st, const double* Khat, const double* Mhat, double sK, double sM, double* kh64,
+                     float* kh32) {
+    hipLaunchKernelGGL(k_uni_coef, dim3(1), dim3(kUniCoefs), 0, st, Khat, Mhat, sK, sM, kh64, kh32);
+}
+
+__global__ void k_uni_penalty(const int64_t* __restrict__ pen, const int32_t* __restrict__ mult, int n_pen, double sf,
+                              const int32_t* __restrict__ pslot, double* __restrict__ pen64,
+                              float* __restrict__ pen32) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n_pen) return;
+    const int64_t d = pen[i];
+    const int r = (int)(d / 3);
+    const int64_t o = 192 * (int64_t)pslot[r >> 6] + 3 * (r & 63) + d % 3;
+    pen64[o] = mult[i] * sf;
+    pen32[o] = (float)(mult[i] * sf);
+}
+
+__global__ void k_uni_clear(int64_t n, double* __restrict__ a, float* __restrict__ b) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    a[i] = 0.0;
+    b[i] = 0.f;
+}
+
+void launch_uni_penalty(hipStream_t st, const int64_t* pen, const int32_t* mult, int n_pen, double sf,
+                        const int32_t* pslot, int n_pslots, double* pen64, float* pen32) {
+    if (n_pslots <= 0) return;
+    const int64_t n = 192 * (int64_t)n_pslots;
+    hipLaunchKernelGGL(k_uni_clear, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, n, pen64, pen32);
+    hipLaunchKernelGGL(k_uni_penalty, dim3((n_pen + 255) / 256), dim3(256), 0, st, pen, mult, n_pen, sf, pslot, pen64,
+                       pen32);
+}
+
+template <typename T, int MODE>
+static int uni3_go(hipStream_t st, const Sell3& A, const UniOp& U, const T* x, T* y, const T* f, double* partials,
+                   Scalars* sc) {
+    const T *w, *kh, *pen;
+    if constexpr (sizeof(T) == 8) {
+        w = U.w64;
+        kh = U.kh64;
+        pen = U.pen64;
+    } else {
+        w = U.w32;
+        kh = U.kh32;
+        pen = U.pen32;
+    }
+    hipLaunchKernelGGL((k_uni3<T, MODE>), dim3(A.n_slices), dim3(kUniWaves * kWave), 0, st, A.n_rows, U.nbr, w, kh,
+                       U.pslot, pen, x, y, f, partials, sc);
+    return A.n_slices;
+}
+
+// the reference-block operator that stands for val, null if none does
+template <typename T>
+static const UniOp* uni_of(const Sell3& A, const T* val) {
+    for (int i = 0; i < A.n_uni; ++i) {
+        if constexpr (sizeof(T) == 8) {
+            if (A.uni[i].val64 && A.uni[i].val64 == val) return A.uni + i;
+        } else {
+            if (A.uni[i].val32 && A.uni[i].val32 == val) return A.uni + i;
+        }
+    }
+    return nullptr;
+}
+
+template <typename T, int MODE>
+static int sell3_go(hipStream_t st, const Sell3& A, const T* val, const T* x, T* y, const T* f, double* partials,
+                    Scalars* sc) {
+    if (const UniOp* U = uni_of(A, val)) return uni3_go<T, MODE>(st, A, *U, x, y, f, partials, sc);
+    const int per = A.waves_per_block;
+    const int nblk = (A.n_slices + per - 1) / per;
+    const int nthr = per * kWave;
+    const bool nt = (int64_t)sizeof(T) * 9 * kWave * A.n_slots > kSellStreamBytes;
     if (nt)
         hipLaunchKernelGGL((k_sell3<T, MODE, true>), dim3(nblk), dim3(nthr), 0, st, A.n_rows, A.n_slices, A.sptr,
                            A.scol, val, x, y, f, partials, sc);
     else
         hipLaunchKernelGGL((k_sell3<T, MODE, false>), dim3(nblk), dim3(nthr), 0, st, A.n_rows, A.n_slices, A.sptr,
                            A.scol, val, x, y, f, partials, sc);
+    return nblk;
 }
 
 template <typename T>
 void launch_sell3(hipStream_t st, int mode, const Sell3& A, const T* val, const T* x, T* y, const T* f,
                   double* partials, Scalars* sc) {
-    const int per = A.waves_per_block;
-    const int nblk = (A.n_slices + per - 1) / per;
-    const int nthr = per * kWave;
-    const bool nt = (int64_t)sizeof(T) * 9 * kWave * A.n_slots > kSellStreamBytes;
     switch (mode) {
         case 0:
-            sell3_go<T, 0>(st, nt, nblk, nthr, A, val, x, y, f, partials, sc);
+            sell3_go<T, 0>(st, A, val, x, y, f, partials, sc);
             break;
         case 1:
-            sell3_go<T, 1>(st, nt, nblk, nthr, A, val, x, y, f, partials, sc);
-            finalize(st, partials, nblk, FIN_PQ, sc);
+            finalize(st, partials, sell3_go<T, 1>(st, A, val, x, y, f, partials, sc), FIN_PQ, sc);
             break;
         case 2:
-            sell3_go<T, 2>(st, nt, nblk, nthr, A, val, x, y, f, partials, sc);
-            finalize(st, partials, nblk, FIN_RR, sc);
+            finalize(st, partials, sell3_go<T, 2>(st, A, val, x, y, f, partials, sc), FIN_RR, sc);
             break;
         case 4:
-            sell3_go<T, 4>(st, nt, nblk, nthr, A, val, x, y, f, partials, sc);
-            finalize(st, partials, nblk, FIN_CG1, sc);
+            finalize(st, partials, sell3_go<T, 4>(st, A, val, x, y, f, partials, sc), FIN_CG1, sc);
             break;
         case 5:
-            sell3_go<T, 5>(st, nt, nblk, nthr, A, val, x, y, f, partials, sc);
-            finalize(st, partials, nblk, FIN_RU_RES, sc);
+            finalize(st, partials, sell3_go<T, 5>(st, A, val, x, y, f, partials, sc), FIN_RU_RES, sc);
             break;
         case 6:
-            sell3_go<T, 6>(st, nt, nblk, nthr, A, val, x, y, f, partials, sc);
-            finalize(st, partials, nblk, FIN_CG1_RU, sc);
+            finalize(st, partials, sell3_go<T, 6>(st, A, val, x, y, f, partials, sc), FIN_CG1_RU, sc);
             break;
         case 7:
-            sell3_go<T, 7>(st, nt, nblk, nthr, A, val, x, y, f, partials, sc);
-            finalize(st, partials, nblk, FIN_PQR, sc);
+            finalize(st, partials, sell3_go<T, 7>(st, A, val, x, y, f, partials, sc), FIN_PQR, sc);
             break;
         default:
-            sell3_go<T, 3>(st, nt, nblk, nthr, A, val, x, y, f, partials, sc);
+            sell3_go<T, 3>(st, A, val, x, y, f, partials, sc);
             break;
     }
 }
@@ -1018,6 +1259,13 @@ void launch_sell3_h(hipStream_t st, int mode, const Sell3& A, const __half* val,
             e1 = cycle_timer_event();
             if (e0 && e1) (void)hipEventRecord(e0, st);
         }
+    }
+    if (A.n_uni > 0 && A.uni[0].val32) {
+        // the context's operator from its reference blocks: FP32, and still fewer bytes
+        if (mode == 3) uni3_go<float, 3>(st, A, A.uni[0], x, y, f, nullptr, nullptr);
+        else uni3_go<float, 0>(st, A, A.uni[0], x, y, f, nullptr, nullptr);
+        if (e0 && e1) (void)hipEventRecord(e1, st);
+        return;
     }
     const int per = A.waves_per_block;
     const int nblk = (A.n_slices + per - 1) / per;

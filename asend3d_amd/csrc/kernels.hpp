@@ -19,6 +19,22 @@ struct Scalars {
     int n_resid;  // mixed step solve: FP64 residual evaluations so far
 };
 
+// Products with an operator on a mesh of translated copies of one element,
+// from its reference blocks (see k_uni3 in kernels.hip): y_r = sum over the
+// local positions a of row node r in its elements of w_a (K x of the element's
+// row a from its reference blocks), plus the penalty on the diagonal.  Stands for the assembled values val64 / val32
+// (null while the operator was not assembled from the reference blocks).
+struct UniOp {
+    const double* val64 = nullptr;
+    const float* val32 = nullptr;
+    const int32_t* nbr = nullptr;  // node at offset o (27, own node where there is none) of lane l: 64 (27 s + o) + l
+    const double *w64 = nullptr, *kh64 = nullptr;  // element weights 64 (8 s + a) + l, blocks 9 (8 a + b) + c, then 8 row sums
+    const float *w32 = nullptr, *kh32 = nullptr;
+    const int32_t* pslot = nullptr;  // per slice: its 64 x 3 penalty terms in pen, -1 = none (null: no penalty)
+    const double* pen64 = nullptr;
+    const float* pen32 = nullptr;
+};
+
 // Sliced-ELL fine operator: 64-row slices of 3x3 blocks (see kernels.hip).
 struct Sell3 {
     int n_rows = 0, n_slices = 0;
@@ -26,6 +42,8 @@ struct Sell3 {
     const int32_t* scol = nullptr;  // column (node row) of slot k, lane l at 64k + l
     int waves_per_block = 4;        // slices (wavefronts) per workgroup of the SpMV: 1, 2, 4 or 8
     int64_t n_slots = 0;            // slots over all slices (sptr[n_slices])
+    const UniOp* uni = nullptr;     // n_uni reference-block operators: products with the value
+    int n_uni = 0;                  // arrays they stand for go through them
 };
 // Operators whose values exceed this are streamed with non-temporal loads
 // (they cannot stay in the 256 MB Infinity Cache, and the loads then keep the
@@ -33,6 +51,8 @@ struct Sell3 {
 // cache-resident between SpMVs.
 constexpr int64_t kSellStreamBytes = 192ll << 20;
 constexpr int kSellMaxWaves = 8;
+// Entries of a reference-block operator's table: 64 3x3 blocks, 8 row sums.
+constexpr int kUniCoefs = 64 * 9 + 8;
 
 // Index of component c (= 3i + j) of block k of row r in the value array.
 __host__ __device__ inline int64_t sell_index(const int32_t* sptr, int r, int k, int c) {
@@ -103,6 +123,17 @@ void launch_to_f32(hipStream_t st, const double* a, float* b, int64_t n);
 void launch_diag_inv(hipStream_t st, int n_rows, const int32_t* sptr, const int32_t* kdiag, const double* K,
                      double* d64, float* d32);
 
+// Tables of a reference-block operator: weights (scale times E per element,
+// or times 1 where E is null), and kUniCoefs entries: the blocks sK Khat + sM
+// Mhat I and their rows' sums over b (sM sum Mhat_ab), in FP64 and FP32.
+void launch_uni_weights(hipStream_t st, int n_slices, const int32_t* el, const double* E, double scale, double* w64,
+                        float* w32);
+void launch_uni_coef(hipStream_t st, const double* Khat, const double* Mhat, double sK, double sM, double* kh64,
+                     float* kh32);
+// penalty terms mult sf of the DOFs pen into the slices' 64 x 3 tables (cleared here)
+void launch_uni_penalty(hipStream_t st, const int64_t* pen, const int32_t* mult, int n_pen, double sf,
+                        const int32_t* pslot, int n_pslots, double* pen64, float* pen32);
+
 // Sliced-ELL SpMV, same modes as launch_spmv3, plus mode 4: y = K x with
 // x = u, f = r and the single-reduction PCG scalars (launch_cg1_*).
 template <typename T>
@@ -119,7 +150,8 @@ void launch_to_f16_rowscaled(hipStream_t st, int n_rows, int n_slices, const int
 void kernel_timer_start();
 int kernel_timer_stop(int64_t* launches, double* total_ms);
 // SpMV with that copy, FP32 accumulation, the row scale restored from the
-// FP32 Jacobi diagonal: mode 0: y = K x; mode 3: y = f - K x.
+// FP32 Jacobi diagonal: mode 0: y = K x; mode 3: y = f - K x.  Where
+// A.uni[0] stands for the operator it is taken instead.
 void launch_sell3_h(hipStream_t st, int mode, const Sell3& A, const __half* val, const float* dinv32, const float* x,
                     float* y, const float* f);
 

@@ -311,10 +311,11 @@ def main():
     log(f"SpMV fp32 {ms32 * 1e3:.1f} us ({gbs32:.0f} GB/s), fp64 {ms64 * 1e3:.1f} us ({gbs64:.0f} GB/s); "
         f"copy {copy_gbs:.0f} GB/s")
     # the timed step's leading kernel, timed inside the pipeline: the
-    # multigrid cycle's FP16 row-scaled SpMV with residual epilogue (y = f - K x:
-    # FP16 values and int32 columns once, x gathered, f, the FP32 row scale
-    # and y once each), HIP events around each of its launches on the context
-    # stream during one more step run with graphs off
+    # multigrid cycle's finest operator product with residual epilogue (y = f - K x),
+    # HIP events around each of its launches on the context stream during one
+    # more step run with graphs off.  On this mesh of translated elements it
+    # comes from the reference blocks: per node 27 int32 neighbours, 8 FP32
+    # weights, x, f and y once each
     cyc = None
     if pc != api.PC_JACOBI:
         ctx.set_graphs(False)
@@ -323,11 +324,11 @@ def main():
         n_cyc, ms_cyc = ctx.cycle_spmv_timing(False)
         ctx.set_graphs(True)
         if n_cyc:
-            cyc_bytes = nnzb * (9 * 2 + 4) + (n_rows + 1) * 4 + prob.n_dof * 4 * 4
+            cyc_bytes = n_rows * (27 + 8) * 4 + prob.n_dof * 4 * 3
             cyc_ms = ms_cyc / n_cyc
             cyc = {"launches": n_cyc, "avg_ms": cyc_ms, "bytes_per_launch": cyc_bytes,
                    "achieved": cyc_bytes / (cyc_ms * 1e-3) / 1e9}
-            log(f"cycle SpMV in the pipeline: {n_cyc} launches, {cyc_ms * 1e3:.2f} us each, "
+            log(f"cycle product in the pipeline: {n_cyc} launches, {cyc_ms * 1e3:.2f} us each, "
                 f"{cyc['achieved']:.0f} GB/s")
 
     c2 = (args.nx, args.ny, args.nz) == (200, 40, 40)
@@ -357,7 +358,7 @@ def main():
         "config": {"workload": f"hex8 cantilever {args.nx}x{args.ny}x{args.nz} static + compliance adjoint",
                    "n_dof": prob.n_dof, "n_elements": prob.mesh.n_el, "tol": args.tol,
                    "fast_precond": {api.PC_JACOBI: "jacobi", api.PC_MG: "mg", api.PC_LEARNED: "learned"}[pc],
-                   "cycle_storage": "fp16 row-scaled finest operator and learned factor (fp32 arithmetic)",
+                   "cycle_storage": "fp32 products from the reference blocks on the finest level, fp16 learned factor",
                    "training": train,
                    "autotune": tuning,
                    "parallelism": "single GPU"},
@@ -376,9 +377,9 @@ def main():
         "wall_s_timed": wall,
         "roofline": ({"bound": "hbm", "achieved": cyc["achieved"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                       "frac": cyc["achieved"] / HBM_PEAK_GBS,
-                      "traffic": measured_traffic("traffic_bytes_per_launch_fp16_cycle", "sell3h_cycle_c2_pmc.md")
-                      if c2 else None,
-                      "kernel": "k_sell3h<3> FP16 cycle SpMV, y = f - K x (timed inside the pipeline)",
+                      "traffic": None,
+                      "kernel": "k_uni3<float, 3> cycle product from the reference blocks, y = f - K x (timed "
+                                "inside the pipeline)",
                       "bytes_per_launch": cyc["bytes_per_launch"], "avg_ms": cyc["avg_ms"],
                       "launches_per_step": cyc["launches"]} if cyc else
                      {"bound": "hbm", "achieved": gbs32, "peak": HBM_PEAK_GBS, "unit": "GB/s",
