@@ -112,7 +112,11 @@ struct asend_ctx {
            *d_sens = nullptr, *d_x64 = nullptr, *d_r2 = nullptr;
     float *d_r32 = nullptr, *d_x32 = nullptr, *d_p32 = nullptr, *d_q32 = nullptr, *d_w32 = nullptr;
 
-    int64_t partials_cap = kMaxPartials;  // blocks whose partial sums d_partials can hold
+    // blocks whose partial sums (3 each) d_partials can hold; behind them the
+    // second reduction's partials of a step and the folded ones
+    int64_t partials_cap = kMaxPartials;
+    double* partials2() const { return d_partials + 3 * partials_cap; }
+    double* fold() const { return partials2() + 2 * kStepBlocks; }
     Scalars* d_sc = nullptr;  // [0] outer/FP64 loop, [1] inner FP32 loop, [2] misc
     Scalars* h_sc = nullptr;  // pinned mirror
     double* d_partials = nullptr;
@@ -197,7 +201,7 @@ struct asend_ctx {
         double *fac = nullptr, *hist = nullptr;
         int64_t *step = nullptr, *its = nullptr, *watch = nullptr;
         int64_t fac_cap = 0, hist_cap = 0, watch_cap = 0;
-        hipGraphExec_t exec_head = nullptr, exec_more = nullptr, exec_tail = nullptr;
+        hipGraphExec_t exec_head = nullptr, exec_more = nullptr, exec_long = nullptr, exec_tail = nullptr;
         int graph_iters = -1, graph_watch = -1;
         // displacement history for the adjoint sweep (save_u: where the step
         // tail stores u, null when not recording) and the adjoint vectors
@@ -326,7 +330,7 @@ void newmark_free(asend_ctx* ctx) {
     nm.fac_cap = nm.hist_cap = nm.watch_cap = nm.uhist_cap = 0;
     nm.save_u = nullptr;
     nm.graph_save = nullptr;
-    for (hipGraphExec_t* e : {&nm.exec_head, &nm.exec_more, &nm.exec_tail}) {
+    for (hipGraphExec_t* e : {&nm.exec_head, &nm.exec_more, &nm.exec_long, &nm.exec_tail}) {
         if (*e) (void)hipGraphExecDestroy(*e);
         *e = nullptr;
     }
@@ -457,15 +461,17 @@ __global__ void k_sub_f32(int64_t n, const float* __restrict__ a, const float* _
 // Device buffers of the FP64 Jacobi PCG solve (ASEND_SOLVE_PCG_FP64): the
 // right-hand side f, the solution u, the outer residual r = f - K u, the
 // correction x of one PCG run, its residual r2, direction p and product q
-// (n_dof doubles each), the reduction partials (2 kMaxPartials doubles) and
-// two loop scalars (sc[0] the outer FP64 residual, sc[1] the PCG run).
+// (n_dof doubles each), the reduction partials (those of every product
+// workgroup, then a step's second ones and the folded ones) and four loop
+// scalars (sc[0] the outer FP64 residual, sc[1] and sc[3] the PCG run).
 struct Fp64Bufs {
-    double *f, *u, *r, *x, *r2, *p, *q, *partials;
+    double *f, *u, *r, *x, *r2, *p, *q, *partials, *partials2, *fold;
     Scalars* sc;
 };
 
 Fp64Bufs ctx_fp64_bufs(asend_ctx* ctx) {
-    return {ctx->d_f, ctx->d_u, ctx->d_r, ctx->d_x64, ctx->d_r2, ctx->d_p, ctx->d_q, ctx->d_partials, ctx->d_sc};
+    return {ctx->d_f, ctx->d_u, ctx->d_r, ctx->d_x64, ctx->d_r2, ctx->d_p, ctx->d_q, ctx->d_partials,
+            ctx->partials2(), ctx->fold(), ctx->d_sc};
 }
 
 __global__ void k_fill64(int64_t n, double v, double* __restrict__ x) {
@@ -489,11 +495,12 @@ int run_jacobi_pcg64(asend_ctx* ctx, const Fp64Bufs& B, double tol, bool stop_ab
     int rc;
     if ((rc = write_scalars_to(ctx, sc, 1))) return rc;
     launch_pcg_init<double>(ctx->st, n, B.r, dinv, B.x, B.r2, B.p, B.partials, sc);
+    Scalars* const slots[2] = {sc, B.sc + 3};
+    const Sell3 A = ctx->fine();
     for (;;) {
         for (int k = 0; k < check_every; ++k) {
-            launch_sell3<double>(ctx->st, 1, ctx->fine(), K, B.p, B.q, nullptr, B.partials, sc);
-            launch_pcg_update<double>(ctx->st, n, dinv, B.x, B.r2, B.p, B.q, B.partials, sc);
-            launch_pcg_dir<double>(ctx->st, n, dinv, B.r2, B.p, sc);
+            launch_pcg_iteration<double>(ctx->st, n, A, K, dinv, B.x, B.r2, B.p, B.q, B.partials, B.partials2, B.fold,
+                                         slots);
         }
         HIPCHK(hipGetLastError());
         if ((rc = read_scalars_from(ctx, sc, 1))) return rc;
@@ -571,14 +578,14 @@ int run_ldl_pcg64(asend_ctx* ctx, const Fp64Bufs& B, double tol, bool stop_abs, 
     double* z = ctx->d_ldl_z;
     launch_pcgz_start(ctx->st, n, B.r, B.x, B.r2);
     ldl_solve_launch(ctx->st, F.d, F.L, B.r2, z, F.work, nullptr);
-    launch_pcgz_dots(ctx->st, n, B.r2, z, B.p, true, B.partials, sc);
+    launch_pcgz_init(ctx->st, n, B.r2, z, B.p, B.partials, sc);
+    Scalars* const slots[2] = {sc, B.sc + 3};
+    const Sell3 A = ctx->fine();
     for (;;) {
         for (int k = 0; k < check_every; ++k) {
-            launch_sell3<double>(ctx->st, 1, ctx->fine(), ctx->d_K64, B.p, B.q, nullptr, B.partials, sc);
-            launch_pcgz_update(ctx->st, n, B.x, B.r2, B.p, B.q, sc);
+            launch_pcgz_step(ctx->st, n, A, ctx->d_K64, B.x, B.r2, B.p, B.q, B.partials, B.fold, slots);
             ldl_solve_launch(ctx->st, F.d, F.L, B.r2, z, F.work, &sc->done);
-            launch_pcgz_dots(ctx->st, n, B.r2, z, B.p, false, B.partials, sc);
-            launch_pcgz_dir(ctx->st, n, z, B.p, sc);
+            launch_pcgz_dir(ctx->st, n, B.r2, z, B.p, B.partials2, slots);
         }
         HIPCHK(hipGetLastError());
         if ((rc = read_scalars_from(ctx, sc, 1))) return rc;
@@ -662,13 +669,15 @@ int run_cg1_pcg(asend_ctx* ctx, int si, const double* b, double* x, bool warm, d
     Scalars* sc = ctx->d_sc + si;
     if (warm) launch_sell3<double>(ctx->st, 3, ctx->fine(), ctx->d_K64, x, ctx->d_r2, b, nullptr, nullptr);
     launch_cg1_init<double>(ctx->st, n, b, !warm, ctx->d_dinv64, x, ctx->d_r2, u, ctx->d_p, s, ctx->d_partials, sc);
+    Scalars* const slots[2] = {sc, ctx->d_sc + 3};
+    const Sell3 A = ctx->fine();
+    int cur = 0;
     for (;;) {
-        for (int k = 0; k < check_every; ++k) {
-            launch_sell3<double>(ctx->st, 4, ctx->fine(), ctx->d_K64, u, ctx->d_q, ctx->d_r2, ctx->d_partials, sc);
-            launch_cg1_update<double>(ctx->st, n, ctx->d_dinv64, x, ctx->d_r2, u, ctx->d_q, ctx->d_p, s, sc);
-        }
+        for (int k = 0; k < check_every; ++k)
+            launch_cg1_iteration<double>(ctx->st, n, A, ctx->d_K64, ctx->d_dinv64, x, ctx->d_r2, u, ctx->d_q, ctx->d_p,
+                                         s, ctx->d_partials, ctx->fold(), slots, &cur);
         HIPCHK(hipGetLastError());
-        if ((rc = read_scalars(ctx, si))) return rc;
+        if ((rc = read_scalars_from(ctx, slots[cur], si))) return rc;
         if (h.done) break;
     }
     return ASEND_OK;
@@ -698,7 +707,7 @@ int run_jacobi_fpcg_ru(asend_ctx* ctx, FcgRefresh& ru, double& rr, double ff, do
         for (int k = 0; k < check_every; ++k) {
             launch_sell3<float>(ctx->st, 7, ctx->fine(), ctx->d_K32, p, q, r, ctx->d_partials, sc);
             launch_fpcg_update<float>(ctx->st, n, dinv, x, r, p, q, ctx->d_partials, sc);
-            launch_pcg_dir<float>(ctx->st, n, dinv, r, p, sc);
+            launch_fpcg_dir<float>(ctx->st, n, dinv, r, p, sc);
         }
         HIPCHK(hipGetLastError());
         if ((rc = read_scalars(ctx, 1))) return rc;
@@ -738,7 +747,7 @@ int residual64(asend_ctx* ctx, const double* f, const double* u, double* r) {
 // solve that needs more has failed to cut iterations and the solve falls back
 // to Jacobi PCG.
 constexpr int64_t kLearnedInnerBudget = 300;
-constexpr int kNewmarkBlock = 24;  // PCG iterations per captured block of a Newmark step
+constexpr int kNewmarkBlock = 16;  // PCG iterations per long captured block of a Newmark step
 constexpr int kMixedRefreshEvery = 4;  // mixed step solver: iterations between reliable-update slots
 // ASEND_NM_AUTO takes the mixed step solver above this FP64 operator size
 constexpr int64_t kMixedAutoBytes = 128ll << 20;
@@ -1312,8 +1321,12 @@ int nl_assemble(asend_ctx* ctx, double fact, double* rhs) {
 namespace {
 constexpr int64_t kNoAllocMaxDof = 1 << 18;
 constexpr int64_t kNoAllocPartials = 2 * (int64_t)kMaxPartials;
-constexpr int64_t kNoAllocScalarDoubles = 64;  // room for the two Scalars
-static_assert(2 * sizeof(Scalars) <= kNoAllocScalarDoubles * sizeof(double), "scalar slot too small");
+// every product workgroup's partial (one per 64-row slice at most) and the
+// 2 kVecBlocks of the start leave room for the tail
+static_assert(kNoAllocPartials - kStepTail >= 2 * kVecBlocks && kNoAllocPartials - kStepTail >= kNoAllocMaxDof / 192 + 1,
+              "partials of the allocation-free solve");
+constexpr int64_t kNoAllocScalarDoubles = 64;  // room for the four Scalars
+static_assert(4 * sizeof(Scalars) <= kNoAllocScalarDoubles * sizeof(double), "scalar slot too small");
 constexpr int64_t kNoAllocDoubles = 7 * kNoAllocMaxDof + kNoAllocPartials + kNoAllocScalarDoubles;
 constexpr int kScratchDevices = 64;
 }  // namespace
@@ -1356,6 +1369,8 @@ Fp64Bufs scratch_fp64_bufs(double* base) {
     B.p = base + 5 * v;
     B.q = base + 6 * v;
     B.partials = base + 7 * v;
+    B.partials2 = B.partials + kNoAllocPartials - kStepTail;
+    B.fold = B.partials2 + 2 * kStepBlocks;
     B.sc = (Scalars*)(base + 7 * v + kNoAllocPartials);
     return B;
 }
@@ -1401,7 +1416,7 @@ int asend_ctx_create(int device, asend_ctx** out) {
     if (hipStreamCreateWithFlags(&ctx->st, hipStreamNonBlocking) != hipSuccess ||
         hipMalloc((void**)&ctx->d_sc, 4 * sizeof(Scalars)) != hipSuccess ||
         hipHostMalloc((void**)&ctx->h_sc, 4 * sizeof(Scalars), hipHostMallocDefault) != hipSuccess ||
-        hipMalloc((void**)&ctx->d_partials, kMaxPartials * 3 * sizeof(double)) != hipSuccess ||
+        hipMalloc((void**)&ctx->d_partials, (kMaxPartials * 3 + kStepTail) * sizeof(double)) != hipSuccess ||
         hipMalloc((void**)&ctx->d_counter, 16 * sizeof(unsigned)) != hipSuccess ||
         hipEventCreate(&ctx->ev0) != hipSuccess || hipEventCreate(&ctx->ev1) != hipSuccess ||
         hipStreamCreateWithFlags(&ctx->st2, hipStreamNonBlocking) != hipSuccess ||
@@ -1652,7 +1667,7 @@ int asend_upload_mesh(asend_ctx* ctx, int elem_type, int64_t n_mesh_nodes, const
     ctx->n_slots = ctx->h_sptr[ctx->n_slices];
     // the SpMV with one slice per workgroup writes one partial per slice
     if (ctx->n_slices > ctx->partials_cap) {
-        int rc0 = dalloc(ctx, &ctx->d_partials, 3 * (size_t)ctx->n_slices);
+        int rc0 = dalloc(ctx, &ctx->d_partials, 3 * (size_t)ctx->n_slices + kStepTail);
         if (rc0) return rc0;
         ctx->partials_cap = ctx->n_slices;
     }
@@ -2756,32 +2771,41 @@ int asend_newmark_run(asend_ctx* ctx, int64_t n_steps, const double* f_shape, co
     mx.p32 = f + 3 * n;
     mx.s32 = f + 4 * n;
     mx.partials = ctx->d_partials;
-    mx.sc = sc;
+    mx.fold = ctx->fold();
+    Scalars* const slots[2] = {sc, ctx->d_sc + 3};
+    mx.sc[0] = slots[0];
+    mx.sc[1] = slots[1];
     mx.n = n;
     mx.ru_factor = nm.inner_tol;
     const int nw = (int)n_watch;
-    // A step is three launch sequences: head (effective load, PCG start and a
-    // first block of iterations), more (another block, repeated until the
-    // step's solve has converged: one small device-to-host read per block),
-    // tail (state update and history).  Each is captured once as a hipGraph.
-    const int blk = std::min(max_it_step, kNewmarkBlock);
-    // single-reduction Jacobi PCG: x = du, r, u = Dinv r, w = K u, p, s = K p;
+    // A step is head (effective load, PCG start), blocks of iterations and tail
+    // (state update and history), each captured once as a hipGraph.  Blocks
+    // come in two lengths: as many as the previous step needed go off without
+    // a word to the host, then the shorter ones, each after a small
+    // device-to-host read, until the step's solve has converged.  (With blocks of 24
+    // only, 57.6 iterations were launched for the 41.4 a step needs on 100x20x20,
+    // each idle one 4.5 us.)
+    // Single-reduction Jacobi PCG: x = du, r, u = Dinv r, w = K u, p, s = K p;
     // mixed: the same recurrence in FP32 with x in FP64, and a reliable-update
     // slot after every kMixedRefreshEvery iterations (a no-op unless a refresh
-    // is pending; the iterations pause while one is)
+    // is pending; the iterations pause while one is).  A block leaves the loop
+    // scalars in the slot it found them in.
     const bool mixed = nm.mixed == ASEND_NM_MIXED || (nm.mixed == ASEND_NM_AUTO && 8 * ctx->nval() > kMixedAutoBytes);
-    auto iterations = [&]() {
-        for (int k = 0; k < blk; ++k) {
+    const int blk = mixed ? 2 * kMixedRefreshEvery : 4;
+    auto iterations = [&](int count) {
+        int cur = 0;
+        for (int k = 0; k < count; ++k) {
             if (mixed) {
-                launch_mixed_iteration(ctx->st, mx);
-                if ((k + 1) % kMixedRefreshEvery == 0 || k + 1 == blk) launch_mixed_refresh(ctx->st, mx);
+                launch_mixed_iteration(ctx->st, mx, &cur);
+                if ((k + 1) % kMixedRefreshEvery == 0) launch_mixed_refresh(ctx->st, mx, &cur);
             } else {
-                launch_sell3<double>(ctx->st, 4, A, ctx->d_K64, nm.cg_u, ctx->d_q, ctx->d_r2, ctx->d_partials, sc);
-                launch_cg1_update<double>(ctx->st, n, ctx->d_dinv64, ctx->d_x64, ctx->d_r2, nm.cg_u, ctx->d_q,
-                                          ctx->d_p, nm.cg_s, sc);
+                launch_cg1_iteration<double>(ctx->st, n, A, ctx->d_K64, ctx->d_dinv64, ctx->d_x64, ctx->d_r2, nm.cg_u,
+                                             ctx->d_q, ctx->d_p, nm.cg_s, ctx->d_partials, ctx->fold(), slots, &cur);
             }
         }
     };
+    static_assert(kNewmarkBlock % (2 * kMixedRefreshEvery) == 0 && kNewmarkBlock % 4 == 0, "block lengths");
+    static_assert((2 * kMixedRefreshEvery + 2) % 2 == 0, "a mixed block returns to its scalar slot");
     auto head = [&]() {
         launch_nm_predict(ctx->st, n, ctx->d_u, nm.v, nm.a, nm.dt, nm.c2, nm.w);
         launch_sell3<double>(ctx->st, 0, ctx->fine(), nm.M64, nm.w, nm.q, nullptr, nullptr, nullptr);
@@ -2802,7 +2826,6 @@ int asend_newmark_run(asend_ctx* ctx, int64_t n_steps, const double* f_shape, co
             launch_cg1_init<double>(ctx->st, n, nm.rhs, false, ctx->d_dinv64, ctx->d_x64, ctx->d_r2, nm.cg_u,
                                     ctx->d_p, nm.cg_s, ctx->d_partials, sc);
         }
-        iterations();
     };
     auto tail = [&]() {
         launch_nm_update(ctx->st, n, ctx->d_x64, nm.w, nm.c_m, nm.dt, nm.gamma, ctx->d_u, nm.v, nm.a);
@@ -2834,8 +2857,8 @@ int asend_newmark_run(asend_ctx* ctx, int64_t n_steps, const double* f_shape, co
     if (graph && (!nm.exec_head || nm.graph_iters != blk || nm.graph_watch != nw || nm.graph_save != nm.save_u ||
                   nm.graph_save_y != nm.save_y || nm.graph_mixed != (int)mixed || nm.graph_ru != mx.ru_factor ||
                   nm.graph_wpb != A.waves_per_block || nm.graph_uni != (ctx->uni[0].val64 ? 1 : 0))) {
-        if ((rc = capture(&nm.exec_head, head)) || (rc = capture(&nm.exec_more, iterations)) ||
-            (rc = capture(&nm.exec_tail, tail)))
+        if ((rc = capture(&nm.exec_head, head)) || (rc = capture(&nm.exec_more, [&]() { iterations(blk); })) ||
+            (rc = capture(&nm.exec_long, [&]() { iterations(kNewmarkBlock); })) || (rc = capture(&nm.exec_tail, tail)))
             return rc;
         nm.graph_iters = blk;
         nm.graph_watch = nw;
@@ -2847,15 +2870,30 @@ int asend_newmark_run(asend_ctx* ctx, int64_t n_steps, const double* f_shape, co
         nm.graph_uni = ctx->uni[0].val64 ? 1 : 0;
     }
     HIPCHK(hipEventRecord(ctx->ev0, ctx->st));
+    int64_t expect = kNewmarkBlock;  // iterations launched before the first read of a step
     for (int64_t s = 0; s < n_steps; ++s) {
         if (graph) HIPCHK(hipGraphLaunch(nm.exec_head, ctx->st));
         else head();
+        int64_t launched = 0;
+        while (launched < expect) {
+            const bool lng = expect - launched > kNewmarkBlock - blk;
+            if (graph) HIPCHK(hipGraphLaunch(lng ? nm.exec_long : nm.exec_more, ctx->st));
+            else iterations(lng ? kNewmarkBlock : blk);
+            launched += lng ? kNewmarkBlock : blk;
+        }
+        bool more = false;
         for (;;) {
             if ((rc = read_scalars(ctx, 1))) return rc;
             if (ctx->h_sc[1].done) break;
             if (graph) HIPCHK(hipGraphLaunch(nm.exec_more, ctx->st));
-            else iterations();
+            else iterations(blk);
+            launched += blk;
+            more = true;
         }
+        // FP64: a convergence test more than its iterations; mixed: pauses for
+        // the refreshes come on top, so what it took, one block less after a
+        // step that needed no second look
+        expect = mixed ? (more ? launched : std::max<int64_t>(launched - blk, blk)) : ctx->h_sc[1].it + 1;
         if (graph) HIPCHK(hipGraphLaunch(nm.exec_tail, ctx->st));
         else tail();
     }

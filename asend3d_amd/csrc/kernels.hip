@@ -518,18 +518,137 @@ enum FinOp {
     FIN_MAX = 5,
     FIN_CG1_INIT = 7,
     FIN_CG1 = 8,
-    FIN_RU_RES = 9,
     FIN_CG1_RU = 10,
     FIN_PQR = 11,
-    FIN_FUPD = 12
+    FIN_FUPD = 12,
+    FIN_RU_LOAD = 13
 };
+
+// whether a finalize has nothing to add: its loop is done, or paused
+__host__ __device__ constexpr int fin_values(int op) {
+    return (op == FIN_INIT || op == FIN_UPDATE || op == FIN_PQR || op == FIN_FUPD)
+               ? 2
+               : ((op == FIN_CG1 || op == FIN_CG1_RU) ? 3 : 1);
+}
+
+__device__ __forceinline__ bool fin_idle(int op, const Scalars& s) {
+    if (op == FIN_PQ || op == FIN_UPDATE || op == FIN_CG1 || op == FIN_PQR || op == FIN_FUPD) return s.done;
+    if (op == FIN_RU_LOAD) return !s.gate;
+    if (op == FIN_CG1_RU) return s.done || s.gate;
+    return false;
+}
+
+// the loop scalars after the sums t of a finalize
+__device__ __forceinline__ void fin_apply(int op, double t0, double t1, double t2, Scalars& s) {
+    switch (op) {
+        case FIN_PQ:
+            s.pq = t0;
+            s.alpha = s.rz / t0;
+            break;
+        case FIN_RR:
+            s.rr = t0;
+            break;
+        case FIN_DOT:
+            s.dot = t0;
+            break;
+        case FIN_INIT:
+            s.rz = t0;
+            s.rr = t1;
+            s.ff = t1;
+            s.it = 0;
+            s.done = (s.stop_abs ? (t0 <= s.tol) : (t1 <= s.tol2 * t1)) || t1 == 0.0;
+            break;
+        case FIN_CG1_INIT:
+            // single-reduction PCG start: t0 = |b|^2
+            s.ff = t0;
+            s.rz = 0.0;
+            s.it = 0;
+            s.done = t0 == 0.0;
+            break;
+        case FIN_CG1: {
+            // single-reduction PCG: t0 = gamma = r.u, t1 = delta = (K u).u,
+            // t2 = r.r of the current residual
+            const double g = t0, d = t1;
+            s.rr = t2;
+            const bool conv = s.stop_abs ? (g <= s.tol) : (t2 <= s.tol2 * s.ff);
+            if (conv || s.it >= s.max_it) {
+                s.done = 1;
+                break;
+            }
+            const double beta = s.it == 0 ? 0.0 : g / s.rz;
+            const double den = s.it == 0 ? d : d - beta * g / s.alpha;
+            if (!(den > 0.0)) {  // lost positive definiteness: stop, reported unconverged
+                s.done = 1;
+                break;
+            }
+            s.beta = beta;
+            s.alpha = g / den;
+            s.rz = g;
+            s.it += 1;
+            break;
+        }
+        case FIN_RU_LOAD:
+            // reliable update: the FP64 residual decides convergence
+            s.rr = t0;
+            s.n_resid += 1;
+            s.gate = 0;
+            if (t0 <= s.tol2 * s.ff || s.n_resid >= kMixedMaxRefresh || s.it >= s.max_it) s.done = 1;
+            break;
+        case FIN_CG1_RU: {
+            // FP32 single-reduction step; s.rr is the FP64 residual of the
+            // last refresh, s.zq the refresh factor squared
+            const double g = t0, d = t1;
+            s.pq = t2;  // recursive residual, FP32 recurrence
+            if (t2 <= s.zq * s.rr || t2 <= s.tol2 * s.ff) {
+                s.gate = 1;
+                break;
+            }
+            if (s.it >= s.max_it) {
+                s.done = 1;
+                break;
+            }
+            const double beta = s.it == 0 ? 0.0 : g / s.rz;
+            const double den = s.it == 0 ? d : d - beta * g / s.alpha;
+            if (!(den > 0.0)) {
+                s.done = 1;
+                break;
+            }
+            s.beta = beta;
+            s.alpha = g / den;
+            s.rz = g;
+            s.it += 1;
+            break;
+        }
+        case FIN_PQR:
+            // flexible step length: t0 = p.q, t1 = p.r
+            s.pq = t0;
+            s.alpha = t1 / t0;
+            break;
+        case FIN_FUPD: {
+            // flexible direction: t0 = (Dinv r).q, t1 = r.r
+            s.beta = -t0 / s.pq;
+            s.rr = t1;
+            s.it += 1;
+            if (t1 <= s.tol2 * s.ff || s.it >= s.max_it || !(t1 == t1)) s.done = 1;
+            break;
+        }
+        case FIN_UPDATE: {
+            s.beta = t0 / s.rz;
+            s.rz = t0;
+            s.rr = t1;
+            s.it += 1;
+            bool conv = s.stop_abs ? (t0 <= s.tol) : (t1 <= s.tol2 * s.ff);
+            if (conv || s.it >= s.max_it) s.done = 1;
+            break;
+        }
+        default:
+            break;
+        }
+}
 
 __global__ __launch_bounds__(kBlock) void k_finalize(const double* __restrict__ partials, int nparts, int op,
                                                      Scalars* sc) {
-    if ((op == FIN_PQ || op == FIN_UPDATE || op == FIN_CG1) && sc->done) return;
-    if (op == FIN_RU_RES && !sc->gate) return;
-    if (op == FIN_CG1_RU && (sc->done || sc->gate)) return;
-    if ((op == FIN_PQR || op == FIN_FUPD) && sc->done) return;
+    if (fin_idle(op, *sc)) return;
     if (op == FIN_MAX) {
         double m = 0.0;
         for (int b = threadIdx.x; b < nparts; b += blockDim.x) m = fmax(m, partials[b]);
@@ -544,10 +663,9 @@ __global__ __launch_bounds__(kBlock) void k_finalize(const double* __restrict__ 
         }
         return;
     }
-    const int nv = (op == FIN_INIT || op == FIN_UPDATE || op == FIN_PQR || op == FIN_FUPD)
-                       ? 2
-                       : ((op == FIN_CG1 || op == FIN_CG1_RU) ? 3 : 1);
+    const int nv = fin_values(op);
     double t[3] = {0.0, 0.0, 0.0};
+#pragma unroll 4
     for (int b = threadIdx.x; b < nparts; b += blockDim.x) {
         t[0] += partials[(size_t)nv * b];
         if (nv >= 2) t[1] += partials[(size_t)nv * b + 1];
@@ -555,112 +673,55 @@ __global__ __launch_bounds__(kBlock) void k_finalize(const double* __restrict__ 
     }
     block_sum<3>(t);
     if (threadIdx.x != 0) return;
-    switch (op) {
-        case FIN_PQ:
-            sc->pq = t[0];
-            sc->alpha = sc->rz / t[0];
-            break;
-        case FIN_RR:
-            sc->rr = t[0];
-            break;
-        case FIN_DOT:
-            sc->dot = t[0];
-            break;
-        case FIN_INIT:
-            sc->rz = t[0];
-            sc->rr = t[1];
-            sc->ff = t[1];
-            sc->it = 0;
-            sc->done = (sc->stop_abs ? (t[0] <= sc->tol) : (t[1] <= sc->tol2 * t[1])) || t[1] == 0.0;
-            break;
-        case FIN_CG1_INIT:
-            // single-reduction PCG start: t0 = |b|^2
-            sc->ff = t[0];
-            sc->rz = 0.0;
-            sc->it = 0;
-            sc->done = t[0] == 0.0;
-            break;
-        case FIN_CG1: {
-            // single-reduction PCG: t0 = gamma = r.u, t1 = delta = (K u).u,
-            // t2 = r.r of the current residual
-            const double g = t[0], d = t[1];
-            sc->rr = t[2];
-            const bool conv = sc->stop_abs ? (g <= sc->tol) : (t[2] <= sc->tol2 * sc->ff);
-            if (conv || sc->it >= sc->max_it) {
-                sc->done = 1;
-                break;
-            }
-            const double beta = sc->it == 0 ? 0.0 : g / sc->rz;
-            const double den = sc->it == 0 ? d : d - beta * g / sc->alpha;
-            if (!(den > 0.0)) {  // lost positive definiteness: stop, reported unconverged
-                sc->done = 1;
-                break;
-            }
-            sc->beta = beta;
-            sc->alpha = g / den;
-            sc->rz = g;
-            sc->it += 1;
-            break;
-        }
-        case FIN_RU_RES:
-            // reliable update: the FP64 residual decides convergence
-            sc->rr = t[0];
-            sc->n_resid += 1;
-            if (t[0] <= sc->tol2 * sc->ff || sc->n_resid >= kMixedMaxRefresh || sc->it >= sc->max_it) {
-                sc->done = 1;
-                sc->gate = 0;
-            }
-            break;
-        case FIN_CG1_RU: {
-            // FP32 single-reduction step; sc->rr is the FP64 residual of the
-            // last refresh, sc->zq the refresh factor squared
-            const double g = t[0], d = t[1];
-            sc->pq = t[2];  // recursive residual, FP32 recurrence
-            if (t[2] <= sc->zq * sc->rr || t[2] <= sc->tol2 * sc->ff) {
-                sc->gate = 1;
-                break;
-            }
-            if (sc->it >= sc->max_it) {
-                sc->done = 1;
-                break;
-            }
-            const double beta = sc->it == 0 ? 0.0 : g / sc->rz;
-            const double den = sc->it == 0 ? d : d - beta * g / sc->alpha;
-            if (!(den > 0.0)) {
-                sc->done = 1;
-                break;
-            }
-            sc->beta = beta;
-            sc->alpha = g / den;
-            sc->rz = g;
-            sc->it += 1;
-            break;
-        }
-        case FIN_PQR:
-            // flexible step length: t0 = p.q, t1 = p.r
-            sc->pq = t[0];
-            sc->alpha = t[1] / t[0];
-            break;
-        case FIN_FUPD: {
-            // flexible direction: t0 = (Dinv r).q, t1 = r.r
-            sc->beta = -t[0] / sc->pq;
-            sc->rr = t[1];
-            sc->it += 1;
-            if (t[1] <= sc->tol2 * sc->ff || sc->it >= sc->max_it || !(t[1] == t[1])) sc->done = 1;
-            break;
-        }
-        case FIN_UPDATE: {
-            sc->beta = t[0] / sc->rz;
-            sc->rz = t[0];
-            sc->rr = t[1];
-            sc->it += 1;
-            bool conv = sc->stop_abs ? (t[0] <= sc->tol) : (t[1] <= sc->tol2 * sc->ff);
-            if (conv || sc->it >= sc->max_it) sc->done = 1;
-            break;
-        }
-        default:
-            break;
-    }
+    fin_apply(op, t[0], t[1], t[2], *sc);
+}
+
+// The finalize of a Krylov step inside the vector kernel that needs it: every
+// block adds the previous launch's partial sums itself, in the same order, so all
+// hold the same scalars; block 0 stores them to out, another slot than in (which
+// other blocks may still be reading).  One launch less per reduction than
+// a one-block kernel between the two, which costs 3.7 us at 700 partials and 7 us
+// at 5,280 against 1 to 2 us here: an iteration on 44,541 nodes (FP64, single
+// reduction) 15.5 -> 14.6 us, on 337,881 nodes (textbook, two reductions) 61.4 ->
+// 52.7 us.
+// The sums are formed whether or not there is anything to do, so that no load
+// waits for another.
+template <int OP>
+__device__ __forceinline__ void step_scalars(const Scalars* __restrict__ in, const double* __restrict__ partials,
+                                             int nparts, Scalars* __restrict__ out, Scalars& sh) {
+    constexpr int nv = fin_values(OP);
+    constexpr int kWords = sizeof(Scalars) / sizeof(double);
+    static_assert(sizeof(Scalars) % sizeof(double) == 0 && kWords <= kWave, "copied by one wavefront");
+    // the last wavefront brings the scalars in, beside the others' sums
+    const int c = (int)threadIdx.x - (kBlock - kWave);
+    if (c >= 0 && c < kWords) reinterpret_cast<double*>(&sh)[c] = reinterpret_cast<const double*>(in)[c];
+    double v[nv];
+#pragma unroll
+    for (int i = 0; i < nv; ++i) v[i] = 0.0;
+#pragma unroll 4
+    for (int b = threadIdx.x; b < nparts; b += kBlock)
+#pragma unroll
+        for (int i = 0; i < nv; ++i) v[i] += partials[(size_t)nv * b + i];
+    block_sum<nv>(v);
+    if (threadIdx.x == 0 && !fin_idle(OP, sh)) fin_apply(OP, v[0], v[nv >= 2 ? 1 : 0], v[nv == 3 ? 2 : 0], sh);
+    __syncthreads();
+    if (blockIdx.x == 0 && threadIdx.x < kWords)
+        reinterpret_cast<double*>(out)[threadIdx.x] = reinterpret_cast<const double*>(&sh)[threadIdx.x];
+}
+
+// Partial sums of more blocks than kStepParts folded to kFoldBlocks, in order.
+template <int NV>
+__global__ __launch_bounds__(kBlock) void k_fold(const double* __restrict__ partials, int nparts,
+                                                 double* __restrict__ out) {
+    const int per = (nparts + gridDim.x - 1) / gridDim.x;
+    const int b0 = blockIdx.x * per, b1 = min(nparts, b0 + per);
+    double v[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) v[i] = 0.0;
+    for (int b = b0 + threadIdx.x; b < b1; b += kBlock)
+#pragma unroll
+        for (int i = 0; i < NV; ++i) v[i] += partials[(size_t)NV * b + i];
+    block_partials<NV>(v, out);
 }
 
 static void finalize(hipStream_t st, const double* partials, int nparts, int op, Scalars* sc) {
@@ -744,38 +805,52 @@ __device__ __forceinline__ T sell_load(const T* p) {
 }
 
 // Row epilogue of the operator products (modes at the block-row SpMV below):
-// (a0, a1, a2) = row r of K x; writes y and adds to the row's partial sums.
+// a = row r of K x, xr and fr the row's own values of x and f (where the mode
+// reads them); writes y and adds to the row's partial sums.
+template <int MODE>
+constexpr bool mode_reads_f() {
+    return MODE >= 2;
+}
+
 template <typename T, int MODE>
-__device__ __forceinline__ void row_epilogue(int r, T a0, T a1, T a2, const T* __restrict__ x, T* __restrict__ y,
-                                             const T* __restrict__ f, double (&part)[3]) {
+__device__ __forceinline__ void row_epilogue(int r, const T (&a)[3], const T (&xr)[3], const T (&fr)[3],
+                                             T* __restrict__ y, double (&part)[3]) {
     const int64_t d = 3 * (int64_t)r;
     if (MODE == 2 || MODE == 3 || MODE == 5) {
-        const T y0 = f[d] - a0, y1 = f[d + 1] - a1, y2 = f[d + 2] - a2;
+        const T y0 = fr[0] - a[0], y1 = fr[1] - a[1], y2 = fr[2] - a[2];
         y[d] = y0;
         y[d + 1] = y1;
         y[d + 2] = y2;
-        part[0] = (double)y0 * y0 + (double)y1 * y1 + (double)y2 * y2;
+        part[0] += (double)y0 * y0 + (double)y1 * y1 + (double)y2 * y2;
         return;
     }
-    y[d] = a0;
-    y[d + 1] = a1;
-    y[d + 2] = a2;
+    y[d] = a[0];
+    y[d + 1] = a[1];
+    y[d + 2] = a[2];
     if (MODE == 0) return;
-    const double x0 = x[d], x1 = x[d + 1], x2 = x[d + 2];
-    const double kx = (double)a0 * x0 + (double)a1 * x1 + (double)a2 * x2;
-    if (MODE == 1) part[0] = kx;
+    const double x0 = xr[0], x1 = xr[1], x2 = xr[2];
+    const double kx = (double)a[0] * x0 + (double)a[1] * x1 + (double)a[2] * x2;
+    if (MODE == 1) part[0] += kx;
     if (MODE == 7) {
         // x = p, f = r: partials p.(K p) and p.r
-        part[0] = kx;
-        part[1] = x0 * f[d] + x1 * f[d + 1] + x2 * f[d + 2];
+        part[0] += kx;
+        part[1] += x0 * fr[0] + x1 * fr[1] + x2 * fr[2];
     }
     if (MODE == 4 || MODE == 6) {
         // x = u (preconditioned residual), f = r: partials r.u, (K u).u, r.r
-        const double r0 = f[d], r1 = f[d + 1], r2 = f[d + 2];
-        part[0] = r0 * x0 + r1 * x1 + r2 * x2;
-        part[1] = kx;
-        part[2] = r0 * r0 + r1 * r1 + r2 * r2;
+        const double r0 = fr[0], r1 = fr[1], r2 = fr[2];
+        part[0] += r0 * x0 + r1 * x1 + r2 * x2;
+        part[1] += kx;
+        part[2] += r0 * r0 + r1 * r1 + r2 * r2;
     }
+}
+
+// the three values of row r
+template <typename T>
+__device__ __forceinline__ void row_values(const T* __restrict__ v, int r, T (&o)[3]) {
+    const T* p = v + 3 * (int64_t)r;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) o[i] = p[i];
 }
 
 // the block's partial sums of a mode, stored for its finalize kernel
@@ -836,7 +911,13 @@ __global__ __launch_bounds__(kSellMaxWaves * kWave) void k_sell3(int n_rows, int
             cp += kWave;
             vp += 9 * kWave;
         }
-        if (r < n_rows) row_epilogue<T, MODE>(r, a0, a1, a2, x, y, f, part);
+        if (r < n_rows) {
+            const T a[3] = {a0, a1, a2};
+            T xr[3] = {0, 0, 0}, fr[3] = {0, 0, 0};
+            if (MODE == 1 || MODE == 4 || MODE == 6 || MODE == 7) row_values(x, r, xr);
+            if (mode_reads_f<MODE>()) row_values(f, r, fr);
+            row_epilogue<T, MODE>(r, a, xr, fr, y, part);
+        }
     }
     mode_partials<MODE>(part, partials);
 }
@@ -884,39 +965,49 @@ __host__ __device__ constexpr int uni_node(int x, int y, int z) {
     return (x < 0 || x > 1 || y < 0 || y > 1 || z < 0 || z > 1) ? -1 : 4 * z + 2 * y + (x ^ y);
 }
 
-// rows' products over the positions A0 and A0 + 1; xr: the row's own values,
-// kh: blocks 9 (8 a + b) + c, then the 8 row sums
-template <typename T, int A0>
-__device__ __forceinline__ void uni_rows(const int32_t* __restrict__ nb, const T* __restrict__ w,
+// offsets that the positions A0 and A0 + 1 reach (their own node left out)
+__host__ __device__ constexpr bool uni_used(int A0, int o) {
+    const int dx = o % 3 - 1, dy = o / 3 % 3 - 1, dz = o / 9 - 1;
+    return o != 13 && (uni_node(uni_px(A0) + dx, uni_py(A0) + dy, uni_pz(A0) + dz) >= 0 ||
+                       uni_node(uni_px(A0 + 1) + dx, uni_py(A0 + 1) + dy, uni_pz(A0 + 1) + dz) >= 0);
+}
+
+// rows' products over the positions A0 and A0 + 1 into a; x_r: the row's own
+// values, kh: blocks 9 (8 a + b) + c, then the 8 row sums.  The indices and
+// weights are on their way while the loop scalars (check) tell whether there is
+// anything to do: false if not.
+template <typename T, int A0, int MODE>
+__device__ __forceinline__ bool uni_rows(const int32_t* __restrict__ nb, const T* __restrict__ w,
                                          const T* __restrict__ kh, const T* __restrict__ x, const T (&xr)[3],
-                                         T (&y)[3]) {
+                                         bool check, const Scalars* sc, T (&y)[3]) {
     constexpr int NA = 2;
+    int32_t c[27];
+#pragma unroll
+    for (int o = 0; o < 27; ++o)
+        if (uni_used(A0, o)) c[o] = nb[64 * o];
     T t[NA][3], wa[NA];
 #pragma unroll
-    for (int a = 0; a < NA; ++a) {
-        wa[a] = w[64 * (A0 + a)];
+    for (int a = 0; a < NA; ++a) wa[a] = w[64 * (A0 + a)];
+    if (check && mode_idle<MODE>(sc)) return false;
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
 #pragma unroll
         for (int i = 0; i < 3; ++i) t[a][i] = kh[576 + A0 + a] * xr[i];
-    }
 #pragma unroll
     for (int dz = -1; dz <= 1; ++dz) {
         T xs[9][3];
 #pragma unroll
         for (int j = 0; j < 9; ++j) {
-            const int dx = j % 3 - 1, dy = j / 3 - 1;
-            bool used = false;
+            const int o = 9 * (dz + 1) + j;
+            if (!uni_used(A0, o)) continue;
+            const T* xp = x + 3 * (int64_t)c[o];
 #pragma unroll
-            for (int a = A0; a < A0 + NA; ++a)
-                used = used || uni_node(uni_px(a) + dx, uni_py(a) + dy, uni_pz(a) + dz) >= 0;
-            if (!used || (dz == 0 && j == 4)) continue;
-            const int64_t c = 3 * (int64_t)nb[64 * (9 * (dz + 1) + j)];
-#pragma unroll
-            for (int i = 0; i < 3; ++i) xs[j][i] = x[c + i];
+            for (int i = 0; i < 3; ++i) xs[j][i] = xp[i];
         }
 #pragma unroll
         for (int j = 0; j < 9; ++j) {
             const int dx = j % 3 - 1, dy = j / 3 - 1;
-            if (dz == 0 && j == 4) continue;
+            if (!uni_used(A0, 9 * (dz + 1) + j)) continue;
 #pragma unroll
             for (int i = 0; i < 3; ++i) xs[j][i] -= xr[i];
 #pragma unroll
@@ -934,47 +1025,54 @@ __device__ __forceinline__ void uni_rows(const int32_t* __restrict__ nb, const T
     for (int a = 0; a < NA; ++a)
 #pragma unroll
         for (int i = 0; i < 3; ++i) y[i] += wa[a] * t[a][i];
+    return true;
 }
 
 template <typename T, int MODE>
-__global__ __launch_bounds__(kUniWaves * kWave) void k_uni3(int n_rows, const int32_t* __restrict__ nbr,
+__global__ __launch_bounds__(kUniWaves * kWave) void k_uni3(int n_rows, int n_slices, int per,
+                                                            const int32_t* __restrict__ nbr,
                                                             const T* __restrict__ w, const T* __restrict__ kh,
                                                             const int32_t* __restrict__ pslot,
                                                             const T* __restrict__ pen, const T* __restrict__ x,
                                                             T* __restrict__ y, const T* __restrict__ f,
                                                             double* partials, const Scalars* sc) {
-    if (mode_idle<MODE>(sc)) return;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int slice = xcd_block(blockIdx.x, gridDim.x);
-    const int r = 64 * slice + lane;
-    const int32_t* nb = nbr + (int64_t)27 * 64 * slice + lane;
-    const T* wl = w + (int64_t)8 * 64 * slice + lane;
-    const T* xp = x + 3 * (int64_t)min(r, n_rows - 1);
-    const T xr[3] = {xp[0], xp[1], xp[2]};
-    T a[3] = {0, 0, 0};
-    if (wv == 0) uni_rows<T, 0>(nb, wl, kh, x, xr, a);
-    else if (wv == 1) uni_rows<T, 2>(nb, wl, kh, x, xr, a);
-    else if (wv == 2) uni_rows<T, 4>(nb, wl, kh, x, xr, a);
-    else uni_rows<T, 6>(nb, wl, kh, x, xr, a);
     __shared__ T sh[3][kUniWaves - 1][kWave];
-    if (wv > 0) {
-#pragma unroll
-        for (int i = 0; i < 3; ++i) sh[i][wv - 1][lane] = a[i];
-    }
-    __syncthreads();
     double part[3] = {0.0, 0.0, 0.0};
-    if (wv == 0 && r < n_rows) {
+    const int s0 = xcd_block(blockIdx.x, gridDim.x) * per, s1 = min(s0 + per, n_slices);
+    for (int slice = s0; slice < s1; ++slice) {
+        const int r = 64 * slice + lane, rc = min(r, n_rows - 1);
+        const int32_t* nb = nbr + (int64_t)27 * 64 * slice + lane;
+        const T* wl = w + (int64_t)8 * 64 * slice + lane;
+        T a[3] = {0, 0, 0}, xr[3], fr[3] = {0, 0, 0};
+        row_values(x, rc, xr);
+        if (mode_reads_f<MODE>() && wv == 0) row_values(f, rc, fr);
+        const bool first = slice == s0;
+        bool live;
+        if (wv == 0) live = uni_rows<T, 0, MODE>(nb, wl, kh, x, xr, first, sc, a);
+        else if (wv == 1) live = uni_rows<T, 2, MODE>(nb, wl, kh, x, xr, first, sc, a);
+        else if (wv == 2) live = uni_rows<T, 4, MODE>(nb, wl, kh, x, xr, first, sc, a);
+        else live = uni_rows<T, 6, MODE>(nb, wl, kh, x, xr, first, sc, a);
+        if (!live) return;  // the same for the whole workgroup
+        if (slice > s0) __syncthreads();  // the previous slice's sums are read
+        if (wv > 0) {
 #pragma unroll
-        for (int v = 0; v < kUniWaves - 1; ++v)
-#pragma unroll
-            for (int i = 0; i < 3; ++i) a[i] += sh[i][v][lane];
-        const int ps = pslot ? pslot[slice] : -1;
-        if (ps >= 0) {
-            const T* pp = pen + 192 * (int64_t)ps + 3 * lane;
-#pragma unroll
-            for (int i = 0; i < 3; ++i) a[i] += pp[i] * xr[i];
+            for (int i = 0; i < 3; ++i) sh[i][wv - 1][lane] = a[i];
         }
-        row_epilogue<T, MODE>(r, a[0], a[1], a[2], x, y, f, part);
+        __syncthreads();
+        if (wv == 0 && r < n_rows) {
+#pragma unroll
+            for (int v = 0; v < kUniWaves - 1; ++v)
+#pragma unroll
+                for (int i = 0; i < 3; ++i) a[i] += sh[i][v][lane];
+            const int ps = pslot ? pslot[slice] : -1;
+            if (ps >= 0) {
+                const T* pp = pen + 192 * (int64_t)ps + 3 * lane;
+#pragma unroll
+                for (int i = 0; i < 3; ++i) a[i] += pp[i] * xr[i];
+            }
+            row_epilogue<T, MODE>(r, a, xr, fr, y, part);
+        }
     }
     mode_partials<MODE>(part, partials);
 }
@@ -1055,9 +1153,11 @@ static int uni3_go(hipStream_t st, const Sell3& A, const UniOp& U, const T* x, T
         kh = U.kh32;
         pen = U.pen32;
     }
-    hipLaunchKernelGGL((k_uni3<T, MODE>), dim3(A.n_slices), dim3(kUniWaves * kWave), 0, st, A.n_rows, U.nbr, w, kh,
-                       U.pslot, pen, x, y, f, partials, sc);
-    return A.n_slices;
+    // at most kStepParts workgroups: the step kernels add that many partials
+    const int per = (A.n_slices + kStepParts - 1) / kStepParts, nblk = (A.n_slices + per - 1) / per;
+    hipLaunchKernelGGL((k_uni3<T, MODE>), dim3(nblk), dim3(kUniWaves * kWave), 0, st, A.n_rows, A.n_slices, per, U.nbr,
+                       w, kh, U.pslot, pen, x, y, f, partials, sc);
+    return nblk;
 }
 
 // the reference-block operator that stands for val, null if none does
@@ -1097,20 +1197,8 @@ void launch_sell3(hipStream_t st, int mode, const Sell3& A, const T* val, const 
         case 0:
             sell3_go<T, 0>(st, A, val, x, y, f, partials, sc);
             break;
-        case 1:
-            finalize(st, partials, sell3_go<T, 1>(st, A, val, x, y, f, partials, sc), FIN_PQ, sc);
-            break;
         case 2:
             finalize(st, partials, sell3_go<T, 2>(st, A, val, x, y, f, partials, sc), FIN_RR, sc);
-            break;
-        case 4:
-            finalize(st, partials, sell3_go<T, 4>(st, A, val, x, y, f, partials, sc), FIN_CG1, sc);
-            break;
-        case 5:
-            finalize(st, partials, sell3_go<T, 5>(st, A, val, x, y, f, partials, sc), FIN_RU_RES, sc);
-            break;
-        case 6:
-            finalize(st, partials, sell3_go<T, 6>(st, A, val, x, y, f, partials, sc), FIN_CG1_RU, sc);
             break;
         case 7:
             finalize(st, partials, sell3_go<T, 7>(st, A, val, x, y, f, partials, sc), FIN_PQR, sc);
@@ -1120,6 +1208,42 @@ void launch_sell3(hipStream_t st, int mode, const Sell3& A, const T* val, const 
             break;
     }
 }
+
+template <typename T>
+StepParts launch_sell3_step(hipStream_t st, int mode, const Sell3& A, const T* val, const T* x, T* y, const T* f,
+                            double* partials, double* fold, const Scalars* sc_in) {
+    Scalars* sc = const_cast<Scalars*>(sc_in);  // read only
+    StepParts P;
+    P.p = partials;
+    int nv = 1;
+    switch (mode) {
+        case 1:
+            P.n = sell3_go<T, 1>(st, A, val, x, y, f, partials, sc);
+            break;
+        case 4:
+            P.n = sell3_go<T, 4>(st, A, val, x, y, f, partials, sc);
+            nv = 3;
+            break;
+        case 5:
+            P.n = sell3_go<T, 5>(st, A, val, x, y, f, partials, sc);
+            break;
+        default:
+            P.n = sell3_go<T, 6>(st, A, val, x, y, f, partials, sc);
+            nv = 3;
+            break;
+    }
+    if (P.n > kStepParts) {
+        if (nv == 1) hipLaunchKernelGGL(k_fold<1>, dim3(kFoldBlocks), dim3(kBlock), 0, st, partials, P.n, fold);
+        else hipLaunchKernelGGL(k_fold<3>, dim3(kFoldBlocks), dim3(kBlock), 0, st, partials, P.n, fold);
+        P.p = fold;
+        P.n = kFoldBlocks;
+    }
+    return P;
+}
+template StepParts launch_sell3_step<double>(hipStream_t, int, const Sell3&, const double*, const double*, double*,
+                                             const double*, double*, double*, const Scalars*);
+template StepParts launch_sell3_step<float>(hipStream_t, int, const Sell3&, const float*, const float*, float*,
+                                            const float*, double*, double*, const Scalars*);
 
 template void launch_sell3<double>(hipStream_t, int, const Sell3&, const double*, const double*, double*,
                                    const double*, double*, Scalars*);
@@ -1288,15 +1412,17 @@ void launch_sell3_h(hipStream_t st, int mode, const Sell3& A, const __half* val,
 // ---------------------------------------------------------------------------
 // Block-row SpMV, b = 3, G lanes per block row, component-major values.
 // MODE 0: y = K x
-// MODE 1: y = K x and (x . y) -> finalize: sc->pq, sc->alpha = sc->rz / pq
+// MODE 1: y = K x and (x . y): with launch_sell3_step the PCG step length
 // MODE 2: y = f - K x (x = current solution, f = load) -> finalize: sc->rr = |y|^2
 // MODE 3: y = f - K x without the norm
 // MODE 4 (sliced-ELL only): y = K x with x = u = Dinv r and f = r, partials of
-//   r.u, y.u and r.r -> finalize: the single-reduction PCG step scalars
+//   r.u, y.u and r.r (the single-reduction PCG step)
 // MODE 5 (sliced-ELL only): MODE 2 when sc->gate is set (mixed solve's
-//   reliable update) -> finalize: sc->rr, convergence on the FP64 residual
-// MODE 6 (sliced-ELL only): MODE 4 paused while sc->gate is set -> finalize:
-//   the mixed solve's FP32 step scalars, or a refresh request
+//   reliable update: convergence on the FP64 residual)
+// MODE 6 (sliced-ELL only): MODE 4 paused while sc->gate is set (the mixed
+//   solve's FP32 step, or a refresh request)
+//   Modes 1, 4, 5 and 6 leave their partials to the step's vector kernel
+//   (launch_sell3_step).
 // MODE 7 (sliced-ELL only): y = K x with x = p and f = r, partials of p.y and
 //   p.r -> finalize: the flexible PCG step length alpha = p.r / p.q
 // Kernels with a scalars pointer return at once when sc->done is set.
@@ -1405,29 +1531,60 @@ __global__ __launch_bounds__(kBlock) void k_pcg_init(int64_t n, const T* __restr
     block_partials<2>(t, partials);
 }
 
-// x += alpha p; r -= alpha q; partials of r.(Dinv r) and r.r
+// p.(K p) -> alpha; x += alpha p; r -= alpha q; partials of r.(Dinv r) and r.r
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_pcg_update(int64_t n, const T* __restrict__ dinv, T* __restrict__ x,
                                                        T* __restrict__ r, const T* __restrict__ p,
-                                                       const T* __restrict__ q, double* partials,
-                                                       const Scalars* sc) {
-    if (sc->done) return;
-    const T alpha = (T)sc->alpha;
+                                                       const T* __restrict__ q, StepParts in, double* partials,
+                                                       const Scalars* s_in, Scalars* s_out) {
+    __shared__ Scalars sc;
+    struct Entry {
+        T x, p, r, q, d;
+    };
+    auto load = [&](int64_t i) { return Entry{x[i], p[i], r[i], q[i], dinv[i]}; };
+    const int64_t step = (int64_t)gridDim.x * blockDim.x, i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    Entry e = load(i0 < n ? i0 : n - 1);
+    step_scalars<FIN_PQ>(s_in, in.p, in.n, s_out, sc);
+    if (sc.done) return;
+    const T alpha = (T)sc.alpha;
     double t[2] = {0.0, 0.0};
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        x[i] += alpha * p[i];
-        T ri = r[i] - alpha * q[i];
+    for (int64_t i = i0; i < n; i += step) {
+        if (i > i0) e = load(i);
+        x[i] = e.x + alpha * e.p;
+        T ri = e.r - alpha * e.q;
         r[i] = ri;
-        t[0] += (double)ri * (dinv[i] * ri);
+        t[0] += (double)ri * (e.d * ri);
         t[1] += (double)ri * ri;
     }
     block_partials<2>(t, partials);
 }
 
-// p = Dinv r + beta p
+// r.z, r.r -> beta and the stop test; p = Dinv r + beta p
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_pcg_dir(int64_t n, const T* __restrict__ dinv, const T* __restrict__ r,
-                                                    T* __restrict__ p, const Scalars* __restrict__ sc) {
+                                                    T* __restrict__ p, StepParts in, const Scalars* s_in,
+                                                    Scalars* s_out) {
+    __shared__ Scalars sc;
+    const int64_t step = (int64_t)gridDim.x * blockDim.x, i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t j = i0 < n ? i0 : n - 1;
+    T d = dinv[j], ri = r[j], pi = p[j];
+    step_scalars<FIN_UPDATE>(s_in, in.p, in.n, s_out, sc);
+    if (sc.done) return;
+    const T beta = (T)sc.beta;
+    for (int64_t i = i0; i < n; i += step) {
+        if (i > i0) {
+            d = dinv[i];
+            ri = r[i];
+            pi = p[i];
+        }
+        p[i] = d * ri + beta * pi;
+    }
+}
+
+// p = Dinv r + beta p with the scalars already formed
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_fpcg_dir(int64_t n, const T* __restrict__ dinv, const T* __restrict__ r,
+                                                     T* __restrict__ p, const Scalars* __restrict__ sc) {
     if (sc->done) return;
     const T beta = (T)sc->beta;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
@@ -1459,23 +1616,27 @@ __global__ __launch_bounds__(kBlock) void k_pcgz_dots(int64_t n, const double* _
     block_partials<2>(t, partials);
 }
 
-// x += alpha p; r -= alpha q
+// p.(K p) -> alpha; x += alpha p; r -= alpha q
 __global__ __launch_bounds__(kBlock) void k_pcgz_update(int64_t n, double* __restrict__ x, double* __restrict__ r,
                                                         const double* __restrict__ p, const double* __restrict__ q,
-                                                        const Scalars* __restrict__ sc) {
-    if (sc->done) return;
-    const double alpha = sc->alpha;
+                                                        StepParts in, const Scalars* s_in, Scalars* s_out) {
+    __shared__ Scalars sc;
+    step_scalars<FIN_PQ>(s_in, in.p, in.n, s_out, sc);
+    if (sc.done) return;
+    const double alpha = sc.alpha;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         x[i] += alpha * p[i];
         r[i] -= alpha * q[i];
     }
 }
 
-// p = z + beta p
+// r.z, r.r -> beta and the stop test; p = z + beta p
 __global__ __launch_bounds__(kBlock) void k_pcgz_dir(int64_t n, const double* __restrict__ z, double* __restrict__ p,
-                                                     const Scalars* __restrict__ sc) {
-    if (sc->done) return;
-    const double beta = sc->beta;
+                                                     StepParts in, const Scalars* s_in, Scalars* s_out) {
+    __shared__ Scalars sc;
+    step_scalars<FIN_UPDATE>(s_in, in.p, in.n, s_out, sc);
+    if (sc.done) return;
+    const double beta = sc.beta;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         p[i] = z[i] + beta * p[i];
 }
@@ -1516,19 +1677,29 @@ __global__ __launch_bounds__(kBlock) void k_cg1_init(int64_t n, const T* __restr
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_cg1_update(int64_t n, const T* __restrict__ dinv, T* __restrict__ x,
                                                        T* __restrict__ r, T* __restrict__ u, const T* __restrict__ w,
-                                                       T* __restrict__ p, T* __restrict__ s,
-                                                       const Scalars* __restrict__ sc) {
-    if (sc->done) return;
-    const T alpha = (T)sc->alpha, beta = (T)sc->beta;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const T pi = u[i] + beta * p[i];
-        const T si = w[i] + beta * s[i];
+                                                       T* __restrict__ p, T* __restrict__ s, StepParts in,
+                                                       const Scalars* s_in, Scalars* s_out) {
+    __shared__ Scalars sc;
+    // the first entry's operands come in while the scalars are formed
+    struct Entry {
+        T u, p, w, s, x, r, d;
+    };
+    auto load = [&](int64_t i) { return Entry{u[i], p[i], w[i], s[i], x[i], r[i], dinv[i]}; };
+    const int64_t step = (int64_t)gridDim.x * blockDim.x, i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    Entry e = load(i0 < n ? i0 : n - 1);
+    step_scalars<FIN_CG1>(s_in, in.p, in.n, s_out, sc);
+    if (sc.done) return;
+    const T alpha = (T)sc.alpha, beta = (T)sc.beta;
+    for (int64_t i = i0; i < n; i += step) {
+        if (i > i0) e = load(i);
+        const T pi = e.u + beta * e.p;
+        const T si = e.w + beta * e.s;
         p[i] = pi;
         s[i] = si;
-        x[i] += alpha * pi;
-        const T ri = r[i] - alpha * si;
+        x[i] = e.x + alpha * pi;
+        const T ri = e.r - alpha * si;
         r[i] = ri;
-        u[i] = dinv[i] * ri;
+        u[i] = e.d * ri;
     }
 }
 
@@ -1585,7 +1756,8 @@ void launch_cg1_init(hipStream_t st, int64_t n, const T* b, bool cold, const T* 
 }
 
 // --- mixed-precision solve under device-side control ----------------------
-__global__ void k_ru_start(Scalars* __restrict__ sc, double ru2) {
+__global__ void k_ru_start(const Scalars* __restrict__ in, Scalars* __restrict__ sc, double ru2) {
+    *sc = *in;
     sc->ff = sc->dot;
     sc->rr = sc->dot;
     sc->zq = ru2;
@@ -1600,29 +1772,43 @@ __global__ void k_ru_start(Scalars* __restrict__ sc, double ru2) {
 __global__ __launch_bounds__(kBlock) void k_cg1_update_mx(int64_t n, const float* __restrict__ dinv,
                                                           double* __restrict__ x, float* __restrict__ r,
                                                           float* __restrict__ u, const float* __restrict__ w,
-                                                          float* __restrict__ p, float* __restrict__ s,
-                                                          const Scalars* __restrict__ sc) {
-    if (sc->done || sc->gate) return;
-    const float alpha = (float)sc->alpha, beta = (float)sc->beta;
-    const double alpha64 = sc->alpha;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const float pi = u[i] + beta * p[i];
-        const float si = w[i] + beta * s[i];
+                                                          float* __restrict__ p, float* __restrict__ s, StepParts in,
+                                                          const Scalars* s_in, Scalars* s_out) {
+    __shared__ Scalars sc;
+    struct Entry {
+        float u, p, w, s, r, d;
+        double x;
+    };
+    auto load = [&](int64_t i) { return Entry{u[i], p[i], w[i], s[i], r[i], dinv[i], x[i]}; };
+    const int64_t step = (int64_t)gridDim.x * blockDim.x, i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    Entry e = load(i0 < n ? i0 : n - 1);
+    step_scalars<FIN_CG1_RU>(s_in, in.p, in.n, s_out, sc);
+    if (sc.done || sc.gate) return;
+    const float alpha = (float)sc.alpha, beta = (float)sc.beta;
+    const double alpha64 = sc.alpha;
+    for (int64_t i = i0; i < n; i += step) {
+        if (i > i0) e = load(i);
+        const float pi = e.u + beta * e.p;
+        const float si = e.w + beta * e.s;
         p[i] = pi;
         s[i] = si;
-        x[i] += alpha64 * (double)pi;
-        const float ri = r[i] - alpha * si;
+        x[i] = e.x + alpha64 * (double)pi;
+        const float ri = e.r - alpha * si;
         r[i] = ri;
-        u[i] = dinv[i] * ri;
+        u[i] = e.d * ri;
     }
 }
-// reliable update: r = (float) r64, u = Dinv r (and p = s = 0 at the start)
+// reliable update: |r64|^2 -> the stop test, then r = (float) r64, u = Dinv r
+// (and p = s = 0 at the start), and the iterations go on
 __global__ __launch_bounds__(kBlock) void k_ru_load(int64_t n, const double* __restrict__ r64,
                                                     const float* __restrict__ dinv, float* __restrict__ r,
                                                     float* __restrict__ u, float* __restrict__ p,
-                                                    float* __restrict__ s, int restart,
-                                                    const Scalars* __restrict__ sc) {
-    if (!sc->gate) return;
+                                                    float* __restrict__ s, int restart, StepParts in,
+                                                    const Scalars* s_in, Scalars* s_out) {
+    __shared__ Scalars sc;
+    const bool due = s_in->gate;
+    step_scalars<FIN_RU_LOAD>(s_in, in.p, in.n, s_out, sc);
+    if (!due || sc.done) return;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         const float ri = (float)r64[i];
         r[i] = ri;
@@ -1633,32 +1819,42 @@ __global__ __launch_bounds__(kBlock) void k_ru_load(int64_t n, const double* __r
         }
     }
 }
-__global__ void k_ru_clear(Scalars* __restrict__ sc) { sc->gate = 0; }
 
-static void mixed_refresh(hipStream_t st, const MixedSolve& m, int restart) {
-    launch_sell3<double>(st, 5, *m.A, m.K64, m.x64, m.r64, m.rhs, m.partials, m.sc);
-    hipLaunchKernelGGL(k_ru_load, dim3(kVecBlocks), dim3(kBlock), 0, st, m.n, m.r64, m.dinv32, m.r32, m.u32, m.p32,
-                       m.s32, restart, (const Scalars*)m.sc);
-    hipLaunchKernelGGL(k_ru_clear, dim3(1), dim3(1), 0, st, m.sc);
+// one refresh slot: reads the loop scalars at *cur, leaves them in the other slot
+static void mixed_refresh(hipStream_t st, const MixedSolve& m, int* cur, int restart) {
+    const StepParts P = launch_sell3_step<double>(st, 5, *m.A, m.K64, m.x64, m.r64, m.rhs, m.partials, m.fold,
+                                                  m.sc[*cur]);
+    hipLaunchKernelGGL(k_ru_load, dim3(step_blocks(m.n)), dim3(kBlock), 0, st, m.n, m.r64, m.dinv32, m.r32, m.u32,
+                       m.p32, m.s32, restart, P, (const Scalars*)m.sc[*cur], m.sc[1 - *cur]);
+    *cur = 1 - *cur;
 }
 
 void launch_mixed_start(hipStream_t st, const MixedSolve& m) {
-    launch_dot64(st, m.n, m.rhs, m.rhs, m.partials, m.sc);
-    hipLaunchKernelGGL(k_ru_start, dim3(1), dim3(1), 0, st, m.sc, m.ru_factor * m.ru_factor);
-    mixed_refresh(st, m, 1);
+    // starts in slot 1 so that the refresh leaves the scalars in slot 0
+    launch_dot64(st, m.n, m.rhs, m.rhs, m.partials, m.sc[0]);
+    hipLaunchKernelGGL(k_ru_start, dim3(1), dim3(1), 0, st, (const Scalars*)m.sc[0], m.sc[1],
+                       m.ru_factor * m.ru_factor);
+    int cur = 1;
+    mixed_refresh(st, m, &cur, 1);
 }
 
-void launch_mixed_iteration(hipStream_t st, const MixedSolve& m) {
-    launch_sell3<float>(st, 6, *m.A, m.K32, m.u32, m.w32, m.r32, m.partials, m.sc);
-    hipLaunchKernelGGL(k_cg1_update_mx, dim3(kVecBlocks), dim3(kBlock), 0, st, m.n, m.dinv32, m.x64, m.r32, m.u32,
-                       m.w32, m.p32, m.s32, (const Scalars*)m.sc);
+void launch_mixed_iteration(hipStream_t st, const MixedSolve& m, int* cur) {
+    const StepParts P = launch_sell3_step<float>(st, 6, *m.A, m.K32, m.u32, m.w32, m.r32, m.partials, m.fold,
+                                                 m.sc[*cur]);
+    hipLaunchKernelGGL(k_cg1_update_mx, dim3(step_blocks(m.n)), dim3(kBlock), 0, st, m.n, m.dinv32, m.x64, m.r32,
+                       m.u32, m.w32, m.p32, m.s32, P, (const Scalars*)m.sc[*cur], m.sc[1 - *cur]);
+    *cur = 1 - *cur;
 }
 
-void launch_mixed_refresh(hipStream_t st, const MixedSolve& m) { mixed_refresh(st, m, 0); }
+void launch_mixed_refresh(hipStream_t st, const MixedSolve& m, int* cur) { mixed_refresh(st, m, cur, 0); }
+
 template <typename T>
-void launch_cg1_update(hipStream_t st, int64_t n, const T* dinv, T* x, T* r, T* u, const T* w, T* p, T* s,
-                       const Scalars* sc) {
-    hipLaunchKernelGGL(k_cg1_update<T>, dim3(kVecBlocks), dim3(kBlock), 0, st, n, dinv, x, r, u, w, p, s, sc);
+void launch_cg1_iteration(hipStream_t st, int64_t n, const Sell3& A, const T* K, const T* dinv, T* x, T* r, T* u, T* w,
+                          T* p, T* s, double* partials, double* fold, Scalars* const sc[2], int* cur) {
+    const StepParts P = launch_sell3_step<T>(st, 4, A, K, u, w, r, partials, fold, sc[*cur]);
+    hipLaunchKernelGGL(k_cg1_update<T>, dim3(step_blocks(n)), dim3(kBlock), 0, st, n, dinv, x, r, u, w, p, s, P,
+                       (const Scalars*)sc[*cur], sc[1 - *cur]);
+    *cur = 1 - *cur;
 }
 
 template <typename T>
@@ -1668,44 +1864,56 @@ void launch_pcg_init(hipStream_t st, int64_t n, const T* b, const T* dinv, T* x,
     finalize(st, partials, kVecBlocks, FIN_INIT, sc);
 }
 template <typename T>
-void launch_pcg_update(hipStream_t st, int64_t n, const T* dinv, T* x, T* r, const T* p, const T* q,
-                       double* partials, Scalars* sc) {
-    hipLaunchKernelGGL(k_pcg_update<T>, dim3(kVecBlocks), dim3(kBlock), 0, st, n, dinv, x, r, p, q, partials, sc);
-    finalize(st, partials, kVecBlocks, FIN_UPDATE, sc);
+void launch_pcg_iteration(hipStream_t st, int64_t n, const Sell3& A, const T* K, const T* dinv, T* x, T* r, T* p, T* q,
+                          double* partials, double* partials2, double* fold, Scalars* const sc[2]) {
+    const StepParts P = launch_sell3_step<T>(st, 1, A, K, p, q, (const T*)nullptr, partials, fold, sc[0]);
+    const int nb = step_blocks(n);
+    hipLaunchKernelGGL(k_pcg_update<T>, dim3(nb), dim3(kBlock), 0, st, n, dinv, x, r, p, q, P, partials2,
+                       (const Scalars*)sc[0], sc[1]);
+    const StepParts P2{partials2, nb};
+    hipLaunchKernelGGL(k_pcg_dir<T>, dim3(nb), dim3(kBlock), 0, st, n, dinv, r, p, P2, (const Scalars*)sc[1], sc[0]);
 }
+
 template <typename T>
-void launch_pcg_dir(hipStream_t st, int64_t n, const T* dinv, const T* r, T* p, const Scalars* sc) {
-    hipLaunchKernelGGL(k_pcg_dir<T>, dim3(kVecBlocks), dim3(kBlock), 0, st, n, dinv, r, p, sc);
+void launch_fpcg_dir(hipStream_t st, int64_t n, const T* dinv, const T* r, T* p, const Scalars* sc) {
+    hipLaunchKernelGGL(k_fpcg_dir<T>, dim3(kVecBlocks), dim3(kBlock), 0, st, n, dinv, r, p, sc);
 }
 
 void launch_pcgz_start(hipStream_t st, int64_t n, const double* b, double* x, double* r) {
     hipLaunchKernelGGL(k_pcgz_start, dim3(kVecBlocks), dim3(kBlock), 0, st, n, b, x, r);
 }
-void launch_pcgz_dots(hipStream_t st, int64_t n, const double* r, const double* z, double* p, bool init,
-                      double* partials, Scalars* sc) {
-    hipLaunchKernelGGL(k_pcgz_dots, dim3(kVecBlocks), dim3(kBlock), 0, st, n, r, z, p, init ? 1 : 0, partials, sc);
-    finalize(st, partials, kVecBlocks, init ? FIN_INIT : FIN_UPDATE, sc);
+void launch_pcgz_init(hipStream_t st, int64_t n, const double* r, const double* z, double* p, double* partials,
+                      Scalars* sc) {
+    hipLaunchKernelGGL(k_pcgz_dots, dim3(kVecBlocks), dim3(kBlock), 0, st, n, r, z, p, 1, partials, sc);
+    finalize(st, partials, kVecBlocks, FIN_INIT, sc);
 }
-void launch_pcgz_update(hipStream_t st, int64_t n, double* x, double* r, const double* p, const double* q,
-                        const Scalars* sc) {
-    hipLaunchKernelGGL(k_pcgz_update, dim3(kVecBlocks), dim3(kBlock), 0, st, n, x, r, p, q, sc);
+void launch_pcgz_step(hipStream_t st, int64_t n, const Sell3& A, const double* K, double* x, double* r,
+                      const double* p, double* q, double* partials, double* fold, Scalars* const sc[2]) {
+    const StepParts P = launch_sell3_step<double>(st, 1, A, K, p, q, nullptr, partials, fold, sc[0]);
+    hipLaunchKernelGGL(k_pcgz_update, dim3(step_blocks(n)), dim3(kBlock), 0, st, n, x, r, p, q, P,
+                       (const Scalars*)sc[0], sc[1]);
 }
-void launch_pcgz_dir(hipStream_t st, int64_t n, const double* z, double* p, const Scalars* sc) {
-    hipLaunchKernelGGL(k_pcgz_dir, dim3(kVecBlocks), dim3(kBlock), 0, st, n, z, p, sc);
+void launch_pcgz_dir(hipStream_t st, int64_t n, const double* r, const double* z, double* p, double* partials2,
+                     Scalars* const sc[2]) {
+    const int nb = step_blocks(n);
+    hipLaunchKernelGGL(k_pcgz_dots, dim3(nb), dim3(kBlock), 0, st, n, r, z, p, 0, partials2, (const Scalars*)sc[1]);
+    const StepParts P2{partials2, nb};
+    hipLaunchKernelGGL(k_pcgz_dir, dim3(nb), dim3(kBlock), 0, st, n, z, p, P2, (const Scalars*)sc[1], sc[0]);
 }
 
 #define INST_PCG(T)                                                                                               \
     template void launch_pcg_init<T>(hipStream_t, int64_t, const T*, const T*, T*, T*, T*, double*, Scalars*);    \
-    template void launch_pcg_update<T>(hipStream_t, int64_t, const T*, T*, T*, const T*, const T*, double*,       \
-                                       Scalars*);                                                                 \
-    template void launch_pcg_dir<T>(hipStream_t, int64_t, const T*, const T*, T*, const Scalars*);               \
+    template void launch_fpcg_dir<T>(hipStream_t, int64_t, const T*, const T*, T*, const Scalars*);              \
     template void launch_cg1_init<T>(hipStream_t, int64_t, const T*, bool, const T*, T*, T*, T*, T*, T*, double*, \
                                      Scalars*);                                                                   \
-    template void launch_cg1_update<T>(hipStream_t, int64_t, const T*, T*, T*, T*, const T*, T*, T*,              \
-                                       const Scalars*);                                                           \
     template void launch_fpcg_update<T>(hipStream_t, int64_t, const T*, T*, T*, const T*, const T*, double*,      \
                                         Scalars*);                                                                \
     template void launch_ru_reload<T>(hipStream_t, int64_t, const T*, const T*, T*, T*, double);
+template void launch_pcg_iteration<double>(hipStream_t, int64_t, const Sell3&, const double*, const double*, double*,
+                                           double*, double*, double*, double*, double*, double*, Scalars* const[2]);
+template void launch_cg1_iteration<double>(hipStream_t, int64_t, const Sell3&, const double*, const double*, double*,
+                                           double*, double*, double*, double*, double*, double*, double*,
+                                           Scalars* const[2], int*);
 INST_PCG(double)
 INST_PCG(float)
 

@@ -134,8 +134,7 @@ void launch_uni_coef(hipStream_t st, const double* Khat, const double* Mhat, dou
 void launch_uni_penalty(hipStream_t st, const int64_t* pen, const int32_t* mult, int n_pen, double sf,
                         const int32_t* pslot, int n_pslots, double* pen64, float* pen32);
 
-// Sliced-ELL SpMV, same modes as launch_spmv3, plus mode 4: y = K x with
-// x = u, f = r and the single-reduction PCG scalars (launch_cg1_*).
+// Sliced-ELL SpMV: modes 0, 2 and 3 as launch_spmv3, and 7 (flexible PCG).
 template <typename T>
 void launch_sell3(hipStream_t st, int mode, const Sell3& A, const T* val, const T* x, T* y, const T* f,
                   double* partials, Scalars* sc);
@@ -155,7 +154,30 @@ int kernel_timer_stop(int64_t* launches, double* total_ms);
 void launch_sell3_h(hipStream_t st, int mode, const Sell3& A, const __half* val, const float* dinv32, const float* x,
                     float* y, const float* f);
 
-// mode 0: y = K x; 1: y = K x, sc->pq = x.y, sc->alpha = sc->rz/pq; 2: y = f - K x, sc->rr = |y|^2
+// Partial sums of a launch, added by the vector kernel that follows it.
+struct StepParts {
+    const double* p = nullptr;
+    int n = 0;
+};
+// A step's vector kernels run on at most kStepBlocks workgroups, each adding
+// the previous launch's partials itself; more than kStepParts of those (20 kB and
+// up per workgroup) are folded to kFoldBlocks by a launch of their own first.
+constexpr int kStepBlocks = 1024;
+constexpr int kStepParts = 2048;
+constexpr int kFoldBlocks = 64;
+// doubles behind a solver's partials: the second reduction's and the folded ones
+constexpr int64_t kStepTail = 2 * kStepBlocks + 3 * kFoldBlocks;
+inline int step_blocks(int64_t n) {
+    const int64_t b = (n + 255) / 256;
+    return (int)(b < 1 ? 1 : (b < kStepBlocks ? b : kStepBlocks));
+}
+// Modes 1, 4, 5 and 6 of the operator product (the scalars at sc decide whether
+// they have work) with their partials left in place (or in fold).
+template <typename T>
+StepParts launch_sell3_step(hipStream_t st, int mode, const Sell3& A, const T* val, const T* x, T* y, const T* f,
+                            double* partials, double* fold, const Scalars* sc);
+
+// mode 0: y = K x; 1 (block rows only): y = K x, sc->pq = x.y, sc->alpha = sc->rz/pq; 2: y = f - K x, sc->rr = |y|^2
 // 3: y = f - K x (no norm).  Modes 1 and 2 launch their single-block finalize kernel after the SpMV.
 template <typename T>
 void launch_spmv3(hipStream_t st, int mode, int n_rows, const int32_t* rp, const int32_t* bc, const T* val,
@@ -164,28 +186,33 @@ void launch_spmv3(hipStream_t st, int mode, int n_rows, const int32_t* rp, const
 template <typename T>
 void launch_pcg_init(hipStream_t st, int64_t n, const T* b, const T* dinv, T* x, T* r, T* p, double* partials,
                      Scalars* sc);
+// One textbook Jacobi PCG iteration: the product with p.q, x, r and their
+// dot products, then the direction.  The loop scalars are read and left in sc[0],
+// sc[1] holds them in between; partials2: 2 kStepBlocks doubles.
 template <typename T>
-void launch_pcg_update(hipStream_t st, int64_t n, const T* dinv, T* x, T* r, const T* p, const T* q,
-                       double* partials, Scalars* sc);
-template <typename T>
-void launch_pcg_dir(hipStream_t st, int64_t n, const T* dinv, const T* r, T* p, const Scalars* sc);
+void launch_pcg_iteration(hipStream_t st, int64_t n, const Sell3& A, const T* K, const T* dinv, T* x, T* r, T* p, T* q,
+                          double* partials, double* partials2, double* fold, Scalars* const sc[2]);
 // Flexible Jacobi PCG step (after launch_sell3 mode 7): x += alpha p,
-// r -= alpha q, beta = -(Dinv r).q / p.q; then launch_pcg_dir.
+// r -= alpha q, beta = -(Dinv r).q / p.q; then launch_fpcg_dir: p = Dinv r + beta p.
 template <typename T>
 void launch_fpcg_update(hipStream_t st, int64_t n, const T* dinv, T* x, T* r, const T* p, const T* q,
                         double* partials, Scalars* sc);
+template <typename T>
+void launch_fpcg_dir(hipStream_t st, int64_t n, const T* dinv, const T* r, T* p, const Scalars* sc);
 // reliable update of a flexible PCG: r = b; p *= ratio (ratio = 0: p = Dinv r)
 template <typename T>
 void launch_ru_reload(hipStream_t st, int64_t n, const T* b, const T* dinv, T* r, T* p, double ratio);
 // Single-reduction Jacobi PCG: start (cold: x = 0, r = b; warm: r = b - K x
-// formed by the caller), then per iteration launch_sell3 mode 4 (w = K u)
-// followed by launch_cg1_update.
+// formed by the caller), then per iteration the product w = K u with its dot
+// products and one vector kernel (launch_cg1_iteration).
 template <typename T>
 void launch_cg1_init(hipStream_t st, int64_t n, const T* b, bool cold, const T* dinv, T* x, T* r, T* u, T* p, T* s,
                      double* partials, Scalars* sc);
+// The loop scalars are read in slot *cur and left in the other one, which
+// becomes *cur.
 template <typename T>
-void launch_cg1_update(hipStream_t st, int64_t n, const T* dinv, T* x, T* r, T* u, const T* w, T* p, T* s,
-                       const Scalars* sc);
+void launch_cg1_iteration(hipStream_t st, int64_t n, const Sell3& A, const T* K, const T* dinv, T* x, T* r, T* u, T* w,
+                          T* p, T* s, double* partials, double* fold, Scalars* const sc[2], int* cur);
 
 // Mixed-precision solve of K x = rhs under device-side control, for launch
 // sequences captured once and replayed: single-reduction Jacobi PCG in FP32
@@ -205,31 +232,35 @@ struct MixedSolve {
     const double* rhs = nullptr;
     double *x64 = nullptr, *r64 = nullptr;
     float *r32 = nullptr, *u32 = nullptr, *w32 = nullptr, *p32 = nullptr, *s32 = nullptr;
-    double* partials = nullptr;
-    Scalars* sc = nullptr;
+    double *partials = nullptr, *fold = nullptr;
+    Scalars* sc[2] = {nullptr, nullptr};  // the loop scalars move between the two slots
     int64_t n = 0;
     double ru_factor = 0.01;
 };
 constexpr int kMixedMaxRefresh = 200;
-// start from the x64 passed in: |rhs|^2, first FP64 residual, FP32 start
+// start from the x64 passed in: |rhs|^2, first FP64 residual, FP32 start; the
+// scalars end in slot 0
 void launch_mixed_start(hipStream_t st, const MixedSolve& m);
-// one FP32 iteration (a no-op once done or while a refresh is pending)
-void launch_mixed_iteration(hipStream_t st, const MixedSolve& m);
-// refresh slot (a no-op unless a refresh is pending)
-void launch_mixed_refresh(hipStream_t st, const MixedSolve& m);
+// one FP32 iteration (a no-op once done or while a refresh is pending), the
+// scalars from slot *cur to the other
+void launch_mixed_iteration(hipStream_t st, const MixedSolve& m, int* cur);
+// refresh slot (a no-op unless a refresh is pending), likewise
+void launch_mixed_refresh(hipStream_t st, const MixedSolve& m, int* cur);
 
 void launch_scale_to_f32(hipStream_t st, int64_t n, const double* r, float* r32, const Scalars* sc);
 void launch_axpy_from_f32(hipStream_t st, int64_t n, double* u, const float* d, const Scalars* sc_outer);
 // PCG whose preconditioner runs as separate launches (z = M^-1 r in between):
-// start x = 0, r = b; dots: r.z and r.r into the loop scalars (init: also
-// p = z, start values; else beta, iteration count and the stop test);
-// update x += alpha p, r -= alpha q; dir p = z + beta p.
+// start x = 0, r = b; init (z of the start): r.z and r.r into sc, p = z; then
+// per iteration step: q = K p, x += alpha p, r -= alpha q (scalars sc[0] ->
+// sc[1]); z = M^-1 r; dir: r.z, r.r, the stop test, p = z + beta p (sc[1] ->
+// sc[0]).
 void launch_pcgz_start(hipStream_t st, int64_t n, const double* b, double* x, double* r);
-void launch_pcgz_dots(hipStream_t st, int64_t n, const double* r, const double* z, double* p, bool init,
-                      double* partials, Scalars* sc);
-void launch_pcgz_update(hipStream_t st, int64_t n, double* x, double* r, const double* p, const double* q,
-                        const Scalars* sc);
-void launch_pcgz_dir(hipStream_t st, int64_t n, const double* z, double* p, const Scalars* sc);
+void launch_pcgz_init(hipStream_t st, int64_t n, const double* r, const double* z, double* p, double* partials,
+                      Scalars* sc);
+void launch_pcgz_step(hipStream_t st, int64_t n, const Sell3& A, const double* K, double* x, double* r,
+                      const double* p, double* q, double* partials, double* fold, Scalars* const sc[2]);
+void launch_pcgz_dir(hipStream_t st, int64_t n, const double* r, const double* z, double* p, double* partials2,
+                     Scalars* const sc[2]);
 
 void launch_dot64(hipStream_t st, int64_t n, const double* a, const double* b, double* partials, Scalars* sc);
 void launch_axpy64(hipStream_t st, int64_t n, double alpha, const double* x, double* y);

@@ -134,3 +134,21 @@ def test_fp32_product(ctx, dims):
     d = ctx.mg_apply(0, x) - y
     assert np.linalg.norm(d[free]) <= 1e-6 * np.linalg.norm(y[free])
     assert np.abs(d[~free] / y[~free]).max() <= 1e-6
+
+
+# step kernels that add the product's partial sums themselves: more product
+# workgroups than they take (assembled values, 8,375 slices by four: folded first)
+# and several slices to a workgroup (reference blocks)
+@pytest.mark.parametrize("distorted", [True, False])
+def test_many_partial_sums(ctx, distorted):
+    gpu_case(f"PCG on 536,000 nodes distorted={distorted}")
+    p = problems.cantilever(66, 89, 88, 66.0, 89.0, 88.0, E=7.0e4, nu=0.3, traction=(0.0, 0.0, -1.0))
+    if distorted:
+        p = problems.distorted(p, 3)
+    problems.upload(ctx, p)
+    ctx.assemble()
+    assert ctx.uniform_elements() != distorted
+    u, st = ctx.solve(p.f, ctx.opts(api.SOLVE_PCG_FP64, api.PC_JACOBI, tol=1e-6, max_it=5000, check_every=33))
+    assert st.converged and st.iterations < 1500
+    res = np.linalg.norm(p.f - ctx.spmv(u)) / np.linalg.norm(p.f)
+    assert res <= 1.01e-6, res
