@@ -804,8 +804,18 @@ __device__ __forceinline__ T sell_load(const T* p) {
     else return *p;
 }
 
-// Row epilogue of the operator products (modes at the block-row SpMV below):
-// a = row r of K x, xr and fr the row's own values of x and f (where the mode
+// Modes of the operator products:
+//   0: y = K x
+//   1: y = K x, partial x.y (the PCG step)
+//   2: y = f - K x, partial |y|^2;   3: without it
+//   4: y = K x with x = u = Dinv r, f = r, partials r.u, y.u, r.r (the
+//      single-reduction PCG step)
+//   5: 2 where sc->gate is set (mixed solve's reliable update)
+//   6: 4 paused while sc->gate is set (the mixed solve's FP32 step)
+//   7: y = K x with x = p, f = r, partials p.y, p.r (the flexible PCG step)
+//   8: a Chebyshev step on f - K x (ChebStep)
+// Launches with loop scalars return at once when they are done.
+// Row epilogue: a = row r of K x, xr and fr the row's own values of x and f (where the mode
 // reads them); writes y and adds to the row's partial sums.
 template <int MODE>
 constexpr bool mode_reads_f() {
@@ -814,8 +824,24 @@ constexpr bool mode_reads_f() {
 
 template <typename T, int MODE>
 __device__ __forceinline__ void row_epilogue(int r, const T (&a)[3], const T (&xr)[3], const T (&fr)[3],
-                                             T* __restrict__ y, double (&part)[3]) {
+                                             T* __restrict__ y, const ChebStep& C, double (&part)[3]) {
     const int64_t d = 3 * (int64_t)r;
+    if (MODE == 8) {
+        float m[9];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) m[k] = C.binv[(int64_t)k * C.n + r];
+        const float c1 = C.coef[0], c2 = C.coef[1];
+        const float r0 = fr[0] - a[0], r1 = fr[1] - a[1], r2 = fr[2] - a[2];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const float v = c1 * C.d[d + i] + c2 * (m[3 * i] * r0 + m[3 * i + 1] * r1 + m[3 * i + 2] * r2);
+            const float o = xr[i] + v;
+            C.d[d + i] = v;
+            C.out[d + i] = o;
+            if (C.q) part[0] += (double)o * C.q[d + i];
+        }
+        return;
+    }
     if (MODE == 2 || MODE == 3 || MODE == 5) {
         const T y0 = fr[0] - a[0], y1 = fr[1] - a[1], y2 = fr[2] - a[2];
         y[d] = y0;
@@ -855,8 +881,8 @@ __device__ __forceinline__ void row_values(const T* __restrict__ v, int r, T (&o
 
 // the block's partial sums of a mode, stored for its finalize kernel
 template <int MODE>
-__device__ __forceinline__ void mode_partials(const double (&part)[3], double* partials) {
-    if (MODE == 0 || MODE == 3) return;
+__device__ __forceinline__ void mode_partials(const double (&part)[3], double* partials, const ChebStep& C) {
+    if (MODE == 0 || MODE == 3 || (MODE == 8 && !C.q)) return;
     if (MODE == 4 || MODE == 6) {
         double t[3] = {part[0], part[1], part[2]};
         block_partials<3>(t, partials);
@@ -872,7 +898,8 @@ __device__ __forceinline__ void mode_partials(const double (&part)[3], double* p
 // whether a mode's launch has nothing to do (converged, or paused)
 template <int MODE>
 __device__ __forceinline__ bool mode_idle(const Scalars* sc) {
-    if (MODE == 1 || MODE == 4 || MODE == 7) return sc->done;
+    if (MODE == 1 || MODE == 4) return sc->done;
+    if (MODE == 7) return sc && sc->done;
     if (MODE == 6) return sc->done || sc->gate;
     if (MODE == 5) return !sc->gate;
     return false;
@@ -883,7 +910,8 @@ __global__ __launch_bounds__(kSellMaxWaves * kWave) void k_sell3(int n_rows, int
                                                                  const int32_t* __restrict__ sptr,
                                                   const int32_t* __restrict__ scol, const T* __restrict__ val,
                                                   const T* __restrict__ x, T* __restrict__ y,
-                                                  const T* __restrict__ f, double* partials, const Scalars* sc) {
+                                                  const T* __restrict__ f, double* partials, const Scalars* sc,
+                                                  ChebStep cheb) {
     if (mode_idle<MODE>(sc)) return;
     const int lb = xcd_block(blockIdx.x, gridDim.x);
     const int slice = lb * (int)(blockDim.x / kWave) + threadIdx.x / kWave;
@@ -914,12 +942,12 @@ __global__ __launch_bounds__(kSellMaxWaves * kWave) void k_sell3(int n_rows, int
         if (r < n_rows) {
             const T a[3] = {a0, a1, a2};
             T xr[3] = {0, 0, 0}, fr[3] = {0, 0, 0};
-            if (MODE == 1 || MODE == 4 || MODE == 6 || MODE == 7) row_values(x, r, xr);
+            if (MODE == 1 || MODE == 4 || MODE >= 6) row_values(x, r, xr);
             if (mode_reads_f<MODE>()) row_values(f, r, fr);
-            row_epilogue<T, MODE>(r, a, xr, fr, y, part);
+            row_epilogue<T, MODE>(r, a, xr, fr, y, cheb, part);
         }
     }
-    mode_partials<MODE>(part, partials);
+    mode_partials<MODE>(part, partials, cheb);
 }
 
 // ---------------------------------------------------------------------------
@@ -1035,7 +1063,7 @@ __global__ __launch_bounds__(kUniWaves * kWave) void k_uni3(int n_rows, int n_sl
                                                             const int32_t* __restrict__ pslot,
                                                             const T* __restrict__ pen, const T* __restrict__ x,
                                                             T* __restrict__ y, const T* __restrict__ f,
-                                                            double* partials, const Scalars* sc) {
+                                                            double* partials, const Scalars* sc, ChebStep cheb) {
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     __shared__ T sh[3][kUniWaves - 1][kWave];
     double part[3] = {0.0, 0.0, 0.0};
@@ -1071,10 +1099,10 @@ __global__ __launch_bounds__(kUniWaves * kWave) void k_uni3(int n_rows, int n_sl
 #pragma unroll
                 for (int i = 0; i < 3; ++i) a[i] += pp[i] * xr[i];
             }
-            row_epilogue<T, MODE>(r, a, xr, fr, y, part);
+            row_epilogue<T, MODE>(r, a, xr, fr, y, cheb, part);
         }
     }
-    mode_partials<MODE>(part, partials);
+    mode_partials<MODE>(part, partials, cheb);
 }
 
 __global__ void k_uni_weights(int n, const int32_t* __restrict__ el, const double* __restrict__ E, double scale,
@@ -1142,7 +1170,7 @@ void launch_uni_penalty(hipStream_t st, const int64_t* pen, const int32_t* mult,
 
 template <typename T, int MODE>
 static int uni3_go(hipStream_t st, const Sell3& A, const UniOp& U, const T* x, T* y, const T* f, double* partials,
-                   Scalars* sc) {
+                   Scalars* sc, const ChebStep& C = ChebStep()) {
     const T *w, *kh, *pen;
     if constexpr (sizeof(T) == 8) {
         w = U.w64;
@@ -1156,7 +1184,7 @@ static int uni3_go(hipStream_t st, const Sell3& A, const UniOp& U, const T* x, T
     // at most kStepParts workgroups: the step kernels add that many partials
     const int per = (A.n_slices + kStepParts - 1) / kStepParts, nblk = (A.n_slices + per - 1) / per;
     hipLaunchKernelGGL((k_uni3<T, MODE>), dim3(nblk), dim3(kUniWaves * kWave), 0, st, A.n_rows, A.n_slices, per, U.nbr,
-                       w, kh, U.pslot, pen, x, y, f, partials, sc);
+                       w, kh, U.pslot, pen, x, y, f, partials, sc, C);
     return nblk;
 }
 
@@ -1175,18 +1203,18 @@ static const UniOp* uni_of(const Sell3& A, const T* val) {
 
 template <typename T, int MODE>
 static int sell3_go(hipStream_t st, const Sell3& A, const T* val, const T* x, T* y, const T* f, double* partials,
-                    Scalars* sc) {
-    if (const UniOp* U = uni_of(A, val)) return uni3_go<T, MODE>(st, A, *U, x, y, f, partials, sc);
+                    Scalars* sc, const ChebStep& C = ChebStep()) {
+    if (const UniOp* U = uni_of(A, val)) return uni3_go<T, MODE>(st, A, *U, x, y, f, partials, sc, C);
     const int per = A.waves_per_block;
     const int nblk = (A.n_slices + per - 1) / per;
     const int nthr = per * kWave;
     const bool nt = (int64_t)sizeof(T) * 9 * kWave * A.n_slots > kSellStreamBytes;
     if (nt)
         hipLaunchKernelGGL((k_sell3<T, MODE, true>), dim3(nblk), dim3(nthr), 0, st, A.n_rows, A.n_slices, A.sptr,
-                           A.scol, val, x, y, f, partials, sc);
+                           A.scol, val, x, y, f, partials, sc, C);
     else
         hipLaunchKernelGGL((k_sell3<T, MODE, false>), dim3(nblk), dim3(nthr), 0, st, A.n_rows, A.n_slices, A.sptr,
-                           A.scol, val, x, y, f, partials, sc);
+                           A.scol, val, x, y, f, partials, sc, C);
     return nblk;
 }
 
@@ -1209,6 +1237,17 @@ void launch_sell3(hipStream_t st, int mode, const Sell3& A, const T* val, const 
     }
 }
 
+// partials as the step kernels take them
+static StepParts folded(hipStream_t st, StepParts P, int nv, double* fold) {
+    if (P.n <= kStepParts) return P;
+    if (nv == 1) hipLaunchKernelGGL(k_fold<1>, dim3(kFoldBlocks), dim3(kBlock), 0, st, P.p, P.n, fold);
+    else if (nv == 2) hipLaunchKernelGGL(k_fold<2>, dim3(kFoldBlocks), dim3(kBlock), 0, st, P.p, P.n, fold);
+    else hipLaunchKernelGGL(k_fold<3>, dim3(kFoldBlocks), dim3(kBlock), 0, st, P.p, P.n, fold);
+    P.p = fold;
+    P.n = kFoldBlocks;
+    return P;
+}
+
 template <typename T>
 StepParts launch_sell3_step(hipStream_t st, int mode, const Sell3& A, const T* val, const T* x, T* y, const T* f,
                             double* partials, double* fold, const Scalars* sc_in) {
@@ -1227,18 +1266,16 @@ StepParts launch_sell3_step(hipStream_t st, int mode, const Sell3& A, const T* v
         case 5:
             P.n = sell3_go<T, 5>(st, A, val, x, y, f, partials, sc);
             break;
+        case 7:
+            P.n = sell3_go<T, 7>(st, A, val, x, y, f, partials, sc);
+            nv = 2;
+            break;
         default:
             P.n = sell3_go<T, 6>(st, A, val, x, y, f, partials, sc);
             nv = 3;
             break;
     }
-    if (P.n > kStepParts) {
-        if (nv == 1) hipLaunchKernelGGL(k_fold<1>, dim3(kFoldBlocks), dim3(kBlock), 0, st, partials, P.n, fold);
-        else hipLaunchKernelGGL(k_fold<3>, dim3(kFoldBlocks), dim3(kBlock), 0, st, partials, P.n, fold);
-        P.p = fold;
-        P.n = kFoldBlocks;
-    }
-    return P;
+    return folded(st, P, nv, fold);
 }
 template StepParts launch_sell3_step<double>(hipStream_t, int, const Sell3&, const double*, const double*, double*,
                                              const double*, double*, double*, const Scalars*);
@@ -1288,46 +1325,45 @@ __global__ __launch_bounds__(kSellMaxWaves * kWave) void k_sell3h(int n_rows, in
                                                                   const __half* __restrict__ val,
                                                                   const float* __restrict__ dinv,
                                                                   const float* __restrict__ x, float* __restrict__ y,
-                                                                  const float* __restrict__ f) {
+                                                                  const float* __restrict__ f, double* partials,
+                                                                  ChebStep cheb) {
     const int lb = xcd_block(blockIdx.x, gridDim.x);
     const int slice = lb * (int)(blockDim.x / kWave) + threadIdx.x / kWave;
     const int lane = threadIdx.x % kWave;
     const int r = slice * kWave + lane;
-    if (slice >= n_slices) return;
-    const int k0 = sptr[slice], k1 = sptr[slice + 1];
-    const int32_t* cp = scol + (int64_t)k0 * kWave + lane;
-    const __half* vp = val + (int64_t)k0 * 9 * kWave + lane;
-    float a0 = 0.f, a1 = 0.f, a2 = 0.f;
+    double part[3] = {0.0, 0.0, 0.0};
+    if (slice < n_slices) {
+        const int k0 = sptr[slice], k1 = sptr[slice + 1];
+        const int32_t* cp = scol + (int64_t)k0 * kWave + lane;
+        const __half* vp = val + (int64_t)k0 * 9 * kWave + lane;
+        float a0 = 0.f, a1 = 0.f, a2 = 0.f;
 #pragma unroll 2
-    for (int k = k0; k < k1; ++k) {
-        const int c = sell_load<NT>(cp);
-        const float x0 = x[3 * (int64_t)c], x1 = x[3 * (int64_t)c + 1], x2 = x[3 * (int64_t)c + 2];
-        float v[9];
+        for (int k = k0; k < k1; ++k) {
+            const int c = sell_load<NT>(cp);
+            const float x0 = x[3 * (int64_t)c], x1 = x[3 * (int64_t)c + 1], x2 = x[3 * (int64_t)c + 2];
+            float v[9];
 #pragma unroll
-        for (int q = 0; q < 9; ++q) {
-            const unsigned short h = sell_load<NT>((const unsigned short*)(vp + q * kWave));
-            v[q] = __half2float(__ushort_as_half(h));
+            for (int q = 0; q < 9; ++q) {
+                const unsigned short h = sell_load<NT>((const unsigned short*)(vp + q * kWave));
+                v[q] = __half2float(__ushort_as_half(h));
+            }
+            a0 += v[0] * x0 + v[1] * x1 + v[2] * x2;
+            a1 += v[3] * x0 + v[4] * x1 + v[5] * x2;
+            a2 += v[6] * x0 + v[7] * x1 + v[8] * x2;
+            cp += kWave;
+            vp += 9 * kWave;
         }
-        a0 += v[0] * x0 + v[1] * x1 + v[2] * x2;
-        a1 += v[3] * x0 + v[4] * x1 + v[5] * x2;
-        a2 += v[6] * x0 + v[7] * x1 + v[8] * x2;
-        cp += kWave;
-        vp += 9 * kWave;
+        if (r < n_rows) {
+            const int64_t d = 3 * (int64_t)r;
+            const float a[3] = {a0 / dinv[d], a1 / dinv[d + 1], a2 / dinv[d + 2]};
+            float xr[3] = {0.f, 0.f, 0.f}, fr[3] = {0.f, 0.f, 0.f};
+            if (MODE == 8) row_values(x, r, xr);
+            if (mode_reads_f<MODE>()) row_values(f, r, fr);
+            row_epilogue<float, MODE>(r, a, xr, fr, y, cheb, part);
+        }
     }
-    if (r >= n_rows) return;
-    const int64_t d = 3 * (int64_t)r;
-    a0 /= dinv[d];
-    a1 /= dinv[d + 1];
-    a2 /= dinv[d + 2];
-    if (MODE == 3) {
-        y[d] = f[d] - a0;
-        y[d + 1] = f[d + 1] - a1;
-        y[d + 2] = f[d + 2] - a2;
-    } else {
-        y[d] = a0;
-        y[d + 1] = a1;
-        y[d + 2] = a2;
-    }
+    // mode 3 leaves its norm aside
+    mode_partials<MODE>(part, partials, cheb);
 }
 
 // Timing of the FP16 cycle SpMV with the residual epilogue (mode 3, the
@@ -1373,140 +1409,64 @@ static hipEvent_t cycle_timer_event() {
     return t.ev[t.used++];
 }
 
-void launch_sell3_h(hipStream_t st, int mode, const Sell3& A, const __half* val, const float* dinv32, const float* x,
-                    float* y, const float* f) {
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    if (g_cycle_timer.on && mode == 3) {
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone) {
-            e0 = cycle_timer_event();
-            e1 = cycle_timer_event();
-            if (e0 && e1) (void)hipEventRecord(e0, st);
-        }
-    }
-    if (A.n_uni > 0 && A.uni[0].val32) {
-        // the context's operator from its reference blocks: FP32, and still fewer bytes
-        if (mode == 3) uni3_go<float, 3>(st, A, A.uni[0], x, y, f, nullptr, nullptr);
-        else uni3_go<float, 0>(st, A, A.uni[0], x, y, f, nullptr, nullptr);
-        if (e0 && e1) (void)hipEventRecord(e1, st);
-        return;
-    }
+template <int MODE>
+static int sell3h_go(hipStream_t st, const Sell3& A, const __half* val, const float* dinv32, const float* x, float* y,
+                     const float* f, double* partials, const ChebStep& C) {
+    // the context's operator from its reference blocks: FP32, and still fewer bytes
+    if (A.n_uni > 0 && A.uni[0].val32)
+        return uni3_go<float, MODE>(st, A, A.uni[0], x, y, f, partials, (Scalars*)nullptr, C);
     const int per = A.waves_per_block;
     const int nblk = (A.n_slices + per - 1) / per;
     const int nthr = per * kWave;
     const bool nt = (int64_t)sizeof(__half) * 9 * kWave * A.n_slots > kSellStreamBytes;
-    auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(nblk), dim3(nthr), 0, st, A.n_rows, A.n_slices, A.sptr, A.scol, val, dinv32, x,
-                           y, f);
-    };
+    if (nt)
+        hipLaunchKernelGGL((k_sell3h<MODE, true>), dim3(nblk), dim3(nthr), 0, st, A.n_rows, A.n_slices, A.sptr, A.scol,
+                           val, dinv32, x, y, f, partials, C);
+    else
+        hipLaunchKernelGGL((k_sell3h<MODE, false>), dim3(nblk), dim3(nthr), 0, st, A.n_rows, A.n_slices, A.sptr,
+                           A.scol, val, dinv32, x, y, f, partials, C);
+    return nblk;
+}
+
+// brackets a launch with the cycle timer's events while it is on
+struct CycleTimed {
+    hipEvent_t e1 = nullptr;
+    hipStream_t st;
+    explicit CycleTimed(hipStream_t s) : st(s) {
+        if (!g_cycle_timer.on) return;
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) return;
+        hipEvent_t e0 = cycle_timer_event();
+        e1 = cycle_timer_event();
+        if (e0 && e1) (void)hipEventRecord(e0, st);
+        else e1 = nullptr;
+    }
+    ~CycleTimed() {
+        if (e1) (void)hipEventRecord(e1, st);
+    }
+};
+
+void launch_sell3_h(hipStream_t st, int mode, const Sell3& A, const __half* val, const float* dinv32, const float* x,
+                    float* y, const float* f) {
     if (mode == 3) {
-        if (nt) go(k_sell3h<3, true>);
-        else go(k_sell3h<3, false>);
+        const CycleTimed timed(st);
+        sell3h_go<3>(st, A, val, dinv32, x, y, f, nullptr, ChebStep());
     } else {
-        if (nt) go(k_sell3h<0, true>);
-        else go(k_sell3h<0, false>);
-    }
-    if (e0 && e1) (void)hipEventRecord(e1, st);
-}
-
-// ---------------------------------------------------------------------------
-// Block-row SpMV, b = 3, G lanes per block row, component-major values.
-// MODE 0: y = K x
-// MODE 1: y = K x and (x . y): with launch_sell3_step the PCG step length
-// MODE 2: y = f - K x (x = current solution, f = load) -> finalize: sc->rr = |y|^2
-// MODE 3: y = f - K x without the norm
-// MODE 4 (sliced-ELL only): y = K x with x = u = Dinv r and f = r, partials of
-//   r.u, y.u and r.r (the single-reduction PCG step)
-// MODE 5 (sliced-ELL only): MODE 2 when sc->gate is set (mixed solve's
-//   reliable update: convergence on the FP64 residual)
-// MODE 6 (sliced-ELL only): MODE 4 paused while sc->gate is set (the mixed
-//   solve's FP32 step, or a refresh request)
-//   Modes 1, 4, 5 and 6 leave their partials to the step's vector kernel
-//   (launch_sell3_step).
-// MODE 7 (sliced-ELL only): y = K x with x = p and f = r, partials of p.y and
-//   p.r -> finalize: the flexible PCG step length alpha = p.r / p.q
-// Kernels with a scalars pointer return at once when sc->done is set.
-// ---------------------------------------------------------------------------
-template <typename T, int G, int MODE>
-__global__ __launch_bounds__(kBlock) void k_spmv3(int n_rows, int rows_per_block, const int32_t* __restrict__ rp,
-                                                  const int32_t* __restrict__ bc, const T* __restrict__ val,
-                                                  const T* __restrict__ x, T* __restrict__ y,
-                                                  const T* __restrict__ f, double* partials, const Scalars* sc) {
-    if (MODE == 1 && sc->done) return;
-    const int lb = xcd_block(blockIdx.x, gridDim.x);
-    const int sub = threadIdx.x % G;
-    const int grp = threadIdx.x / G;
-    constexpr int kGroups = kBlock / G;
-    const int r0 = lb * rows_per_block;
-    int r1 = r0 + rows_per_block;
-    if (r1 > n_rows) r1 = n_rows;
-    double part = 0.0;
-    for (int r = r0 + grp; r < r1; r += kGroups) {
-        const int s = rp[r], nb = rp[r + 1] - s;
-        const T* v = val + 9 * (int64_t)s;
-        T a0 = 0, a1 = 0, a2 = 0;
-        for (int k = sub; k < nb; k += G) {
-            const int c = bc[s + k];
-            const T x0 = x[3 * (int64_t)c], x1 = x[3 * (int64_t)c + 1], x2 = x[3 * (int64_t)c + 2];
-            a0 += v[0 * nb + k] * x0 + v[1 * nb + k] * x1 + v[2 * nb + k] * x2;
-            a1 += v[3 * nb + k] * x0 + v[4 * nb + k] * x1 + v[5 * nb + k] * x2;
-            a2 += v[6 * nb + k] * x0 + v[7 * nb + k] * x1 + v[8 * nb + k] * x2;
-        }
-#pragma unroll
-        for (int o = G / 2; o > 0; o >>= 1) {
-            a0 += __shfl_xor(a0, o, G);
-            a1 += __shfl_xor(a1, o, G);
-            a2 += __shfl_xor(a2, o, G);
-        }
-        if (sub == 0) {
-            if (MODE == 2 || MODE == 3) {
-                T y0 = f[3 * (int64_t)r] - a0, y1 = f[3 * (int64_t)r + 1] - a1, y2 = f[3 * (int64_t)r + 2] - a2;
-                y[3 * (int64_t)r] = y0;
-                y[3 * (int64_t)r + 1] = y1;
-                y[3 * (int64_t)r + 2] = y2;
-                part += (double)y0 * y0 + (double)y1 * y1 + (double)y2 * y2;
-            } else {
-                y[3 * (int64_t)r] = a0;
-                y[3 * (int64_t)r + 1] = a1;
-                y[3 * (int64_t)r + 2] = a2;
-                if (MODE == 1)
-                    part += (double)a0 * x[3 * (int64_t)r] + (double)a1 * x[3 * (int64_t)r + 1] +
-                            (double)a2 * x[3 * (int64_t)r + 2];
-            }
-        }
-    }
-    if (MODE == 0 || MODE == 3) return;
-    double t[1] = {part};
-    block_partials<1>(t, partials);
-}
-
-template <typename T>
-void launch_spmv3(hipStream_t st, int mode, int n_rows, const int32_t* rp, const int32_t* bc, const T* val,
-                  const T* x, T* y, const T* f, double* partials, Scalars* sc) {
-    constexpr int G = 32;
-    const int nblk = kSpmvBlocks;
-    int rpb = (n_rows + nblk - 1) / nblk;
-    if (mode == 0) {
-        hipLaunchKernelGGL((k_spmv3<T, G, 0>), dim3(nblk), dim3(kBlock), 0, st, n_rows, rpb, rp, bc, val, x, y, f,
-                           partials, sc);
-    } else if (mode == 1) {
-        hipLaunchKernelGGL((k_spmv3<T, G, 1>), dim3(nblk), dim3(kBlock), 0, st, n_rows, rpb, rp, bc, val, x, y, f,
-                           partials, sc);
-        finalize(st, partials, nblk, FIN_PQ, sc);
-    } else if (mode == 2) {
-        hipLaunchKernelGGL((k_spmv3<T, G, 2>), dim3(nblk), dim3(kBlock), 0, st, n_rows, rpb, rp, bc, val, x, y, f,
-                           partials, sc);
-        finalize(st, partials, nblk, FIN_RR, sc);
-    } else {
-        hipLaunchKernelGGL((k_spmv3<T, G, 3>), dim3(nblk), dim3(kBlock), 0, st, n_rows, rpb, rp, bc, val, x, y, f,
-                           partials, sc);
+        sell3h_go<0>(st, A, val, dinv32, x, y, f, nullptr, ChebStep());
     }
 }
 
-template void launch_spmv3<double>(hipStream_t, int, int, const int32_t*, const int32_t*, const double*,
-                                   const double*, double*, const double*, double*, Scalars*);
-template void launch_spmv3<float>(hipStream_t, int, int, const int32_t*, const int32_t*, const float*, const float*,
-                                  float*, const float*, double*, Scalars*);
+StepParts launch_cheb_step(hipStream_t st, const Sell3& A, const float* val, const __half* val16, const float* dinv32,
+                           const float* x, const float* b, const ChebStep& C, double* partials, double* fold) {
+    StepParts P;
+    P.p = partials;
+    {
+        const CycleTimed timed(st);
+        P.n = val16 ? sell3h_go<8>(st, A, val16, dinv32, x, nullptr, b, partials, C)
+                    : sell3_go<float, 8>(st, A, val, x, nullptr, b, partials, nullptr, C);
+    }
+    return C.q ? folded(st, P, 1, fold) : StepParts();
+}
 
 // ---------------------------------------------------------------------------
 // Jacobi PCG vector kernels (T = double for the FP64 solver, float for the

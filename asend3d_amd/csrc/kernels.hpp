@@ -35,6 +35,18 @@ struct UniOp {
     const float* pen32 = nullptr;
 };
 
+// One block-Jacobi Chebyshev step inside the product of its residual (mode 8):
+// with res = f - K x, z = Binv res, d = c1 d + c2 z, out = x + d; where q is
+// given also the partials of out.q.
+struct ChebStep {
+    const float* binv = nullptr;  // 3x3 block inverses, component-major (9 x n)
+    const float* coef = nullptr;  // c1, c2
+    float* d = nullptr;
+    float* out = nullptr;  // not x: other rows still read it
+    const float* q = nullptr;
+    int n = 0;
+};
+
 // Sliced-ELL fine operator: 64-row slices of 3x3 blocks (see kernels.hip).
 struct Sell3 {
     int n_rows = 0, n_slices = 0;
@@ -134,7 +146,9 @@ void launch_uni_coef(hipStream_t st, const double* Khat, const double* Mhat, dou
 void launch_uni_penalty(hipStream_t st, const int64_t* pen, const int32_t* mult, int n_pen, double sf,
                         const int32_t* pslot, int n_pslots, double* pen64, float* pen32);
 
-// Sliced-ELL SpMV: modes 0, 2 and 3 as launch_spmv3, and 7 (flexible PCG).
+// Sliced-ELL SpMV, mode 0: y = K x; 2: y = f - K x, sc->rr = |y|^2; 3: y = f - K x;
+// 7: y = K x and the flexible PCG step length (modes 2 and 7 launch a one-block
+// finalize kernel).
 template <typename T>
 void launch_sell3(hipStream_t st, int mode, const Sell3& A, const T* val, const T* x, T* y, const T* f,
                   double* partials, Scalars* sc);
@@ -171,17 +185,18 @@ inline int step_blocks(int64_t n) {
     const int64_t b = (n + 255) / 256;
     return (int)(b < 1 ? 1 : (b < kStepBlocks ? b : kStepBlocks));
 }
-// Modes 1, 4, 5 and 6 of the operator product (the scalars at sc decide whether
-// they have work) with their partials left in place (or in fold).
+// Modes 1, 4, 5, 6 and 7 of the operator product (the scalars at sc decide
+// whether they have work; null with mode 7: always) with their partials left in
+// place (or in fold).
 template <typename T>
 StepParts launch_sell3_step(hipStream_t st, int mode, const Sell3& A, const T* val, const T* x, T* y, const T* f,
                             double* partials, double* fold, const Scalars* sc);
 
-// mode 0: y = K x; 1 (block rows only): y = K x, sc->pq = x.y, sc->alpha = sc->rz/pq; 2: y = f - K x, sc->rr = |y|^2
-// 3: y = f - K x (no norm).  Modes 1 and 2 launch their single-block finalize kernel after the SpMV.
-template <typename T>
-void launch_spmv3(hipStream_t st, int mode, int n_rows, const int32_t* rp, const int32_t* bc, const T* val,
-                  const T* x, T* y, const T* f, double* partials, Scalars* sc);
+// One Chebyshev step of the multigrid cycle on the finest level (ChebStep; its
+// product as launch_sell3_h where val16 is given, else of val); the out.q
+// partials where C.q is given.
+StepParts launch_cheb_step(hipStream_t st, const Sell3& A, const float* val, const __half* val16, const float* dinv32,
+                           const float* x, const float* b, const ChebStep& C, double* partials, double* fold);
 
 template <typename T>
 void launch_pcg_init(hipStream_t st, int64_t n, const T* b, const T* dinv, T* x, T* r, T* p, double* partials,

@@ -135,6 +135,7 @@ struct Level {
     float* d_pval = nullptr;
     // work vectors
     float *x = nullptr, *b = nullptr, *r = nullptr, *d = nullptr;
+    float* x2 = nullptr;  // the cycle's other iterate (a fused step reads x and writes the next)
     double lmax = 0.0;
 };
 
@@ -160,7 +161,8 @@ struct Multigrid {
     double* d_Ainv = nullptr;
     // FCG work vectors (fine level)
     float *r = nullptr, *z = nullptr, *p = nullptr, *q = nullptr;
-    double* partials = nullptr;
+    // block partials: pairs of the finest products (or z.q), the update's r.r, folded sums
+    double *partials = nullptr, *partials_rr = nullptr, *fold = nullptr;
     // the learned smoother's bound estimated on its own stream while the
     // hierarchy is set up on another (mg_learned_bound_begin/end): its own
     // reduction scratch and result
@@ -191,7 +193,8 @@ struct Multigrid {
     // (coefficients formed on the device, value in d_lam[0])
     bool fine_pending = false;
     hipStream_t lam_stream = nullptr;
-    double* sv = nullptr;      // device scalars of the FCG loop
+    // device scalars of the FCG loop: before the update, (SV_MID) before the direction
+    double* sv = nullptr;
     double* h_sv = nullptr;    // pinned mirror
     // Chebyshev smoother: point (0) or block (1) Jacobi, degree and interval
     // [lo, hi] * lambda_max
@@ -295,79 +298,181 @@ void fr(T*& p) {
 // ---------------------------------------------------------------------------
 __constant__ int kCorner[8][3] = {{0, 0, 0}, {1, 0, 0}, {1, 1, 0}, {0, 1, 0}, {0, 0, 1}, {1, 0, 1}, {1, 1, 1}, {0, 1, 1}};
 
-// Restriction: coarse node (I,J,K) <- sum of up to 27 fine nodes.
-__global__ void k_restrict3(int ncx, int ncy, int ncz, int nfx, int nfy, const int* __restrict__ rix,
-                            const float* __restrict__ rwx, const int* __restrict__ riy, const float* __restrict__ rwy,
-                            const int* __restrict__ riz, const float* __restrict__ rwz,
-                            const int32_t* __restrict__ frank, const float* __restrict__ rf, float* __restrict__ bc) {
-    int64_t N = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t total = (int64_t)(ncx + 1) * (ncy + 1) * (ncz + 1);
-    if (N >= total) return;
-    int I = (int)(N % (ncx + 1));
-    int J = (int)((N / (ncx + 1)) % (ncy + 1));
-    int K = (int)(N / ((int64_t)(ncx + 1) * (ncy + 1)));
-    float s0 = 0.f, s1 = 0.f, s2 = 0.f;
-    for (int c = 0; c < 3; ++c) {
-        int k = riz[3 * K + c];
-        if (k < 0) continue;
-        float wz = rwz[3 * K + c];
-        for (int b = 0; b < 3; ++b) {
-            int j = riy[3 * J + b];
-            if (j < 0) continue;
-            float wyz = wz * rwy[3 * J + b];
-            for (int a = 0; a < 3; ++a) {
-                int i = rix[3 * I + a];
-                if (i < 0) continue;
-                float w = wyz * rwx[3 * I + a];
-                int64_t g = i + (int64_t)(nfx + 1) * (j + (int64_t)(nfy + 1) * k);
-                int64_t row = frank ? frank[g] : g;
-                s0 += w * rf[3 * row];
-                s1 += w * rf[3 * row + 1];
-                s2 += w * rf[3 * row + 2];
-            }
-        }
+// The transfers take one thread per node and component, 64 nodes a block, with
+// absent taps read at weight zero so that every load of a stage is in flight
+// at once: a thread per node that branched on each tap was a chain of up to 27
+// dependent loads.  Mean over the five levels under 337,881 nodes: restriction
+// 10.6 us and its level's first smoothing step 3.5 us -> 6.8 us together, prolongation
+// 7.2 -> 5.6 us.
+constexpr int kTransferNodes = 64;
+constexpr int kTransferBlock = 3 * kTransferNodes;
+
+// Restriction: coarse node (I,J,K) <- sum of up to 27 fine nodes.  FIRST: with the
+// coarse level's first smoothing step from zero, d = x = c2 Binv b.
+template <bool FIRST>
+__global__ __launch_bounds__(kTransferBlock) void k_restrict3(
+    int ncx, int ncy, int ncz, int nfx, int nfy, const int* __restrict__ rix, const float* __restrict__ rwx,
+    const int* __restrict__ riy, const float* __restrict__ rwy, const int* __restrict__ riz,
+    const float* __restrict__ rwz, const int32_t* __restrict__ frank, const float* __restrict__ rf,
+    float* __restrict__ bc, const float* __restrict__ binv, const float* __restrict__ coef, float* __restrict__ d,
+    float* __restrict__ x) {
+    __shared__ float sb[kTransferBlock];
+    const int total = (ncx + 1) * (ncy + 1) * (ncz + 1);
+    const int nd = threadIdx.x / 3, comp = threadIdx.x - 3 * nd;
+    const int N = blockIdx.x * kTransferNodes + nd;
+    const bool live = N < total;
+    float m[3] = {0.f, 0.f, 0.f}, c2 = 0.f;
+    if (FIRST && live) {
+        c2 = coef[1];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) m[j] = binv[(int64_t)(3 * comp + j) * total + N];
     }
-    bc[3 * N] = s0;
-    bc[3 * N + 1] = s1;
-    bc[3 * N + 2] = s2;
+    if (live) {
+        const int I = N % (ncx + 1), J = (N / (ncx + 1)) % (ncy + 1), K = N / ((ncx + 1) * (ncy + 1));
+        int ix[3], iy[3], iz[3];
+        float wx[3], wy[3], wz[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            ix[a] = rix[3 * I + a];
+            iy[a] = riy[3 * J + a];
+            iz[a] = riz[3 * K + a];
+            wx[a] = rwx[3 * I + a];
+            wy[a] = rwy[3 * J + a];
+            wz[a] = rwz[3 * K + a];
+        }
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            if (ix[a] < 0) ix[a] = 0, wx[a] = 0.f;
+            if (iy[a] < 0) iy[a] = 0, wy[a] = 0.f;
+            if (iz[a] < 0) iz[a] = 0, wz[a] = 0.f;
+        }
+        float v[27];
+#pragma unroll
+        for (int t = 0; t < 27; ++t) {
+            const int64_t g = ix[t % 3] + (int64_t)(nfx + 1) * (iy[t / 3 % 3] + (int64_t)(nfy + 1) * iz[t / 9]);
+            v[t] = rf[3 * (int64_t)(frank ? frank[g] : g) + comp];
+        }
+        float s = 0.f;
+#pragma unroll
+        for (int t = 0; t < 27; ++t) {
+            const float w = wz[t / 9] * wy[t / 3 % 3] * wx[t % 3];
+            // not a tap: whatever stands there stays out, not only finite values
+            s += w != 0.f ? w * v[t] : 0.f;
+        }
+        bc[3 * (int64_t)N + comp] = s;
+        if (FIRST) sb[threadIdx.x] = s;
+    }
+    if (!FIRST) return;
+    __syncthreads();
+    if (live) {
+        const float v = c2 * (m[0] * sb[3 * nd] + m[1] * sb[3 * nd + 1] + m[2] * sb[3 * nd + 2]);
+        d[3 * (int64_t)N + comp] = v;
+        x[3 * (int64_t)N + comp] = v;
+    }
 }
 
 // Prolongation-add: fine node (i,j,k) += sum of up to 8 coarse parents.
-__global__ void k_prolong_add3(int nfx, int nfy, int nfz, int ncx, int ncy, const int* __restrict__ pix,
-                               const float* __restrict__ pwx, const int* __restrict__ piy,
-                               const float* __restrict__ pwy, const int* __restrict__ piz,
-                               const float* __restrict__ pwz, const int32_t* __restrict__ frank,
-                               const float* __restrict__ xc, float* __restrict__ xf) {
-    int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t total = (int64_t)(nfx + 1) * (nfy + 1) * (nfz + 1);
+__global__ __launch_bounds__(kTransferBlock) void k_prolong_add3(
+    int nfx, int nfy, int nfz, int ncx, int ncy, const int* __restrict__ pix, const float* __restrict__ pwx,
+    const int* __restrict__ piy, const float* __restrict__ pwy, const int* __restrict__ piz,
+    const float* __restrict__ pwz, const int32_t* __restrict__ frank, const float* __restrict__ xc,
+    float* __restrict__ xf) {
+    const int64_t total = (int64_t)(nfx + 1) * (nfy + 1) * (nfz + 1);
+    const int nd = threadIdx.x / 3, comp = threadIdx.x - 3 * nd;
+    const int64_t g = (int64_t)blockIdx.x * kTransferNodes + nd;
     if (g >= total) return;
-    int i = (int)(g % (nfx + 1));
-    int j = (int)((g / (nfx + 1)) % (nfy + 1));
-    int k = (int)(g / ((int64_t)(nfx + 1) * (nfy + 1)));
-    float s0 = 0.f, s1 = 0.f, s2 = 0.f;
-    for (int c = 0; c < 2; ++c) {
-        int K = piz[2 * k + c];
-        if (K < 0) continue;
-        float wz = pwz[2 * k + c];
-        for (int b = 0; b < 2; ++b) {
-            int J = piy[2 * j + b];
-            if (J < 0) continue;
-            float wyz = wz * pwy[2 * j + b];
-            for (int a = 0; a < 2; ++a) {
-                int I = pix[2 * i + a];
-                if (I < 0) continue;
-                float w = wyz * pwx[2 * i + a];
-                int64_t N = I + (int64_t)(ncx + 1) * (J + (int64_t)(ncy + 1) * K);
-                s0 += w * xc[3 * N];
-                s1 += w * xc[3 * N + 1];
-                s2 += w * xc[3 * N + 2];
-            }
-        }
+    const int64_t row = frank ? frank[g] : g;
+    const int i = (int)(g % (nfx + 1)), j = (int)((g / (nfx + 1)) % (nfy + 1));
+    const int k = (int)(g / ((int64_t)(nfx + 1) * (nfy + 1)));
+    int ix[2], iy[2], iz[2];
+    float wx[2], wy[2], wz[2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+        ix[a] = pix[2 * i + a];
+        iy[a] = piy[2 * j + a];
+        iz[a] = piz[2 * k + a];
+        wx[a] = pwx[2 * i + a];
+        wy[a] = pwy[2 * j + a];
+        wz[a] = pwz[2 * k + a];
     }
-    int64_t row = frank ? frank[g] : g;
-    xf[3 * row] += s0;
-    xf[3 * row + 1] += s1;
-    xf[3 * row + 2] += s2;
+    const float x0 = xf[3 * row + comp];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+        if (ix[a] < 0) ix[a] = 0, wx[a] = 0.f;
+        if (iy[a] < 0) iy[a] = 0, wy[a] = 0.f;
+        if (iz[a] < 0) iz[a] = 0, wz[a] = 0.f;
+    }
+    float v[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+        v[t] = xc[3 * (ix[t & 1] + (int64_t)(ncx + 1) * (iy[t >> 1 & 1] + (int64_t)(ncy + 1) * iz[t >> 2])) + comp];
+    float s = 0.f;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        const float w = wz[t >> 2] * wy[t >> 1 & 1] * wx[t & 1];
+        s += w != 0.f ? w * v[t] : 0.f;
+    }
+    xf[3 * row + comp] = x0 + s;
+}
+
+// Products with a coarse operator (block rows of up to 27 blocks, values
+// component-major per row): half a wavefront per row, its lanes the row's blocks,
+// so that all of a row's loads are one burst of 9 coalesced reads.
+//   0: y = K x;  3: y = b - K x;  8: a Chebyshev step on b - K x (ChebStep)
+// Mode 8 is the residual and the smoothing update of a step in one launch, both
+// little more than a launch each on the deeper levels: mean over the levels under
+// 337,881 nodes 5.8 + 3.4 us -> 5.7 us, under 45,120 nodes 3.8 + 3.3 -> 3.6 us.
+template <int MODE>
+__global__ __launch_bounds__(kBlock) void k_coarse3(int n_rows, const int32_t* __restrict__ rp,
+                                                    const int32_t* __restrict__ bc, const float* __restrict__ val,
+                                                    const float* __restrict__ x, float* __restrict__ y,
+                                                    const float* __restrict__ b, ChebStep C) {
+    constexpr int G = 32;
+    const int sub = threadIdx.x % G;
+    const int r = blockIdx.x * (kBlock / G) + threadIdx.x / G;
+    if (r >= n_rows) return;
+    const int s = rp[r], nb = rp[r + 1] - s;
+    const float* v = val + 9 * (int64_t)s;
+    // lanes 0 to 2 finish one component each; what they need travels beside the values
+    const int64_t d = 3 * (int64_t)r;
+    const int i = min(sub, 2);
+    float m[3] = {0.f, 0.f, 0.f}, f[3] = {0.f, 0.f, 0.f}, di = 0.f, xi = 0.f, c1 = 0.f, c2 = 0.f;
+    if (MODE == 3) f[0] = b[d + i];
+    if (MODE == 8) {
+        c1 = C.coef[0];
+        c2 = C.coef[1];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            m[j] = C.binv[(int64_t)(3 * i + j) * C.n + r];
+            f[j] = b[d + j];
+        }
+        di = C.d[d + i];
+        xi = x[d + i];
+    }
+    float a0 = 0.f, a1 = 0.f, a2 = 0.f;
+    for (int k = sub; k < nb; k += G) {
+        const int c = bc[s + k];
+        const float x0 = x[3 * (int64_t)c], x1 = x[3 * (int64_t)c + 1], x2 = x[3 * (int64_t)c + 2];
+        a0 += v[0 * nb + k] * x0 + v[1 * nb + k] * x1 + v[2 * nb + k] * x2;
+        a1 += v[3 * nb + k] * x0 + v[4 * nb + k] * x1 + v[5 * nb + k] * x2;
+        a2 += v[6 * nb + k] * x0 + v[7 * nb + k] * x1 + v[8 * nb + k] * x2;
+    }
+#pragma unroll
+    for (int o = G / 2; o > 0; o >>= 1) {
+        a0 += __shfl_xor(a0, o, G);
+        a1 += __shfl_xor(a1, o, G);
+        a2 += __shfl_xor(a2, o, G);
+    }
+    if (sub > 2) return;
+    const float ai = i == 0 ? a0 : (i == 1 ? a1 : a2);
+    if (MODE == 0) y[d + i] = ai;
+    if (MODE == 3) y[d + i] = f[0] - ai;
+    if (MODE == 8) {
+        const float z = m[0] * (f[0] - a0) + m[1] * (f[1] - a1) + m[2] * (f[2] - a2);
+        const float e = c1 * di + c2 * z;
+        C.d[d + i] = e;
+        C.out[d + i] = xi + e;
+    }
 }
 
 // Level-1 element matrices from the fine mesh.  One wave per coarse element,
@@ -583,34 +688,32 @@ __global__ void k_binv32(int n_rows, const int32_t* __restrict__ sptr, const int
     for (int k = 0; k < 9; ++k) binv[(int64_t)k * n_rows + r] = (float)inv[k];
 }
 
-// Block-Jacobi Chebyshev steps (z_r = Binv_r r_r per node), coefficients
-// (c1, c2) read from device memory so that captured graphs stay valid when
-// the bounds change:   first: d = c2 z, x = d;   step: d = c1 d + c2 z, x += d
-template <bool FIRST>
-__global__ void k_cheb_block(int n_nodes, const float* __restrict__ binv, const float* __restrict__ r,
-                             const float* __restrict__ coef, float* __restrict__ d, float* __restrict__ x) {
-    const float c1 = coef[0], c2 = coef[1];
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n_nodes; i += gridDim.x * blockDim.x) {
-        const float r0 = r[3 * i], r1 = r[3 * i + 1], r2 = r[3 * i + 2];
-        float m[9];
-        for (int k = 0; k < 9; ++k) m[k] = binv[(int64_t)k * n_nodes + i];
-        const float z[3] = {m[0] * r0 + m[1] * r1 + m[2] * r2, m[3] * r0 + m[4] * r1 + m[5] * r2,
-                            m[6] * r0 + m[7] * r1 + m[8] * r2};
-        for (int c = 0; c < 3; ++c) {
-            if (FIRST) {
-                const float v = c2 * z[c];
-                d[3 * i + c] = v;
-                x[3 * i + c] = v;
-            } else {
-                const float v = c1 * d[3 * i + c] + c2 * z[c];
-                d[3 * i + c] = v;
-                x[3 * i + c] += v;
-            }
-        }
+// First step of a block-Jacobi Chebyshev smoothing from zero (z_r = Binv_r r_r per
+// node): d = c2 z, x = d; the others are in their residual's product
+// (ChebStep).  The coefficients (c1, c2) are read from device memory so that
+// captured graphs stay valid when the bounds change.
+__device__ __forceinline__ void cheb_first(int i, int n_nodes, const float* __restrict__ binv, float r0, float r1,
+                                           float r2, float c2, float* __restrict__ d, float* __restrict__ x) {
+    float m[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) m[k] = binv[(int64_t)k * n_nodes + i];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const float v = c2 * (m[3 * c] * r0 + m[3 * c + 1] * r1 + m[3 * c + 2] * r2);
+        d[3 * (int64_t)i + c] = v;
+        x[3 * (int64_t)i + c] = v;
     }
 }
 
-// The same per DOF, z = dinv r (point Jacobi) or z = r (already preconditioned)
+__global__ void k_cheb_block(int n_nodes, const float* __restrict__ binv, const float* __restrict__ r,
+                             const float* __restrict__ coef, float* __restrict__ d, float* __restrict__ x) {
+    const float c2 = coef[1];
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n_nodes; i += gridDim.x * blockDim.x)
+        cheb_first(i, n_nodes, binv, r[3 * (int64_t)i], r[3 * (int64_t)i + 1], r[3 * (int64_t)i + 2], c2, d, x);
+}
+
+// Chebyshev steps per DOF, z = dinv r (point Jacobi) or z = r (already preconditioned):
+// first: d = c2 z, x = d;   step: d = c1 d + c2 z, x += d
 template <bool FIRST>
 __global__ void k_cheb_dof(int64_t n, const float* __restrict__ dinv, const float* __restrict__ r,
                            const float* __restrict__ coef, float* __restrict__ d, float* __restrict__ x) {
@@ -914,72 +1017,110 @@ __global__ __launch_bounds__(256) void k_dense_gemv(int n, const double* __restr
 // FCG helpers --------------------------------------------------------------
 // sv layout: 0 pq, 1 pr, 2 rr, 3 rr0, 4 alpha, 5 beta, 6 zq, 7 tol2, 8 it, 9 max_it, 10 done
 enum { SV_PQ = 0, SV_PR, SV_RR, SV_RR0, SV_ALPHA, SV_BETA, SV_ZQ, SV_TOL2, SV_IT, SV_MAXIT, SV_DONE, SV_N };
+constexpr int SV_MID = 16;  // the scalars between an iteration's two vector kernels
 
-__global__ __launch_bounds__(kBlock) void k_dot2(int64_t n, const float* __restrict__ a, const float* __restrict__ b,
-                                                 const float* __restrict__ c, const float* __restrict__ d,
-                                                 double* partials, const double* __restrict__ sv) {
+// partial z.q
+__global__ __launch_bounds__(kBlock) void k_dot(int64_t n, const float* __restrict__ a, const float* __restrict__ b,
+                                                double* partials, const double* __restrict__ sv) {
     if (sv[SV_DONE] != 0.0) return;
-    double t[2] = {0.0, 0.0};
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        t[0] += (double)a[i] * b[i];
-        t[1] += (double)c[i] * d[i];
-    }
-    block_partials<2>(t, partials);
-}
-
-// op 0: pq, pr -> alpha ; op 1: rr -> done test ; op 2: zq -> beta ; op 3: rr0 init
-__global__ __launch_bounds__(kBlock) void k_fcg_fin(const double* __restrict__ partials, int nparts, int op,
-                                                    double* __restrict__ sv) {
-    if (op != 3 && sv[SV_DONE] != 0.0) return;
-    const int nv = (op == 0 || op == 2) ? 2 : 1;
-    double t[2] = {0.0, 0.0};
-    for (int b = threadIdx.x; b < nparts; b += blockDim.x) {
-        t[0] += partials[(size_t)nv * b];
-        if (nv == 2) t[1] += partials[(size_t)nv * b + 1];
-    }
-    block_sum<2>(t);
-    if (threadIdx.x != 0) return;
-    if (op == 0) {
-        sv[SV_PQ] = t[0];
-        sv[SV_PR] = t[1];
-        sv[SV_ALPHA] = t[1] / t[0];
-    } else if (op == 1) {
-        sv[SV_RR] = t[0];
-        sv[SV_IT] += 1.0;
-        if (t[0] <= sv[SV_TOL2] * sv[SV_RR0] || sv[SV_IT] >= sv[SV_MAXIT] || !(t[0] == t[0])) sv[SV_DONE] = 1.0;
-    } else if (op == 2) {
-        sv[SV_ZQ] = t[0];
-        sv[SV_BETA] = -t[0] / sv[SV_PQ];
-    } else {
-        sv[SV_RR0] = t[0];
-        sv[SV_RR] = t[0];
-        sv[SV_IT] = 0.0;
-        sv[SV_DONE] = (t[0] == 0.0) ? 1.0 : 0.0;
-    }
-}
-
-// x += alpha p; r -= alpha q; partial r.r
-__global__ __launch_bounds__(kBlock) void k_fcg_update(int64_t n, float* __restrict__ x, float* __restrict__ r,
-                                                       const float* __restrict__ p, const float* __restrict__ q,
-                                                       double* partials, const double* __restrict__ sv) {
-    if (sv[SV_DONE] != 0.0) return;
-    const float alpha = (float)sv[SV_ALPHA];
     double t[1] = {0.0};
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        x[i] += alpha * p[i];
-        float ri = r[i] - alpha * q[i];
-        r[i] = ri;
-        t[0] += (double)ri * ri;
-    }
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        t[0] += (double)a[i] * b[i];
     block_partials<1>(t, partials);
 }
 
-// p = z + beta p
-__global__ void k_fcg_dir(int64_t n, const float* __restrict__ z, float* __restrict__ p,
-                          const double* __restrict__ sv) {
-    if (sv[SV_DONE] != 0.0) return;
-    const float beta = (float)sv[SV_BETA];
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+// rr0 from the start's partials
+__global__ __launch_bounds__(kBlock) void k_fcg_start(const double* __restrict__ partials, int nparts,
+                                                      double* __restrict__ sv) {
+    double t[1] = {0.0};
+    for (int b = threadIdx.x; b < nparts; b += blockDim.x) t[0] += partials[b];
+    block_sum<1>(t);
+    if (threadIdx.x != 0) return;
+    sv[SV_RR0] = t[0];
+    sv[SV_RR] = t[0];
+    sv[SV_IT] = 0.0;
+    sv[SV_DONE] = (t[0] == 0.0) ? 1.0 : 0.0;
+}
+
+// An iteration's reductions are added up inside the two vector kernels that need
+// them, by every block in the same order (block 0 stores the scalars to the
+// other slot), and the dots in the products that form their vectors: a one-block
+// kernel per reduction took 4.7 us and a dot's own pass 5.8 us.  An iteration
+// on 1,013,643 DOF 385 -> 290 us with the cycle's fused steps, on 135,360 DOF 235 -> 160 us.
+
+// alpha = p.r / p.q; x += alpha p; r -= alpha q; partial r.r.  SMOOTH: with the
+// V-cycle's first smoothing step of the new r (d = x2 = c2 Binv r), whose own
+// pass would read r again.
+template <bool SMOOTH>
+__global__ __launch_bounds__(kBlock) void k_fcg_update(int n_nodes, float* __restrict__ x, float* __restrict__ r,
+                                                       const float* __restrict__ p, const float* __restrict__ q,
+                                                       const double* __restrict__ pq, int npq,
+                                                       double* __restrict__ partials, const double* __restrict__ in,
+                                                       double* __restrict__ out, const float* __restrict__ binv,
+                                                       const float* __restrict__ coef, float* __restrict__ d,
+                                                       float* __restrict__ x2) {
+    __shared__ double sh[SV_N];
+    const int c = (int)threadIdx.x - (kBlock - kWave);
+    if (c >= 0 && c < SV_N) sh[c] = in[c];
+    double t[2] = {0.0, 0.0};
+#pragma unroll 4
+    for (int b = threadIdx.x; b < npq; b += kBlock) {
+        t[0] += pq[2 * (int64_t)b];
+        t[1] += pq[2 * (int64_t)b + 1];
+    }
+    block_sum<2>(t);
+    if (threadIdx.x == 0 && sh[SV_DONE] == 0.0) {
+        sh[SV_PQ] = t[0];
+        sh[SV_PR] = t[1];
+        sh[SV_ALPHA] = t[1] / t[0];
+    }
+    __syncthreads();
+    if (blockIdx.x == 0 && threadIdx.x < SV_N) out[threadIdx.x] = sh[threadIdx.x];
+    if (sh[SV_DONE] != 0.0) return;
+    const float alpha = (float)sh[SV_ALPHA];
+    const float c2 = SMOOTH ? coef[1] : 0.f;
+    double rr[1] = {0.0};
+    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n_nodes; i += gridDim.x * kBlock) {
+        const int64_t e = 3 * (int64_t)i;
+        float rn[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            x[e + k] += alpha * p[e + k];
+            rn[k] = r[e + k] - alpha * q[e + k];
+            r[e + k] = rn[k];
+            rr[0] += (double)rn[k] * rn[k];
+        }
+        if (SMOOTH) cheb_first(i, n_nodes, binv, rn[0], rn[1], rn[2], c2, d, x2);
+    }
+    block_partials<1>(rr, partials);
+}
+
+// convergence of r.r; beta = -z.q / p.q; p = z + beta p
+__global__ __launch_bounds__(kBlock) void k_fcg_dir(int64_t n, const float* __restrict__ z, float* __restrict__ p,
+                                                    const double* __restrict__ zq, int nzq,
+                                                    const double* __restrict__ rr, int nrr,
+                                                    const double* __restrict__ in, double* __restrict__ out) {
+    __shared__ double sh[SV_N];
+    const int c = (int)threadIdx.x - (kBlock - kWave);
+    if (c >= 0 && c < SV_N) sh[c] = in[c];
+    double t[2] = {0.0, 0.0};
+#pragma unroll 4
+    for (int b = threadIdx.x; b < nzq; b += kBlock) t[0] += zq[b];
+#pragma unroll 4
+    for (int b = threadIdx.x; b < nrr; b += kBlock) t[1] += rr[b];
+    block_sum<2>(t);
+    if (threadIdx.x == 0 && sh[SV_DONE] == 0.0) {
+        sh[SV_RR] = t[1];
+        sh[SV_IT] += 1.0;
+        if (t[1] <= sh[SV_TOL2] * sh[SV_RR0] || sh[SV_IT] >= sh[SV_MAXIT] || !(t[1] == t[1])) sh[SV_DONE] = 1.0;
+        sh[SV_ZQ] = t[0];
+        sh[SV_BETA] = -t[0] / sh[SV_PQ];
+    }
+    __syncthreads();
+    if (blockIdx.x == 0 && threadIdx.x < SV_N) out[threadIdx.x] = sh[threadIdx.x];
+    if (sh[SV_DONE] != 0.0) return;
+    const float beta = (float)sh[SV_BETA];
+    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
         p[i] = z[i] + beta * p[i];
 }
 
@@ -1062,10 +1203,19 @@ void build_structured_pattern(Level& lv, std::vector<int32_t>& kdiag, std::vecto
                 elems[fill[(i & 1) + 2 * (j & 1) + 4 * (k & 1)]++] = (int32_t)(i + (int64_t)nx * (j + (int64_t)ny * k));
 }
 
+template <int MODE>
+void launch_coarse(hipStream_t st, const Level& lv, const float* x, float* y, const float* b,
+                   const ChebStep& C = ChebStep()) {
+    constexpr int kRows = kBlock / 32;
+    const int n = (int)lv.n_nodes;
+    hipLaunchKernelGGL(k_coarse3<MODE>, dim3((n + kRows - 1) / kRows), dim3(kBlock), 0, st, n, lv.d_rp, lv.d_bc,
+                       lv.d_val, x, y, b, C);
+}
+
 int apply_level(Multigrid* mg, hipStream_t st, int l, const float* x, float* y) {
     Level& lv = mg->L[l];
     if (l == 0) launch_sell3<float>(st, 0, mg->fine, lv.d_val, x, y, nullptr, nullptr, nullptr);
-    else launch_spmv3<float>(st, 0, (int)lv.n_nodes, lv.d_rp, lv.d_bc, lv.d_val, x, y, nullptr, nullptr, nullptr);
+    else launch_coarse<0>(st, lv, x, y, nullptr);
     return ASEND_OK;
 }
 
@@ -1081,18 +1231,48 @@ void residual_level(Multigrid* mg, hipStream_t st, int l, const float* b, const 
     Level& lv = mg->L[l];
     if (l == 0 && cycle_half(mg)) launch_sell3_h(st, 3, mg->fine, mg->val16, mg->dinv16, x, r, b);
     else if (l == 0) launch_sell3<float>(st, 3, mg->fine, lv.d_val, x, r, b, nullptr, nullptr);
-    else launch_spmv3<float>(st, 3, (int)lv.n_nodes, lv.d_rp, lv.d_bc, lv.d_val, x, r, b, nullptr, nullptr);
+    else launch_coarse<3>(st, lv, x, r, b);
 }
 
-// Chebyshev smoothing of degree mg->cheb_degree on level l with the
-// preconditioner M = 3x3 block Jacobi (default) or point Jacobi; the finest
-// level uses the learned factor P = L L^T instead when it is selected.  The
-// step coefficients live in device memory (coef_slot).
+// Whether level l smooths with 3x3 block Jacobi, whose steps after the first are
+// part of their residual's product.
+bool block_smoothed(const Multigrid* mg, int l) {
+    return mg->smoother_kind == 1 && !(l == 0 && mg->fine_smoother == 1);
+}
+
+// First block-Jacobi step from zero on level l: d = x = c2 Binv b.
+void smooth_first(Multigrid* mg, hipStream_t st, int l, const float* b, float* x) {
+    Level& lv = mg->L[l];
+    hipLaunchKernelGGL(k_cheb_block, dim3(nb_for(lv.n_nodes)), dim3(256), 0, st, (int)lv.n_nodes, lv.binv, b,
+                       mg->d_coef + coef_slot(mg, l, 0), lv.d, x);
+}
+
+// Block-Jacobi step k on level l, x -> out; the partials of out.q where q is given
+// (finest level).
+StepParts smooth_step(Multigrid* mg, hipStream_t st, int l, int k, const float* b, const float* x, float* out,
+                      const float* q) {
+    Level& lv = mg->L[l];
+    ChebStep C;
+    C.binv = lv.binv;
+    C.coef = mg->d_coef + coef_slot(mg, l, k);
+    C.d = lv.d;
+    C.out = out;
+    C.q = q;
+    C.n = (int)lv.n_nodes;
+    if (l == 0)
+        return launch_cheb_step(st, mg->fine, lv.d_val, cycle_half(mg) ? mg->val16 : nullptr, mg->dinv16, x, b, C,
+                                mg->partials, mg->fold);
+    launch_coarse<8>(st, lv, x, nullptr, b, C);
+    return StepParts();
+}
+
+// Chebyshev smoothing of degree mg->cheb_degree on level l, in place, with point
+// Jacobi or, on the finest level when it is selected, the learned factor
+// P = L L^T.  The step coefficients live in device memory (coef_slot).
 void smooth(Multigrid* mg, hipStream_t st, int l, const float* b, float* x, bool zero_start) {
     Level& lv = mg->L[l];
     const bool learned = (l == 0 && mg->fine_smoother == 1);
-    const bool block = !learned && mg->smoother_kind == 1;
-    const float* dinv = (learned || block) ? nullptr : lv.d_dinv;
+    const float* dinv = learned ? nullptr : lv.d_dinv;
     const float* coef = mg->d_coef + coef_slot(mg, learned ? (int)mg->L.size() : l, 0);
     const int nblk = nb_for(lv.n_nodes);
     for (int k = 0; k < mg->cheb_degree; ++k) {
@@ -1101,15 +1281,6 @@ void smooth(Multigrid* mg, hipStream_t st, int l, const float* b, float* x, bool
         if (!first) {
             residual_level(mg, st, l, b, x, lv.r);
             r = lv.r;
-        }
-        if (block) {
-            if (first)
-                hipLaunchKernelGGL(k_cheb_block<true>, dim3(nblk), dim3(256), 0, st, (int)lv.n_nodes, lv.binv, r,
-                                   coef + 2 * k, lv.d, x);
-            else
-                hipLaunchKernelGGL(k_cheb_block<false>, dim3(nblk), dim3(256), 0, st, (int)lv.n_nodes, lv.binv, r,
-                                   coef + 2 * k, lv.d, x);
-            continue;
         }
         if (learned && cycle_half(mg) && mg->factor.Ls16) {
             // FP16 factor, Chebyshev step fused into its second product
@@ -1129,41 +1300,70 @@ void smooth(Multigrid* mg, hipStream_t st, int l, const float* b, float* x, bool
     }
 }
 
-void restrict_to(Multigrid* mg, hipStream_t st, int l, const float* rf, float* bc) {
+// bc = R rf; `first`: with the first smoothing step of level l + 1 into its x2.
+void restrict_to(Multigrid* mg, hipStream_t st, int l, const float* rf, float* bc, bool first = false) {
     Level& c = mg->L[l + 1];
     Level& f = mg->L[l];
     const int32_t* frank = (l == 0) ? mg->d_rank0 : nullptr;
-    int64_t nnodes = c.n_nodes;
-    hipLaunchKernelGGL(k_restrict3, dim3((unsigned)((nnodes + 255) / 256)), dim3(256), 0, st, c.n[0], c.n[1], c.n[2],
-                       f.n[0], f.n[1], c.dax.ri[0], c.dax.rw[0], c.dax.ri[1], c.dax.rw[1], c.dax.ri[2], c.dax.rw[2],
-                       frank, rf, bc);
+    const unsigned nblk = (unsigned)((c.n_nodes + kTransferNodes - 1) / kTransferNodes);
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(nblk), dim3(kTransferBlock), 0, st, c.n[0], c.n[1], c.n[2], f.n[0], f.n[1],
+                           c.dax.ri[0], c.dax.rw[0], c.dax.ri[1], c.dax.rw[1], c.dax.ri[2], c.dax.rw[2], frank, rf, bc,
+                           c.binv, mg->d_coef + coef_slot(mg, l + 1, 0), c.d, c.x2);
+    };
+    if (first) go(k_restrict3<true>);
+    else go(k_restrict3<false>);
 }
 
 void prolong_add(Multigrid* mg, hipStream_t st, int l, const float* xc, float* xf) {
     Level& c = mg->L[l + 1];
     Level& f = mg->L[l];
     const int32_t* frank = (l == 0) ? mg->d_rank0 : nullptr;
-    int64_t nnodes = f.n_nodes;
-    hipLaunchKernelGGL(k_prolong_add3, dim3((unsigned)((nnodes + 255) / 256)), dim3(256), 0, st, f.n[0], f.n[1],
-                       f.n[2], c.n[0], c.n[1], c.dax.pi[0], c.dax.pw[0], c.dax.pi[1], c.dax.pw[1], c.dax.pi[2],
-                       c.dax.pw[2], frank, xc, xf);
+    const unsigned nblk = (unsigned)((f.n_nodes + kTransferNodes - 1) / kTransferNodes);
+    hipLaunchKernelGGL(k_prolong_add3, dim3(nblk), dim3(kTransferBlock), 0, st, f.n[0], f.n[1], f.n[2], c.n[0],
+                       c.n[1], c.dax.pi[0], c.dax.pw[0], c.dax.pi[1], c.dax.pw[1], c.dax.pi[2], c.dax.pw[2], frank, xc,
+                       xf);
 }
 
-// One V-cycle: x = M b on level l (x overwritten).
-void vcycle(Multigrid* mg, hipStream_t st, int l, const float* b, float* x) {
+// One V-cycle: x = M b on level l (x overwritten; not the level's x2).  first_done:
+// the first smoothing step already stands in the level's d and x2 (block Jacobi).
+// With q (finest level, block Jacobi) the partials of x.q come back.
+// Block Jacobi alternates between x2 and x, 2 * degree - 1 times, so that the last
+// step ends in x.
+StepParts vcycle(Multigrid* mg, hipStream_t st, int l, const float* b, float* x, bool first_done = false,
+                 const float* q = nullptr) {
     const int nl = (int)mg->L.size();
     if (l == nl - 1) {
         hipLaunchKernelGGL(k_dense_gemv, dim3((mg->nco + 3) / 4), dim3(256), 0, st, mg->nco, mg->d_Ainv, b, x);
-        return;
+        return StepParts();
     }
     Level& lv = mg->L[l];
     Level& cv = mg->L[l + 1];
-    smooth(mg, st, l, b, x, true);
-    residual_level(mg, st, l, b, x, lv.r);
-    restrict_to(mg, st, l, lv.r, cv.b);
-    vcycle(mg, st, l + 1, cv.b, cv.x);
-    prolong_add(mg, st, l, cv.x, x);
-    smooth(mg, st, l, b, x, false);
+    const bool coarse_first = l + 1 < nl - 1 && block_smoothed(mg, l + 1);
+    auto coarse = [&](float* xl) {
+        residual_level(mg, st, l, b, xl, lv.r);
+        restrict_to(mg, st, l, lv.r, cv.b, coarse_first);
+        vcycle(mg, st, l + 1, cv.b, cv.x, coarse_first);
+        prolong_add(mg, st, l, cv.x, xl);
+    };
+    if (!block_smoothed(mg, l)) {
+        smooth(mg, st, l, b, x, true);
+        coarse(x);
+        smooth(mg, st, l, b, x, false);
+        return StepParts();
+    }
+    float *cur = lv.x2, *nxt = x;
+    StepParts P;
+    auto step = [&](int k, const float* qk) {
+        P = smooth_step(mg, st, l, k, b, cur, nxt, qk);
+        std::swap(cur, nxt);
+    };
+    const int D = mg->cheb_degree;
+    if (!first_done) smooth_first(mg, st, l, b, cur);
+    for (int k = 1; k < D; ++k) step(k, nullptr);
+    coarse(cur);
+    for (int k = 0; k < D; ++k) step(k, k == D - 1 ? q : nullptr);
+    return P;
 }
 
 // kPowerIts steps of the power iteration for lambda_max(M A) on level l,
@@ -1224,6 +1424,7 @@ void free_level(Level& lv) {
     fr(lv.d_pidx);
     fr(lv.d_pval);
     fr(lv.x);
+    fr(lv.x2);
     fr(lv.b);
     fr(lv.r);
     fr(lv.d);
@@ -1307,6 +1508,7 @@ int mg_create(Multigrid** out, int nx, int ny, int nz, const int32_t* rank_of_gr
     if (mg->L.size() < 2) return mgfail(mg, ASEND_ERR_UNSUPPORTED, "grid too small for a multigrid hierarchy");
     for (auto& lv : mg->L) {
         MGCHK(hipMalloc((void**)&lv.x, lv.n_dof * sizeof(float)));
+        MGCHK(hipMalloc((void**)&lv.x2, lv.n_dof * sizeof(float)));
         MGCHK(hipMalloc((void**)&lv.b, lv.n_dof * sizeof(float)));
         MGCHK(hipMalloc((void**)&lv.r, lv.n_dof * sizeof(float)));
         MGCHK(hipMalloc((void**)&lv.d, lv.n_dof * sizeof(float)));
@@ -1321,7 +1523,10 @@ int mg_create(Multigrid** out, int nx, int ny, int nz, const int32_t* rank_of_gr
     MGCHK(hipMalloc((void**)&mg->z, n0 * sizeof(float)));
     MGCHK(hipMalloc((void**)&mg->p, n0 * sizeof(float)));
     MGCHK(hipMalloc((void**)&mg->q, n0 * sizeof(float)));
-    MGCHK(hipMalloc((void**)&mg->partials, 2 * 4096 * sizeof(double)));
+    const size_t n_pair = 2 * (size_t)std::max(4096, mg->fine.n_slices);
+    MGCHK(hipMalloc((void**)&mg->partials, (n_pair + kStepBlocks + 3 * kFoldBlocks) * sizeof(double)));
+    mg->partials_rr = mg->partials + n_pair;
+    mg->fold = mg->partials_rr + kStepBlocks;
     MGCHK(hipMalloc((void**)&mg->sv, 32 * sizeof(double)));
     MGCHK(hipMalloc((void**)&mg->d_lam, kMaxLevels * sizeof(double)));
     MGCHK(hipMalloc((void**)&mg->partials_b, kVecBlocks * sizeof(double)));
@@ -1820,11 +2025,6 @@ int mg_fcg_solve(Multigrid* mg, hipStream_t st, const float* b, float* x, double
         int rc = fine_bound(mg, st);
         if (rc) return rc;
     }
-    // z = B r: one V-cycle, or the learned factor alone
-    auto apply_b = [&](const float* r, float* z) {
-        if (precond == 1) launch_factor_apply(st, mg->factor, r, mg->ft, z);
-        else vcycle(mg, st, 0, r, z);
-    };
     Level& l0 = mg->L[0];
     const int64_t n = l0.n_dof;
     const int nvb = kVecBlocks;
@@ -1839,34 +2039,47 @@ int mg_fcg_solve(Multigrid* mg, hipStream_t st, const float* b, float* x, double
     std::memcpy(mg->h_sv, init, sizeof(init));
     MGCHK(hipMemcpyAsync(mg->sv, mg->h_sv, sizeof(init), hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_fcg_init, dim3(nvb), dim3(kBlock), 0, st, n, b, x, mg->r, mg->partials);
-    hipLaunchKernelGGL(k_fcg_fin, dim3(1), dim3(kBlock), 0, st, mg->partials, nvb, 3, mg->sv);
-    // z = M r ; p = z
-    apply_b(mg->r, mg->z);
-    hipLaunchKernelGGL(k_copy, dim3(nb_for(n)), dim3(256), 0, st, n, mg->z, mg->p);
+    hipLaunchKernelGGL(k_fcg_start, dim3(1), dim3(kBlock), 0, st, mg->partials, nvb, mg->sv);
+    // p = z = B r: one V-cycle, or the learned factor alone
+    if (precond == 1) launch_factor_apply(st, mg->factor, mg->r, mg->ft, mg->p);
+    else vcycle(mg, st, 0, mg->r, mg->p);
     // The learned factor alone is measured against its own untrained start
     // (block Jacobi) on the assembled FP32 values both are built from: 1,368
     // against 1,648 iterations on 40x8x8.  With the reference blocks' more
     // exact products block Jacobi takes 1,051 and the trained factor 1,107.
     Sell3 op = mg->fine;
     if (precond == 1) op.n_uni = 0;
+    // the V-cycle's first smoothing step rides on the update, z.q on its last
+    const bool fused = precond == 0 && block_smoothed(mg, 0);
+    double* const mid = mg->sv + SV_MID;
+    const int nub = step_blocks(l0.n_nodes), ndb = step_blocks(n);
     // one block of check_every iterations; kernels only (scalars stay on the
     // device), so the block can be captured once and replayed as a graph
     auto iterations = [&]() {
         for (int k = 0; k < check_every; ++k) {
-            // q = A p ; alpha = (p.r)/(p.q)
-            launch_sell3<float>(st, 0, op, l0.d_val, mg->p, mg->q, nullptr, nullptr, nullptr);
-            hipLaunchKernelGGL(k_dot2, dim3(nvb), dim3(kBlock), 0, st, n, mg->p, mg->q, mg->p, mg->r, mg->partials,
-                               mg->sv);
-            hipLaunchKernelGGL(k_fcg_fin, dim3(1), dim3(kBlock), 0, st, mg->partials, nvb, 0, mg->sv);
-            hipLaunchKernelGGL(k_fcg_update, dim3(nvb), dim3(kBlock), 0, st, n, x, mg->r, mg->p, mg->q, mg->partials,
-                               mg->sv);
-            hipLaunchKernelGGL(k_fcg_fin, dim3(1), dim3(kBlock), 0, st, mg->partials, nvb, 1, mg->sv);
-            // z = M r ; beta = -(z.q)/(p.q) ; p = z + beta p
-            apply_b(mg->r, mg->z);
-            hipLaunchKernelGGL(k_dot2, dim3(nvb), dim3(kBlock), 0, st, n, mg->z, mg->q, mg->z, mg->q, mg->partials,
-                               mg->sv);
-            hipLaunchKernelGGL(k_fcg_fin, dim3(1), dim3(kBlock), 0, st, mg->partials, nvb, 2, mg->sv);
-            hipLaunchKernelGGL(k_fcg_dir, dim3(nvb), dim3(kBlock), 0, st, n, mg->z, mg->p, mg->sv);
+            // q = A p ; alpha = (p.r)/(p.q) ; x, r
+            const StepParts pq =
+                launch_sell3_step<float>(st, 7, op, l0.d_val, mg->p, mg->q, mg->r, mg->partials, mg->fold, nullptr);
+            auto update = [&](auto kern) {
+                hipLaunchKernelGGL(kern, dim3(nub), dim3(kBlock), 0, st, (int)l0.n_nodes, x, mg->r, mg->p, mg->q, pq.p,
+                                   pq.n, mg->partials_rr, mg->sv, mid, l0.binv, mg->d_coef + coef_slot(mg, 0, 0), l0.d,
+                                   l0.x2);
+            };
+            if (fused) update(k_fcg_update<true>);
+            else update(k_fcg_update<false>);
+            // z = B r ; beta = -(z.q)/(p.q) ; p = z + beta p
+            StepParts zq;
+            if (fused) {
+                zq = vcycle(mg, st, 0, mg->r, mg->z, true, mg->q);
+            } else {
+                if (precond == 1) launch_factor_apply(st, mg->factor, mg->r, mg->ft, mg->z);
+                else vcycle(mg, st, 0, mg->r, mg->z);
+                hipLaunchKernelGGL(k_dot, dim3(nvb), dim3(kBlock), 0, st, n, mg->z, mg->q, mg->partials, mid);
+                zq.p = mg->partials;
+                zq.n = nvb;
+            }
+            hipLaunchKernelGGL(k_fcg_dir, dim3(ndb), dim3(kBlock), 0, st, n, mg->z, mg->p, zq.p, zq.n,
+                               mg->partials_rr, nub, mid, mg->sv);
         }
     };
     Multigrid::FcgGraph* gr = nullptr;

@@ -102,6 +102,40 @@ def test_vcycle_symmetric_positive(ctx):
     assert b1 @ x1 > 0 and b2 @ x2 > 0
 
 
+@pytest.mark.parametrize("kind, degree", [(1, 1), (1, 2), (1, 3), (0, 1), (0, 2)])
+@pytest.mark.parametrize("mesh, bits", [("lattice", 16), ("distorted", 16), ("distorted", 32)])
+def test_cycle_steps(ctx, kind, degree, mesh, bits):
+    """The cycle's forms over the smoothers, degrees (both parities of its two
+    iterates) and finest operators, on an odd grid of four levels: symmetric, a
+    contraction in the energy norm, and preconditioning a solve of 1e-9.  All
+    vectors are FP32: a symmetry defect of 1e-3 of the energy is its rounding over
+    the smoother's range, a wrong iterate is of the order of the energy itself."""
+    gpu_case(f"cycle steps {kind} {degree} {mesh} {bits}")
+    dims = (37, 9, 7)
+    p = problems.heterogeneous(*dims, seed=8)
+    if mesh == "distorted":
+        p = problems.distorted(p, 3)
+    ctx.mg_set_smoother(kind, degree)
+    problems.upload(ctx, p)
+    ctx.set_grid(*dims)
+    ctx.mg_set_smoother(kind, degree)
+    ctx.mg_set_cycle_precision(bits)
+    ctx.assemble()
+    assert len(ctx.mg_info()) >= 3
+    rng = np.random.default_rng(5)
+    e1, e2 = (rng.standard_normal(p.n_dof).astype(np.float32) for _ in range(2))
+    A = lambda v: ctx.mg_apply(0, np.ascontiguousarray(v, dtype=np.float32)).astype(np.float64)
+    b1, b2 = A(e1), A(e2)
+    x1 = ctx.mg_vcycle(b1.astype(np.float32)).astype(np.float64)
+    x2 = ctx.mg_vcycle(b2.astype(np.float32)).astype(np.float64)
+    assert abs(b2 @ x1 - b1 @ x2) <= 1e-3 * np.sqrt((b1 @ x1) * (b2 @ x2))
+    rest = e1 - x1
+    assert rest @ A(rest) < 0.5 * (e1 @ b1)
+    _, st = ctx.solve(p.f, ctx.opts(api.SOLVE_IR_MIXED, api.PC_MG, tol=1e-9, inner_tol=1e-3, max_it=2000,
+                                    check_every=3))
+    assert st.converged and st.rel_residual <= 1e-9 and st.iterations < 200
+
+
 @pytest.mark.parametrize("dims", [(14, 5, 4), (40, 8, 8)])
 def test_mg_mixed_solve_matches_ldl(ctx, dims):
     gpu_case(f"mg mixed solve {dims}")
