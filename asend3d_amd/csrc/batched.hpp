@@ -15,8 +15,9 @@ constexpr int kNrhs = 16;  // right-hand sides per variant advanced together
 struct OperatorView {
     int n_rows = 0;                 // block rows (nodes)
     int n_slices = 0;
-    int64_t n_slots = 0;
-    const int32_t* h_sptr = nullptr;  // host copy of the slice pointer
+    const int32_t* order = nullptr;   // batch_row_order (host)
+    const int32_t* h_rp = nullptr;    // block-row pointers (host)
+    const int32_t* sptr = nullptr;
     const int32_t* scol = nullptr;
     const float* K32 = nullptr;
     const double* K64 = nullptr;
@@ -33,15 +34,15 @@ struct BatchStats {
 };
 
 struct Batch;
+// Order of a variant's rows in a batch: order[i] is the row that stands i-th.
+std::vector<int32_t> batch_row_order(int64_t n, const int32_t* rp, const int32_t* bc, const double* xyz);
 int batch_create(Batch** out, const std::vector<OperatorView>& ops);
 void batch_destroy(Batch* b);
 const char* batch_error(const Batch* b);
-int64_t batch_rows_total(const Batch* b);
-int64_t batch_row_offset(const Batch* b, int v);
-// h_F / h_U: [rows_total][3][kNrhs] (FP64, host); systems with rhs index >= nrhs
-// or zero right-hand side are skipped.
+// rhs / x: per variant nrhs vectors of its DOFs, one after another (FP64, host);
+// zero right-hand sides are skipped.
 // verbose != 0 prints one progress line per refinement to stderr.
-int batch_solve(Batch* b, const double* h_F, double* h_U, int nrhs, double tol, double inner_tol, int64_t max_it,
+int batch_solve(Batch* b, const double* const* rhs, double* const* x, int nrhs, double tol, double inner_tol, int64_t max_it,
                 int check_every, int verbose, BatchStats* stats);
 
 }  // namespace asend

@@ -39,6 +39,7 @@ struct asend_ctx {
     int64_t n_nodes = 0, n_dof = 0, n_el = 0, nnzb = 0;
     int64_t grid[3] = {0, 0, 0};
     std::vector<int32_t> h_rp, h_bc, h_color_ptr;
+    std::vector<int32_t> batch_order;  // row order in batches (formed on first use)
 
     int32_t *d_conn_r = nullptr, *d_rp = nullptr, *d_bc = nullptr, *d_kdiag = nullptr, *d_elems = nullptr;
     // fine operator storage: sliced ELL of 3x3 blocks, 64-row slices
@@ -352,6 +353,7 @@ void ldl_release(asend_ctx* ctx) {
 }
 
 void free_mesh(asend_ctx* ctx) {
+    ctx->batch_order.clear();
     ldl_release(ctx);
     ctx->ldl_block_dofs = -1;
     dfree(ctx->d_dmat);
@@ -2419,7 +2421,6 @@ int asend_bench_spmv(asend_ctx* ctx, int precision, int n_iter, double* avg_ms) 
 
 struct asend_batch {
     Batch* b = nullptr;
-    std::vector<int64_t> n_dof;
     std::string err;
 };
 
@@ -2442,13 +2443,18 @@ int asend_batch_create(asend_ctx* const* variants, int n_variants, asend_batch**
         OperatorView& o = ops[v];
         o.n_rows = (int)c->n_nodes;
         o.n_slices = (int)c->n_slices;
-        o.n_slots = c->n_slots;
-        o.h_sptr = c->h_sptr.data();
+        if (c->batch_order.empty()) {
+            std::vector<double> xyz(3 * c->n_nodes);
+            HIPCHK_CTX(hipMemcpy(xyz.data(), c->d_xyz_r, xyz.size() * 8, hipMemcpyDeviceToHost));
+            c->batch_order = batch_row_order(c->n_nodes, c->h_rp.data(), c->h_bc.data(), xyz.data());
+        }
+        o.order = c->batch_order.data();
+        o.h_rp = c->h_rp.data();
+        o.sptr = c->d_sptr;
         o.scol = c->d_scol;
         o.K32 = c->d_K32;
         o.K64 = c->d_K64;
         o.dinv32 = c->d_dinv32;
-        ab->n_dof.push_back(c->n_dof);
         HIPCHK_CTX(hipStreamSynchronize(c->st));
     }
     int rc = batch_create(&ab->b, ops);
@@ -2473,24 +2479,11 @@ int asend_batch_solve(asend_batch* ab, int nrhs, const double* const* rhs, doubl
                       double inner_tol, int64_t max_it, int check_every, int verbose, asend_batch_stats* stats) {
     if (!ab || !ab->b || !rhs || !x || nrhs < 1 || nrhs > kNrhs) return ASEND_ERR_ARG;
     Batch* b = ab->b;
-    const int nv = (int)ab->n_dof.size();
-    const int64_t ne = batch_rows_total(b) * 3 * kNrhs;
-    std::vector<double> F(ne, 0.0), U(ne, 0.0);
-    for (int v = 0; v < nv; ++v) {
-        const int64_t nd = ab->n_dof[v], off = batch_row_offset(b, v) * 3;
-        for (int j = 0; j < nrhs; ++j)
-            for (int64_t d = 0; d < nd; ++d) F[(off + d) * kNrhs + j] = rhs[v][j * nd + d];
-    }
     BatchStats bs;
-    int rc = batch_solve(b, F.data(), U.data(), nrhs, tol, inner_tol, max_it, check_every, verbose, &bs);
+    int rc = batch_solve(b, rhs, x, nrhs, tol, inner_tol, max_it, check_every, verbose, &bs);
     if (rc) {
         ab->err = batch_error(b);
         return rc;
-    }
-    for (int v = 0; v < nv; ++v) {
-        const int64_t nd = ab->n_dof[v], off = batch_row_offset(b, v) * 3;
-        for (int j = 0; j < nrhs; ++j)
-            for (int64_t d = 0; d < nd; ++d) x[v][j * nd + d] = U[(off + d) * kNrhs + j];
     }
     if (stats) {
         stats->outer_iterations = bs.outer_iterations;

@@ -796,7 +796,7 @@ void launch_diag_inv(hipStream_t st, int n_rows, const int32_t* sptr, const int3
 // row (zero blocks pad rows shorter than the slice width), its column index
 // at scol[64*k + lane] and its 9 values at val[64*(9k + c) + lane], so every
 // load of the wavefront is one contiguous 256 B (FP32) / 512 B (FP64) burst
-// and no cross-lane reduction is needed.  Modes as the block-row SpMV.
+// and no cross-lane reduction is needed.
 // ---------------------------------------------------------------------------
 template <bool NT, typename T>
 __device__ __forceinline__ T sell_load(const T* p) {

@@ -6,7 +6,6 @@
 
 namespace asend {
 
-constexpr int kSpmvBlocks = 4096;  // blocks of the block-row SpMV (each a contiguous row range)
 constexpr int kVecBlocks = 2048;   // blocks of the streaming vector kernels
 constexpr int kMaxPartials = 8192; // partial-sum slots per reduction value
 

@@ -106,3 +106,36 @@ def test_batch_matches_single_solves():
     b.close()
     for c in ctxs:
         c.close()
+
+
+@pytest.mark.parametrize("nrhs", [1, 16])
+@pytest.mark.parametrize("grids", [[(1, 1, 1)], [(4, 3, 3), (3, 1, 2), (9, 8, 6)]], ids=["one cell", "three"])
+def test_batch_row_order(grids, nrhs):
+    """Variants whose nodes fill no whole brick or slice, one of them on a distorted
+    mesh, with one and all right-hand sides: every system against the FP64 solve
+    of its own context (both to 1e-9 of the load, so the solutions to that
+    times the condition number, below 1e7 here, of the clamped bodies)."""
+    gpu_case(f"batch order {grids} {nrhs}")
+    ps = [problems.heterogeneous(*g, seed=3 + i) for i, g in enumerate(grids)]
+    ps[-1] = problems.distorted(ps[-1], 2)
+    rng = np.random.default_rng(7)
+    rhs = [rng.standard_normal((nrhs, p.n_dof)) for p in ps]
+    for p, r in zip(ps, rhs):
+        r[:, p.pen_dofs] = 0.0
+    ctxs = []
+    for p in ps:
+        c = api.Context(0)
+        problems.upload(c, p)
+        c.assemble()
+        ctxs.append(c)
+    b = api.Batch(ctxs)
+    xs, st = b.solve(rhs, tol=1e-9, inner_tol=1e-3, check_every=4)
+    assert st.unconverged == 0 and st.max_rel_residual <= 1e-9, st.as_dict()
+    o = api.Context.opts(api.SOLVE_PCG_FP64, api.PC_JACOBI, tol=1e-12, max_it=100000, check_every=16)
+    for c, r, x in zip(ctxs, rhs, xs):
+        for j in range(nrhs):
+            u = c.solve(r[j], o)[0]
+            assert np.abs(x[j] - u).max() <= 1e-6 * np.abs(u).max(), j
+    b.close()
+    for c in ctxs:
+        c.close()
