@@ -814,18 +814,28 @@ __device__ __forceinline__ T sell_load(const T* p) {
 //   6: 4 paused while sc->gate is set (the mixed solve's FP32 step)
 //   7: y = K x with x = p, f = r, partials p.y, p.r (the flexible PCG step)
 //   8: a Chebyshev step on f - K x (ChebStep)
+//   9: a power step out = Binv (K x) / 2 (ChebStep: binv, out, n)
 // Launches with loop scalars return at once when they are done.
 // Row epilogue: a = row r of K x, xr and fr the row's own values of x and f (where the mode
 // reads them); writes y and adds to the row's partial sums.
 template <int MODE>
 constexpr bool mode_reads_f() {
-    return MODE >= 2;
+    return MODE >= 2 && MODE != 9;
 }
 
 template <typename T, int MODE>
 __device__ __forceinline__ void row_epilogue(int r, const T (&a)[3], const T (&xr)[3], const T (&fr)[3],
                                              T* __restrict__ y, const ChebStep& C, double (&part)[3]) {
     const int64_t d = 3 * (int64_t)r;
+    if (MODE == 9) {
+        float m[9];
+#pragma unroll
+        for (int k = 0; k < 9; ++k) m[k] = C.binv[(int64_t)k * C.n + r];
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            C.out[d + i] = kPowerScale * (float)(m[3 * i] * a[0] + m[3 * i + 1] * a[1] + m[3 * i + 2] * a[2]);
+        return;
+    }
     if (MODE == 8) {
         float m[9];
 #pragma unroll
@@ -882,7 +892,7 @@ __device__ __forceinline__ void row_values(const T* __restrict__ v, int r, T (&o
 // the block's partial sums of a mode, stored for its finalize kernel
 template <int MODE>
 __device__ __forceinline__ void mode_partials(const double (&part)[3], double* partials, const ChebStep& C) {
-    if (MODE == 0 || MODE == 3 || (MODE == 8 && !C.q)) return;
+    if (MODE == 0 || MODE == 3 || MODE == 9 || (MODE == 8 && !C.q)) return;
     if (MODE == 4 || MODE == 6) {
         double t[3] = {part[0], part[1], part[2]};
         block_partials<3>(t, partials);
@@ -1454,6 +1464,12 @@ void launch_sell3_h(hipStream_t st, int mode, const Sell3& A, const __half* val,
     } else {
         sell3h_go<0>(st, A, val, dinv32, x, y, f, nullptr, ChebStep());
     }
+}
+
+void launch_power_step(hipStream_t st, const Sell3& A, const float* val, const __half* val16, const float* dinv32,
+                       const float* x, const ChebStep& C) {
+    if (val16) sell3h_go<9>(st, A, val16, dinv32, x, nullptr, nullptr, nullptr, C);
+    else sell3_go<float, 9>(st, A, val, x, nullptr, nullptr, nullptr, nullptr, C);
 }
 
 StepParts launch_cheb_step(hipStream_t st, const Sell3& A, const float* val, const __half* val16, const float* dinv32,

@@ -197,6 +197,12 @@ StepParts launch_sell3_step(hipStream_t st, int mode, const Sell3& A, const T* v
 StepParts launch_cheb_step(hipStream_t st, const Sell3& A, const float* val, const __half* val16, const float* dinv32,
                            const float* x, const float* b, const ChebStep& C, double* partials, double* fold);
 
+// One step of the power iteration that bounds the block-Jacobi smoother of the finest
+// level: out = Binv (A x) / 2 (the product as launch_cheb_step's).
+constexpr float kPowerScale = 0.5f;
+void launch_power_step(hipStream_t st, const Sell3& A, const float* val, const __half* val16, const float* dinv32,
+                       const float* x, const ChebStep& C);
+
 template <typename T>
 void launch_pcg_init(hipStream_t st, int64_t n, const T* b, const T* dinv, T* x, T* r, T* p, double* partials,
                      Scalars* sc);

@@ -159,6 +159,7 @@ struct Multigrid {
     // coarsest dense inverse
     int nco = 0;
     double* d_Ainv = nullptr;
+    double* d_gj = nullptr;  // scratch of its elimination: pivot block's inverse, pivot rows
     // FCG work vectors (fine level)
     float *r = nullptr, *z = nullptr, *p = nullptr, *q = nullptr;
     // block partials: pairs of the finest products (or z.q), the update's r.r, folded sums
@@ -418,7 +419,8 @@ __global__ __launch_bounds__(kTransferBlock) void k_prolong_add3(
 // Products with a coarse operator (block rows of up to 27 blocks, values
 // component-major per row): half a wavefront per row, its lanes the row's blocks,
 // so that all of a row's loads are one burst of 9 coalesced reads.
-//   0: y = K x;  3: y = b - K x;  8: a Chebyshev step on b - K x (ChebStep)
+//   0: y = K x;  3: y = b - K x;  8: a Chebyshev step on b - K x (ChebStep);
+//   9: a power step out = Binv (K x) / 2
 // Mode 8 is the residual and the smoothing update of a step in one launch, both
 // little more than a launch each on the deeper levels: mean over the levels under
 // 337,881 nodes 5.8 + 3.4 us -> 5.7 us, under 45,120 nodes 3.8 + 3.3 -> 3.6 us.
@@ -438,6 +440,9 @@ __global__ __launch_bounds__(kBlock) void k_coarse3(int n_rows, const int32_t* _
     const int i = min(sub, 2);
     float m[3] = {0.f, 0.f, 0.f}, f[3] = {0.f, 0.f, 0.f}, di = 0.f, xi = 0.f, c1 = 0.f, c2 = 0.f;
     if (MODE == 3) f[0] = b[d + i];
+    if (MODE == 9)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) m[j] = C.binv[(int64_t)(3 * i + j) * C.n + r];
     if (MODE == 8) {
         c1 = C.coef[0];
         c2 = C.coef[1];
@@ -467,6 +472,7 @@ __global__ __launch_bounds__(kBlock) void k_coarse3(int n_rows, const int32_t* _
     const float ai = i == 0 ? a0 : (i == 1 ? a1 : a2);
     if (MODE == 0) y[d + i] = ai;
     if (MODE == 3) y[d + i] = f[0] - ai;
+    if (MODE == 9) C.out[d + i] = kPowerScale * (m[0] * a0 + m[1] * a1 + m[2] * a2);
     if (MODE == 8) {
         const float z = m[0] * (f[0] - a0) + m[1] * (f[1] - a1) + m[2] * (f[2] - a2);
         const float e = c1 * di + c2 * z;
@@ -800,43 +806,44 @@ __global__ void k_cheb_step(int64_t n, const float* __restrict__ dinv, const flo
 // kept in lam_out.  A broken-down estimate (not finite or not positive)
 // writes zero coefficients (no smoothing) and is reported when the host
 // reads the bounds back.
-// Power iteration helpers.  x is kept at the scale of the previous step:
-// step k computes w = M A (x / |x|), |w|^2 (the estimate of lambda_max^2 of
-// M A), and stores x = w.  M is the 3x3 block-Jacobi (binv), point-Jacobi
-// (dinv) or identity (both null: y already preconditioned) smoother.
+// Power iteration helpers.
+// Block Jacobi: lambda_max lies between 1 (a vector on one node) and 24 (the trace
+// of an element's block-scaled matrix), so 20 steps of x = M A x / 2 stay within
+// 1e-6 to 4e21 of the start and need no norm but those of the last two vectors:
+// a step is the product alone (mode 9), 5.7 us on a coarse level against 11.5 us
+// with the norm's two launches.
+// The others keep x at the scale of the previous step: step k computes
+// w = M A (x / |x|), |w|^2 (the estimate of lambda_max^2 of M A), and stores
+// x = w.  M is the point-Jacobi (dinv) or identity (null: y already
+// preconditioned) smoother.
 
 // The second half of a step after y = A x: w = s M y with s = 1 / sqrt(*nrm_prev)
 // (1 on the first step, whose x is the raw start), x = w, partial |w|^2 per
 // workgroup (k_power_fin adds them).
-__global__ __launch_bounds__(kBlock) void k_power_finish(int n_nodes, const float* __restrict__ binv,
-                                                         const float* __restrict__ dinv, const float* __restrict__ y,
-                                                         float* __restrict__ x, const double* __restrict__ nrm_prev,
-                                                         double* partials) {
+__global__ __launch_bounds__(kBlock) void k_power_finish(int64_t n, const float* __restrict__ dinv,
+                                                         const float* __restrict__ y, float* __restrict__ x,
+                                                         const double* __restrict__ nrm_prev, double* partials) {
     const float s = nrm_prev ? (float)(1.0 / sqrt(*nrm_prev)) : 1.f;
     double t[1] = {0.0};
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n_nodes; i += gridDim.x * blockDim.x) {
-        const float r0 = y[3 * i], r1 = y[3 * i + 1], r2 = y[3 * i + 2];
-        float z0 = r0, z1 = r1, z2 = r2;
-        if (binv) {
-            float m[9];
-            for (int q = 0; q < 9; ++q) m[q] = binv[(int64_t)q * n_nodes + i];
-            z0 = m[0] * r0 + m[1] * r1 + m[2] * r2;
-            z1 = m[3] * r0 + m[4] * r1 + m[5] * r2;
-            z2 = m[6] * r0 + m[7] * r1 + m[8] * r2;
-        } else if (dinv) {
-            z0 *= dinv[3 * i];
-            z1 *= dinv[3 * i + 1];
-            z2 *= dinv[3 * i + 2];
-        }
-        z0 *= s;
-        z1 *= s;
-        z2 *= s;
-        x[3 * i] = z0;
-        x[3 * i + 1] = z1;
-        x[3 * i + 2] = z2;
-        t[0] += (double)z0 * z0 + (double)z1 * z1 + (double)z2 * z2;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        const float z = s * (dinv ? y[i] * dinv[i] : y[i]);
+        x[i] = z;
+        t[0] += (double)z * z;
     }
     block_partials<1>(t, partials);
+}
+
+// Of the last two vectors of a block-Jacobi power iteration: the partials of their
+// squared norms are added here, *out = lambda^2.
+__global__ __launch_bounds__(kBlock) void k_power_ratio(const double* __restrict__ partials, int nparts,
+                                                        double* __restrict__ out) {
+    double t[2] = {0.0, 0.0};
+    for (int b = threadIdx.x; b < nparts; b += blockDim.x) {
+        t[0] += partials[2 * b];
+        t[1] += partials[2 * b + 1];
+    }
+    block_sum<2>(t);
+    if (threadIdx.x == 0) *out = t[1] / (t[0] * (double)(kPowerScale * kPowerScale));
 }
 
 // *out = sum of the step's partials, in workgroup order
@@ -924,81 +931,90 @@ __global__ __launch_bounds__(1024) void k_gauss_jordan_lds(int n, double* __rest
     for (int64_t t = threadIdx.x; t < (int64_t)n * n; t += blockDim.x) Ag[t] = A[t];
 }
 
-// Blocked in-place Gauss-Jordan inverse of an SPD matrix (no pivoting),
-// kGjBs pivots per step K (columns k0 .. k0 + kb - 1), two launches per step:
-//   k_gj_pivot: P = A_KK^-1, then the pivot row panel A_{K,:} <- P A_{K,:}
-//               (A_KK <- P);
-//   k_gj_update: every other row i, A_ij <- (j in K ? 0 : A_ij) - sum_l A_il(old) (new A_K)_lj.
+// Blocked in-place Gauss-Jordan inverse of an SPD matrix (no pivoting), kGjBs
+// pivots per step K (columns k0 .. k0 + kb - 1), two launches per step:
+//   k_gj_pivot: P = A_KK^-1 and a copy S of the pivot row panel A_{K,:};
+//   k_gj_update, one workgroup per row i: with c = A_{i,K} P (rows of K: c = -P_i),
+//               A_ij <- (row of K ? 0 : A_ij) - c S_j outside K, -c in it.
 // This is the scalar elimination applied kb pivots at a time; A is streamed
 // once per step by many workgroups instead of once per pivot by one.
+// A step on 224 DOF took 83 us in the pivot kernel, which formed the whole panel
+// P S by itself and passed the pivot column through LDS, and 11 us in the update;
+// 17 and 11 us now.
 constexpr int kGjBs = 32;
 
-// one workgroup of 256 threads
-__global__ __launch_bounds__(256) void k_gj_pivot(int n, int k0, double* __restrict__ A) {
-    __shared__ double P[kGjBs * kGjBs];
-    const int kb = min(kGjBs, n - k0);
-    const int tid = threadIdx.x;
-    for (int t = tid; t < kb * kb; t += blockDim.x) P[t] = A[(int64_t)(k0 + t / kb) * n + k0 + t % kb];
-    __syncthreads();
-    // P <- P^-1 in one wavefront without barriers: lane j < 32 holds column j,
-    // padded with the identity to 32 x 32; the pivot column of each step is
-    // read from lane kk by shuffles
-    if (tid < 64) {
-        const int j = tid;
-        double a[kGjBs];
-#pragma unroll
-        for (int i = 0; i < kGjBs; ++i) a[i] = (j < kb && i < kb) ? P[i * kb + j] : (i == j ? 1.0 : 0.0);
-        for (int kk = 0; kk < kb; ++kk) {
-            double akk = 0.0;
-#pragma unroll
-            for (int i = 0; i < kGjBs; ++i) akk = (i == kk) ? a[i] : akk;
-            const double ip = 1.0 / __shfl(akk, kk);
-            const double rk = (j == kk ? 1.0 : akk) * ip;
-#pragma unroll
-            for (int i = 0; i < kGjBs; ++i) {
-                const double ci = __shfl(a[i], kk);
-                a[i] = (i == kk) ? rk : (j == kk ? 0.0 : a[i]) - ci * rk;
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < kGjBs; ++i)
-            if (j < kb && i < kb) P[i * kb + j] = a[i];
-    }
-    __syncthreads();
-    // row panel, one column per thread (each thread reads its column before
-    // writing it)
-    for (int j = tid; j < n; j += blockDim.x) {
-        if (j >= k0 && j < k0 + kb) {
-            for (int m = 0; m < kb; ++m) A[(int64_t)(k0 + m) * n + j] = P[m * kb + (j - k0)];
-        } else {
-            double col[kGjBs];
-#pragma unroll
-            for (int l = 0; l < kGjBs; ++l) col[l] = l < kb ? A[(int64_t)(k0 + l) * n + j] : 0.0;
-            for (int m = 0; m < kb; ++m) {
-                double acc = 0.0;
-#pragma unroll
-                for (int l = 0; l < kGjBs; ++l)
-                    if (l < kb) acc += P[m * kb + l] * col[l];
-                A[(int64_t)(k0 + m) * n + j] = acc;
-            }
-        }
-    }
+// value of lane l in all lanes (l the same in all)
+__device__ __forceinline__ double lane_value(double v, int l) {
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_readlane((int)b, l), hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// one workgroup (256 threads) per row outside the pivot block
-__global__ __launch_bounds__(256) void k_gj_update(int n, int k0, double* __restrict__ A) {
-    __shared__ double c[kGjBs];
+// one workgroup of 256 threads; P: kGjBs x kGjBs
+__global__ __launch_bounds__(256) void k_gj_pivot(int n, int k0, const double* __restrict__ A, double* __restrict__ P,
+                                                  double* __restrict__ S) {
     const int kb = min(kGjBs, n - k0);
-    const int i = (int)blockIdx.x < k0 ? (int)blockIdx.x : (int)blockIdx.x + kb;
-    if ((int)threadIdx.x < kb) c[threadIdx.x] = A[(int64_t)i * n + k0 + threadIdx.x];
+    if (threadIdx.x >= kWave) {
+        // the other wavefronts copy the panel
+        for (int64_t t = threadIdx.x - kWave; t < (int64_t)kb * n; t += blockDim.x - kWave) S[t] = A[(int64_t)k0 * n + t];
+        return;
+    }
+    // one wavefront without barriers: lane j < 32 holds column j, padded with the
+    // identity to 32 x 32.  The rows move up by one at each pivot (and stand as
+    // they were after 32), so that the pivot row is always a[0].
+    const int j = threadIdx.x;
+    double a[kGjBs];
+#pragma unroll
+    for (int i = 0; i < kGjBs; ++i)
+        a[i] = (j < kb && i < kb) ? A[(int64_t)(k0 + i) * n + k0 + j] : (i == j ? 1.0 : 0.0);
+    for (int kk = 0; kk < kGjBs; ++kk) {
+        const bool own = j == kk;
+        const double ip = 1.0 / lane_value(a[0], kk);
+        const double rk = (own ? 1.0 : a[0]) * ip;
+#pragma unroll
+        for (int i = 1; i < kGjBs; ++i) {
+            const double ci = lane_value(a[i], kk);
+            a[i - 1] = (own ? 0.0 : a[i]) - ci * rk;
+        }
+        a[kGjBs - 1] = rk;
+    }
+#pragma unroll
+    for (int i = 0; i < kGjBs; ++i)
+        if (j < kGjBs) P[i * kGjBs + j] = a[i];
+}
+
+// one workgroup (256 threads) per row
+__global__ __launch_bounds__(256) void k_gj_update(int n, int k0, double* __restrict__ A, const double* __restrict__ P,
+                                                   const double* __restrict__ S) {
+    __shared__ double c[kGjBs], aik[kGjBs];
+    const int kb = min(kGjBs, n - k0);
+    const int i = blockIdx.x;
+    const bool pivot = i >= k0 && i < k0 + kb;
+    double* row = A + (int64_t)i * n;
+    if (threadIdx.x < kGjBs) aik[threadIdx.x] = (int)threadIdx.x < kb ? row[k0 + threadIdx.x] : 0.0;
+    __syncthreads();
+    if (threadIdx.x < kGjBs) {
+        double t = 0.0;
+        if (pivot) {
+            t = -P[(i - k0) * kGjBs + threadIdx.x];
+        } else {
+#pragma unroll
+            for (int l = 0; l < kGjBs; ++l) t += aik[l] * P[l * kGjBs + threadIdx.x];
+        }
+        c[threadIdx.x] = t;
+    }
     __syncthreads();
     for (int j = threadIdx.x; j < n; j += blockDim.x) {
-        const bool in_k = (j >= k0 && j < k0 + kb);
-        double acc = in_k ? 0.0 : A[(int64_t)i * n + j];
+        double acc;
+        if (j >= k0 && j < k0 + kb) {
+            acc = -c[j - k0];
+        } else {
+            acc = pivot ? 0.0 : row[j];
 #pragma unroll
-        for (int l = 0; l < kGjBs; ++l)
-            if (l < kb) acc -= c[l] * A[(int64_t)(k0 + l) * n + j];
-        A[(int64_t)i * n + j] = acc;
+            for (int l = 0; l < kGjBs; ++l)
+                if (l < kb) acc -= c[l] * S[(int64_t)l * n + j];
+        }
+        row[j] = acc;
     }
 }
 
@@ -1372,11 +1388,25 @@ StepParts vcycle(Multigrid* mg, hipStream_t st, int l, const float* b, float* x,
 void enqueue_power(Multigrid* mg, hipStream_t st, int l, bool learned, const PowerScratch& ps) {
     Level& lv = mg->L[l];
     const int64_t n = lv.n_dof;
-    const bool block = !learned && mg->smoother_kind == 1;
-    const float* binv = block ? lv.binv : nullptr;
-    const float* dinv = (learned || block) ? nullptr : lv.d_dinv;
     hipLaunchKernelGGL(k_fill_hash, dim3(nb_for(n)), dim3(256), 0, st, n, lv.x);
     const int nblk = std::min<int>(kVecBlocks, (int)((lv.n_nodes + kBlock - 1) / kBlock));
+    if (!learned && mg->smoother_kind == 1) {
+        float *cur = lv.x, *nxt = lv.x2;
+        for (int it = 0; it < kPowerIts; ++it) {
+            ChebStep C;
+            C.binv = lv.binv;
+            C.out = nxt;
+            C.n = (int)lv.n_nodes;
+            if (l == 0)
+                launch_power_step(st, mg->fine, lv.d_val, cycle_half(mg) ? mg->val16 : nullptr, mg->dinv16, cur, C);
+            else launch_coarse<9>(st, lv, cur, nullptr, nullptr, C);
+            std::swap(cur, nxt);
+        }
+        hipLaunchKernelGGL(k_dot2_partials, dim3(nblk), dim3(kBlock), 0, st, n, nxt, nxt, cur, cur, ps.partials);
+        hipLaunchKernelGGL(k_power_ratio, dim3(1), dim3(kBlock), 0, st, ps.partials, nblk, ps.out);
+        return;
+    }
+    const float* dinv = learned ? nullptr : lv.d_dinv;
     for (int it = 0; it < kPowerIts; ++it) {
         apply_cycle_op(mg, st, l, lv.x, lv.r);
         const float* y = lv.r;
@@ -1387,8 +1417,7 @@ void enqueue_power(Multigrid* mg, hipStream_t st, int l, bool learned, const Pow
         }
         const double* prev = it == 0 ? nullptr : ps.pp + (it - 1) % 2;
         double* out = it == kPowerIts - 1 ? ps.out : ps.pp + it % 2;
-        hipLaunchKernelGGL(k_power_finish, dim3(nblk), dim3(kBlock), 0, st, (int)lv.n_nodes, binv, dinv, y, lv.x, prev,
-                           ps.partials);
+        hipLaunchKernelGGL(k_power_finish, dim3(nblk), dim3(kBlock), 0, st, n, dinv, y, lv.x, prev, ps.partials);
         hipLaunchKernelGGL(k_power_fin, dim3(1), dim3(kBlock), 0, st, ps.partials, nblk, out);
     }
 }
@@ -1518,6 +1547,7 @@ int mg_create(Multigrid** out, int nx, int ny, int nz, const int32_t* rank_of_gr
     mg->h_coef.assign(2 * kChebMaxDegree * (mg->L.size() + 1), 0.f);
     MGCHK(hipMalloc((void**)&mg->d_coef, mg->h_coef.size() * sizeof(float)));
     MGCHK(hipMalloc((void**)&mg->d_Ainv, (size_t)mg->nco * mg->nco * sizeof(double)));
+    MGCHK(hipMalloc((void**)&mg->d_gj, (size_t)kGjBs * (kGjBs + mg->nco) * sizeof(double)));
     const int64_t n0 = mg->L[0].n_dof;
     MGCHK(hipMalloc((void**)&mg->r, n0 * sizeof(float)));
     MGCHK(hipMalloc((void**)&mg->z, n0 * sizeof(float)));
@@ -1529,10 +1559,10 @@ int mg_create(Multigrid** out, int nx, int ny, int nz, const int32_t* rank_of_gr
     mg->fold = mg->partials_rr + kStepBlocks;
     MGCHK(hipMalloc((void**)&mg->sv, 32 * sizeof(double)));
     MGCHK(hipMalloc((void**)&mg->d_lam, kMaxLevels * sizeof(double)));
-    MGCHK(hipMalloc((void**)&mg->partials_b, kVecBlocks * sizeof(double)));
+    MGCHK(hipMalloc((void**)&mg->partials_b, 2 * kVecBlocks * sizeof(double)));
     MGCHK(hipMalloc((void**)&mg->sv_b, 4 * sizeof(double)));
     MGCHK(hipHostMalloc((void**)&mg->h_sv_b, sizeof(double), hipHostMallocDefault));
-    MGCHK(hipMalloc((void**)&mg->partials_c, kVecBlocks * sizeof(double)));
+    MGCHK(hipMalloc((void**)&mg->partials_c, 2 * kVecBlocks * sizeof(double)));
     MGCHK(hipMalloc((void**)&mg->sv_c, 4 * sizeof(double)));
     mg->pw_main.partials = mg->partials;
     mg->pw_main.out = mg->sv + SV_N;
@@ -1557,6 +1587,7 @@ void mg_destroy(Multigrid* mg) {
     for (auto& lv : mg->L) free_level(lv);
     fr(mg->o_rank0);
     fr(mg->d_Ainv);
+    fr(mg->d_gj);
     fr(mg->r);
     fr(mg->z);
     fr(mg->p);
@@ -2000,11 +2031,10 @@ int mg_setup(Multigrid* mg, hipStream_t st, const double* d_E, const double* d_n
                            mg->nco, mg->d_Ainv);
     else
         for (int k0 = 0; k0 < mg->nco; k0 += kGjBs) {
-            const int kb = std::min(kGjBs, mg->nco - k0);
-            hipLaunchKernelGGL(k_gj_pivot, dim3(1), dim3(256), 0, st, mg->nco, k0, mg->d_Ainv);
-            if (mg->nco > kb)
-                hipLaunchKernelGGL(k_gj_update, dim3((unsigned)(mg->nco - kb)), dim3(256), 0, st, mg->nco, k0,
-                                   mg->d_Ainv);
+            hipLaunchKernelGGL(k_gj_pivot, dim3(1), dim3(256), 0, st, mg->nco, k0, mg->d_Ainv, mg->d_gj,
+                               mg->d_gj + kGjBs * kGjBs);
+            hipLaunchKernelGGL(k_gj_update, dim3((unsigned)mg->nco), dim3(256), 0, st, mg->nco, k0, mg->d_Ainv,
+                               mg->d_gj, mg->d_gj + kGjBs * kGjBs);
         }
     MGCHK(hipGetLastError());
     // join the power streams: everything that uses the hierarchy is ordered
