@@ -698,10 +698,7 @@ __device__ __forceinline__ void step_scalars(const Scalars* __restrict__ in, con
     double v[nv];
 #pragma unroll
     for (int i = 0; i < nv; ++i) v[i] = 0.0;
-#pragma unroll 4
-    for (int b = threadIdx.x; b < nparts; b += kBlock)
-#pragma unroll
-        for (int i = 0; i < nv; ++i) v[i] += partials[(size_t)nv * b + i];
+    thread_sums<nv>(partials, nparts, v);
     block_sum<nv>(v);
     if (threadIdx.x == 0 && !fin_idle(OP, sh)) fin_apply(OP, v[0], v[nv >= 2 ? 1 : 0], v[nv == 3 ? 2 : 0], sh);
     __syncthreads();

@@ -1079,11 +1079,7 @@ __global__ __launch_bounds__(kBlock) void k_fcg_update(int n_nodes, float* __res
     const int c = (int)threadIdx.x - (kBlock - kWave);
     if (c >= 0 && c < SV_N) sh[c] = in[c];
     double t[2] = {0.0, 0.0};
-#pragma unroll 4
-    for (int b = threadIdx.x; b < npq; b += kBlock) {
-        t[0] += pq[2 * (int64_t)b];
-        t[1] += pq[2 * (int64_t)b + 1];
-    }
+    thread_sums<2>(pq, npq, t);
     block_sum<2>(t);
     if (threadIdx.x == 0 && sh[SV_DONE] == 0.0) {
         sh[SV_PQ] = t[0];
@@ -1119,11 +1115,10 @@ __global__ __launch_bounds__(kBlock) void k_fcg_dir(int64_t n, const float* __re
     __shared__ double sh[SV_N];
     const int c = (int)threadIdx.x - (kBlock - kWave);
     if (c >= 0 && c < SV_N) sh[c] = in[c];
-    double t[2] = {0.0, 0.0};
-#pragma unroll 4
-    for (int b = threadIdx.x; b < nzq; b += kBlock) t[0] += zq[b];
-#pragma unroll 4
-    for (int b = threadIdx.x; b < nrr; b += kBlock) t[1] += rr[b];
+    double tz[1] = {0.0}, tr[1] = {0.0};
+    thread_sums<1>(zq, nzq, tz);
+    thread_sums<1>(rr, nrr, tr);
+    double t[2] = {tz[0], tr[0]};
     block_sum<2>(t);
     if (threadIdx.x == 0 && sh[SV_DONE] == 0.0) {
         sh[SV_RR] = t[1];
