@@ -84,6 +84,9 @@ struct asend_ctx {
         double *w64 = nullptr, *kh64 = nullptr;
         float *w32 = nullptr, *kh32 = nullptr;
     } uni_bufs[2];
+    // penalty terms, room for every slice: allocated with the mesh, since
+    // captured graphs hold their addresses while asend_set_penalty changes the
+    // penalised DOFs
     double* d_uni_pen64 = nullptr;
     float* d_uni_pen32 = nullptr;
     int n_uni_pslots = 0;
@@ -1765,7 +1768,8 @@ int asend_upload_mesh(asend_ctx* ctx, int elem_type, int64_t n_mesh_nodes, const
         if (uni_tables(n_nodes, n_el, conn_r, nbr, el)) {
             const size_t ns = (size_t)ctx->n_slices;
             if ((rc = dalloc(ctx, &ctx->d_uni_nbr, nbr.size())) || (rc = dalloc(ctx, &ctx->d_uni_el, el.size())) ||
-                (rc = dalloc(ctx, &ctx->d_uni_pslot, ns)))
+                (rc = dalloc(ctx, &ctx->d_uni_pslot, ns)) || (rc = dalloc(ctx, &ctx->d_uni_pen64, 192 * ns)) ||
+                (rc = dalloc(ctx, &ctx->d_uni_pen32, 192 * ns)))
                 return rc;
             for (auto& b : ctx->uni_bufs)
                 if ((rc = dalloc(ctx, &b.w64, 512 * ns)) || (rc = dalloc(ctx, &b.w32, 512 * ns)) ||
@@ -1913,10 +1917,8 @@ int asend_set_penalty(asend_ctx* ctx, int64_t n, const int64_t* dofs, double sf)
         for (int64_t d : u)
             if (ps[d / 192] < 0) ps[d / 192] = n_ps++;
         ctx->uni[0] = UniOp();
-        if ((rc = dalloc(ctx, &ctx->d_uni_pen64, 192 * (size_t)n_ps)) ||
-            (rc = dalloc(ctx, &ctx->d_uni_pen32, 192 * (size_t)n_ps)))
-            return rc;
-        HIPCHK(hipMemcpy(ctx->d_uni_pslot, ps.data(), ps.size() * 4, hipMemcpyHostToDevice));
+        HIPCHK(hipMemcpyAsync(ctx->d_uni_pslot, ps.data(), ps.size() * 4, hipMemcpyHostToDevice, ctx->st));
+        HIPCHK(hipStreamSynchronize(ctx->st));
         ctx->n_uni_pslots = n_ps;
     }
     ctx->n_pen = (int)u.size();

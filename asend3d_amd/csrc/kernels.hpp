@@ -22,7 +22,9 @@ struct Scalars {
 // from its reference blocks (see k_uni3 in kernels.hip): y_r = sum over the
 // local positions a of row node r in its elements of w_a (K x of the element's
 // row a from its reference blocks), plus the penalty on the diagonal.  Stands for the assembled values val64 / val32
-// (null while the operator was not assembled from the reference blocks).
+// (null while the operator was not assembled from the reference blocks).  A captured
+// launch holds every pointer here by value: the tables keep their addresses as
+// long as the mesh.
 struct UniOp {
     const double* val64 = nullptr;
     const float* val32 = nullptr;

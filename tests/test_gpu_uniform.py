@@ -152,3 +152,85 @@ def test_many_partial_sums(ctx, distorted):
     assert st.converged and st.iterations < 1500
     res = np.linalg.norm(p.f - ctx.spmv(u)) / np.linalg.norm(p.f)
     assert res <= 1.01e-6, res
+
+
+# constraint sets that touch few slices, more of them, and fewer again
+def constraint_sets(p):
+    x = p.mesh.xyz
+    di = np.asarray(p.dof_index).reshape(-1, 6)[:, :3]
+    left, right, floor = (np.isclose(x[:, 0], 0.0), np.isclose(x[:, 0], x[:, 0].max()), np.isclose(x[:, 2], 0.0))
+    half = left & (x[:, 1] <= 0.5 * x[:, 1].max())
+    return [di[s].reshape(-1).astype(np.int64) for s in (left, left | right | floor, half)]
+
+
+@pytest.mark.parametrize("precond", [api.PC_MG, api.PC_LEARNED])
+def test_new_constraints_between_solves(precond):
+    """A context whose captured iterations have run goes on after each new set
+    of constraints as a context that never had another one: the same
+    iterations and solution, and that of the assembled matrix."""
+    gpu_case(f"constraints changed between multigrid solves, preconditioner {precond}")
+    dims = (33, 9, 7)
+    p = problems.heterogeneous(*dims, seed=6, sigma_ln=0.7)
+    f = np.random.default_rng(2).standard_normal(p.n_dof)
+
+    def make():
+        c = api.Context(0)
+        c.learned_init(1)
+        problems.upload(c, p)
+        c.set_grid(*dims)
+        return c
+
+    def solve(c, pen):
+        c.set_penalty(pen, 0.0)
+        c.assemble()
+        rhs = f.copy()
+        rhs[pen] = 0.0
+        u, st = c.solve(rhs, c.opts(api.SOLVE_IR_MIXED, precond, tol=1e-9, inner_tol=1e-3, max_it=2000, check_every=3))
+        assert st.converged and st.fallback_used == 0
+        rp, cols, vals = c.get_matrix()
+        ref = spla.spsolve(sp.csr_matrix((vals, cols, rp), shape=(p.n_dof, p.n_dof)).tocsc(), rhs)
+        assert np.linalg.norm(u - ref) <= 1e-5 * np.linalg.norm(ref)
+        return u, st.iterations
+
+    old = make()
+    for k, pen in enumerate(constraint_sets(p)):
+        new = make()
+        (u, it), (u_new, it_new) = solve(old, pen), solve(new, pen)
+        assert it == it_new and np.array_equal(u, u_new), (k, it, it_new)
+        new.close()
+    old.close()
+
+
+@pytest.mark.parametrize("mode", [api.NM_FP64, api.NM_MIXED])
+def test_new_constraints_between_newmark_runs(mode):
+    """The same of Newmark steps, whose captured launches also outlive a change
+    of the constraints."""
+    gpu_case(f"constraints changed between Newmark runs, solver {mode}")
+    p = problems.cantilever(20, 5, 4)
+    n = 30
+    fac = np.sin(np.pi * np.arange(n) / n)
+    f = np.random.default_rng(4).standard_normal(p.n_dof)
+
+    def make(pen):
+        c = api.Context(0)
+        problems.upload(c, p, rho=np.full(p.mesh.n_el, 7850.0))
+        c.set_penalty(pen, 0.0)
+        c.newmark_set_solver(mode)
+        c.newmark_setup(5e-5, 0.25, 0.5)
+        return c
+
+    def run(c):
+        _, u, v, a, st = c.newmark_run(n, f, fac, tol=1e-10, max_it_step=400)
+        assert st.graph_used == 1 and st.unconverged_steps == 0
+        return u, v, a, st.total_iterations
+
+    sets = constraint_sets(p)
+    old = make(sets[0])
+    for k, pen in enumerate(sets):
+        if k:
+            old.set_penalty(pen, 0.0)
+        new = make(pen)
+        a, b = run(old), run(new)
+        assert a[3] == b[3] and all(np.array_equal(x, y) for x, y in zip(a[:3], b[:3])), (k, a[3], b[3])
+        new.close()
+    old.close()
