@@ -189,6 +189,7 @@ struct Multigrid {
     // the finest level's block-Jacobi bound was enqueued by mg_fine_setup
     // (coefficients formed on the device, value in d_lam[0])
     bool fine_pending = false;
+    bool fine_broken = false;  // neither form of its estimate came to a bound
     hipStream_t lam_stream = nullptr;
     // device scalars of the FCG loop: before the update, (SV_MID) before the direction
     double* sv = nullptr;
@@ -848,17 +849,15 @@ __global__ void k_cheb_step(int64_t n, const float* __restrict__ dinv, const flo
     }
 }
 
-// Chebyshev coefficients of one level from its power-iteration estimate
-// lambda = sqrt(nrm2[0]), the device twin of cheb_coefficients; lambda is
-// kept in lam_out.  A broken-down estimate (not finite or not positive)
-// writes zero coefficients (no smoothing) and is reported when the host
-// reads the bounds back.
 // Power iteration helpers.
-// Block Jacobi: lambda_max lies between 1 (a vector on one node) and 24 (the trace
-// of an element's block-scaled matrix), so 20 steps of x = M A x / 2 stay within
-// 1e-6 to 4e21 of the start and need no norm but those of the last two vectors:
-// a step is the product alone (mode 9), 5.7 us on a coarse level against 11.5 us
-// with the norm's two launches.
+// Block Jacobi: where A is positive definite lambda_max lies between 1 (a vector on
+// one node) and 27 (the blocks of a row; 24 from semidefinite element matrices),
+// so 20 steps of x = M A x / 2 stay within 1e-6 to 4e22 of the start and need no
+// norm but those of the last two vectors: a step is the product alone (mode 9),
+// 5.7 us on a coarse level against 11.5 us with the norm's two launches.  On the
+// finest level an indefinite A (a tangent between Newton steps, K minus a shift)
+// has no such bound, and past 160 the steps leave the range of FP32; the estimate
+// is then formed again with the norm of every step (estimate_lmax).
 // The others keep x at the scale of the previous step: step k computes
 // w = M A (x / |x|), |w|^2 (the estimate of lambda_max^2 of M A), and stores
 // x = w.  M is the point-Jacobi (dinv) or identity (null: y already
@@ -902,6 +901,11 @@ __global__ __launch_bounds__(kBlock) void k_power_fin(const double* __restrict__
     if (threadIdx.x == 0) *out = t[0];
 }
 
+// Chebyshev coefficients of one level from its power-iteration estimate
+// lambda = sqrt(nrm2[0]), the device twin of cheb_coefficients; lambda is
+// kept in lam_out.  A broken-down estimate (not finite or not positive)
+// writes zero coefficients (no smoothing) and is reported when the host
+// reads the bounds back.
 __global__ void k_cheb_coef(const double* __restrict__ nrm2, double lo_frac, double hi_frac, int degree,
                             float* __restrict__ out, double* __restrict__ lam_out) {
     if (blockIdx.x != 0 || threadIdx.x != 0) return;
@@ -1395,11 +1399,15 @@ StepParts vcycle(Multigrid* mg, hipStream_t st, int l, const float* b, float* x,
 // kPowerIts steps of the power iteration for lambda_max(M A) on level l,
 // enqueued on st with the given reduction scratch; ||M A x||^2 of the last
 // step lands in nrm2[0].
-void enqueue_power(Multigrid* mg, hipStream_t st, int l, bool learned, const PowerScratch& ps) {
+void enqueue_power(Multigrid* mg, hipStream_t st, int l, bool learned, const PowerScratch& ps,
+                   bool normalised = false) {
     Level& lv = mg->L[l];
     const int64_t n = lv.n_dof;
     hipLaunchKernelGGL(k_fill_hash, dim3(nb_for(n)), dim3(256), 0, st, n, lv.x);
     const int nblk = std::min<int>(kVecBlocks, (int)((lv.n_nodes + kBlock - 1) / kBlock));
+    // |w|^2 of step it - 1 and of step it
+    auto norm_in = [&](int it) { return it == 0 ? nullptr : ps.pp + (it - 1) % 2; };
+    auto norm_out = [&](int it) { return it == kPowerIts - 1 ? ps.out : ps.pp + it % 2; };
     if (!learned && mg->smoother_kind == 1) {
         float *cur = lv.x, *nxt = lv.x2;
         for (int it = 0; it < kPowerIts; ++it) {
@@ -1410,8 +1418,15 @@ void enqueue_power(Multigrid* mg, hipStream_t st, int l, bool learned, const Pow
             if (l == 0)
                 launch_power_step(st, mg->fine, lv.d_val, cycle_half(mg) ? mg->val16 : nullptr, mg->dinv16, cur, C);
             else launch_coarse<9>(st, lv, cur, nullptr, nullptr, C);
-            std::swap(cur, nxt);
+            if (normalised) {
+                hipLaunchKernelGGL(k_power_finish, dim3(nblk), dim3(kBlock), 0, st, n, (const float*)nullptr, nxt, cur,
+                                   norm_in(it), ps.partials);
+                hipLaunchKernelGGL(k_power_fin, dim3(1), dim3(kBlock), 0, st, ps.partials, nblk, norm_out(it));
+            } else {
+                std::swap(cur, nxt);
+            }
         }
+        if (normalised) return;
         hipLaunchKernelGGL(k_dot2_partials, dim3(nblk), dim3(kBlock), 0, st, n, nxt, nxt, cur, cur, ps.partials);
         hipLaunchKernelGGL(k_power_ratio, dim3(1), dim3(kBlock), 0, st, ps.partials, nblk, ps.out);
         return;
@@ -1425,10 +1440,9 @@ void enqueue_power(Multigrid* mg, hipStream_t st, int l, bool learned, const Pow
             else launch_factor_apply(st, mg->factor, lv.r, mg->ft, mg->fz);
             y = mg->fz;
         }
-        const double* prev = it == 0 ? nullptr : ps.pp + (it - 1) % 2;
-        double* out = it == kPowerIts - 1 ? ps.out : ps.pp + it % 2;
-        hipLaunchKernelGGL(k_power_finish, dim3(nblk), dim3(kBlock), 0, st, n, dinv, y, lv.x, prev, ps.partials);
-        hipLaunchKernelGGL(k_power_fin, dim3(1), dim3(kBlock), 0, st, ps.partials, nblk, out);
+        hipLaunchKernelGGL(k_power_finish, dim3(nblk), dim3(kBlock), 0, st, n, dinv, y, lv.x, norm_in(it),
+                           ps.partials);
+        hipLaunchKernelGGL(k_power_fin, dim3(1), dim3(kBlock), 0, st, ps.partials, nblk, norm_out(it));
     }
 }
 
@@ -1438,15 +1452,21 @@ int estimate_lmax(Multigrid* mg, hipStream_t st, int l, bool learned, double* ou
     // deterministic pseudo-random start vector (a smooth start such as the
     // constant vector lies near the rigid-body modes and converges slowly);
     // kPowerIts steps without host round trips, ||M A x|| with ||x|| = 1 of
-    // the last step is the estimate
-    enqueue_power(mg, st, l, learned, mg->pw_main);
-    MGCHK(hipGetLastError());
-    MGCHK(hipMemcpyAsync(mg->h_sv, mg->sv + SV_N, sizeof(double), hipMemcpyDeviceToHost, st));
-    MGCHK(hipStreamSynchronize(st));
-    const double lam = std::sqrt(mg->h_sv[0]);
-    if (!(lam > 0.0) || !std::isfinite(lam)) return mgfail(mg, ASEND_ERR_NUMERIC, "power iteration broke down");
-    *out = lam;
-    return ASEND_OK;
+    // the last step is the estimate.  Block Jacobi without the steps' norms
+    // first, with them where that left the range of FP32.
+    const bool block = !learned && mg->smoother_kind == 1;
+    for (int pass = 0; pass < (block ? 2 : 1); ++pass) {
+        enqueue_power(mg, st, l, learned, mg->pw_main, pass == 1);
+        MGCHK(hipGetLastError());
+        MGCHK(hipMemcpyAsync(mg->h_sv, mg->sv + SV_N, sizeof(double), hipMemcpyDeviceToHost, st));
+        MGCHK(hipStreamSynchronize(st));
+        const double lam = std::sqrt(mg->h_sv[0]) / (pass == 1 ? (double)kPowerScale : 1.0);
+        if (lam > 0.0 && std::isfinite(lam)) {
+            *out = lam;
+            return ASEND_OK;
+        }
+    }
+    return mgfail(mg, ASEND_ERR_NUMERIC, "power iteration broke down");
 }
 
 void free_level(Level& lv) {
@@ -1654,12 +1674,9 @@ int mg_set_smoother(Multigrid* mg, int kind, int degree, double lo_frac, double 
     return ASEND_OK;
 }
 
-// Block-Jacobi Chebyshev bound of the finest level, estimated on first use
-// after a setup (host synchronisation: call outside graph capture).
-int fine_bound(Multigrid* mg, hipStream_t st) {
-    if (mg->L.size() < 2 || mg->L[0].lmax > 0.0) return ASEND_OK;
-    // enqueued with the setup: its coefficients are already on the device
-    if (mg->fine_pending) return ASEND_OK;
+// Estimates the finest level's Jacobi Chebyshev bound now and puts its coefficients on
+// the device.
+int form_fine_bound(Multigrid* mg, hipStream_t st) {
     int rc = estimate_lmax(mg, st, 0, false, &mg->L[0].lmax);
     if (rc) return rc;
     const int slot = coef_slot(mg, 0, 0);
@@ -1670,25 +1687,56 @@ int fine_bound(Multigrid* mg, hipStream_t st) {
     return ASEND_OK;
 }
 
-// Recompute the device Chebyshev coefficients from the stored bounds (after a
-// change of degree or interval that keeps the Jacobi kind).
-int mg_check_bounds(Multigrid* mg) {
-    if (!mg->lam_pending) return ASEND_OK;
-    MGCHK(hipStreamSynchronize(mg->lam_stream));
-    mg->lam_pending = false;
-    const size_t l_first = mg->fine_pending ? 0 : 1;
-    mg->fine_pending = false;
-    for (size_t l = l_first; l + 1 < mg->L.size(); ++l) {
-        const double lam = mg->h_lam[l];
-        if (!(lam > 0.0) || !std::isfinite(lam)) {
-            mg->ready = false;
-            return mgfail(mg, ASEND_ERR_NUMERIC, "power iteration broke down");
-        }
-        mg->L[l].lmax = lam;
+// Block-Jacobi Chebyshev bound of the finest level, estimated on first use
+// after a setup (host synchronisation: call outside graph capture).
+int fine_bound(Multigrid* mg, hipStream_t st) {
+    if (mg->L.size() < 2 || mg->L[0].lmax > 0.0) return ASEND_OK;
+    // enqueued with the setup: its coefficients are already on the device
+    if (mg->fine_pending) return ASEND_OK;
+    return form_fine_bound(mg, st);
+}
+
+// The host's look at a finest bound that was enqueued with the setup, once st has
+// been waited for.  Where it left the range of FP32 (zero coefficients on the
+// device) it is formed again: *formed says that cycles that ran before lacked
+// their finest smoothing.  A bound that cannot be formed stays pending for
+// mg_check_bounds to report, the cycle without that smoothing.
+int settle_fine_bound(Multigrid* mg, hipStream_t st, bool* formed) {
+    *formed = false;
+    if (!mg->lam_pending || !mg->fine_pending || mg->fine_broken) return ASEND_OK;
+    const double lam = mg->h_lam[0];
+    if (lam > 0.0 && std::isfinite(lam)) {
+        mg->L[0].lmax = lam;
+    } else {
+        const int rc = form_fine_bound(mg, st);
+        if (rc && rc != ASEND_ERR_NUMERIC) return rc;
+        mg->fine_broken = rc != ASEND_OK;
+        if (mg->fine_broken) return ASEND_OK;
+        *formed = true;
     }
+    mg->fine_pending = false;
     return ASEND_OK;
 }
 
+int mg_check_bounds(Multigrid* mg) {
+    if (!mg->lam_pending) return ASEND_OK;
+    MGCHK(hipStreamSynchronize(mg->lam_stream));
+    bool formed = false;
+    int rc = settle_fine_bound(mg, mg->lam_stream, &formed);
+    if (!rc && mg->fine_pending) rc = mgfail(mg, ASEND_ERR_NUMERIC, "power iteration broke down");
+    mg->lam_pending = false;
+    mg->fine_pending = false;
+    for (size_t l = 1; l + 1 < mg->L.size() && !rc; ++l) {
+        const double lam = mg->h_lam[l];
+        if (!(lam > 0.0) || !std::isfinite(lam)) rc = mgfail(mg, ASEND_ERR_NUMERIC, "power iteration broke down");
+        else mg->L[l].lmax = lam;
+    }
+    if (rc) mg->ready = false;
+    return rc;
+}
+
+// Recompute the device Chebyshev coefficients from the stored bounds (after a
+// change of degree or interval that keeps the Jacobi kind).
 int mg_refresh_coefficients(Multigrid* mg, hipStream_t st) {
     if (!mg->ready) return ASEND_OK;
     int rc = mg_check_bounds(mg);
@@ -1946,6 +1994,7 @@ int mg_fine_setup(Multigrid* mg, hipStream_t st, const float* d_K32, const float
         hipLaunchKernelGGL(k_cheb_coef, dim3(1), dim3(64), 0, st, mg->sv_b, mg->cheb_lo, mg->cheb_hi, mg->cheb_degree,
                            mg->d_coef + coef_slot(mg, 0, 0), mg->d_lam + 0);
         mg->fine_pending = true;
+        mg->fine_broken = false;
     }
     MGCHK(hipGetLastError());
     return ASEND_OK;
@@ -2058,20 +2107,25 @@ int mg_fcg_solve(Multigrid* mg, hipStream_t st, const float* b, float* x, double
     const int64_t n = l0.n_dof;
     const int nvb = kVecBlocks;
     if (fallback_used) *fallback_used = 0;
-    // scalars
-    double init[SV_N];
-    std::memset(init, 0, sizeof(init));
-    // with reliable updates the FP64 residual decides convergence: the
-    // device-side test stops only at max_it
-    init[SV_TOL2] = ru ? 0.0 : rel_tol * rel_tol;
-    init[SV_MAXIT] = (double)max_it;
-    std::memcpy(mg->h_sv, init, sizeof(init));
-    MGCHK(hipMemcpyAsync(mg->sv, mg->h_sv, sizeof(init), hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(k_fcg_init, dim3(nvb), dim3(kBlock), 0, st, n, b, x, mg->r, mg->partials);
-    hipLaunchKernelGGL(k_fcg_start, dim3(1), dim3(kBlock), 0, st, mg->partials, nvb, mg->sv);
-    // p = z = B r: one V-cycle, or the learned factor alone
-    if (precond == 1) launch_factor_apply(st, mg->factor, mg->r, mg->ft, mg->p);
-    else vcycle(mg, st, 0, mg->r, mg->p);
+    auto start = [&]() -> hipError_t {
+        // scalars
+        double init[SV_N];
+        std::memset(init, 0, sizeof(init));
+        // with reliable updates the FP64 residual decides convergence: the
+        // device-side test stops only at max_it
+        init[SV_TOL2] = ru ? 0.0 : rel_tol * rel_tol;
+        init[SV_MAXIT] = (double)max_it;
+        std::memcpy(mg->h_sv, init, sizeof(init));
+        const hipError_t e = hipMemcpyAsync(mg->sv, mg->h_sv, sizeof(init), hipMemcpyHostToDevice, st);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(k_fcg_init, dim3(nvb), dim3(kBlock), 0, st, n, b, x, mg->r, mg->partials);
+        hipLaunchKernelGGL(k_fcg_start, dim3(1), dim3(kBlock), 0, st, mg->partials, nvb, mg->sv);
+        // p = z = B r: one V-cycle, or the learned factor alone
+        if (precond == 1) launch_factor_apply(st, mg->factor, mg->r, mg->ft, mg->p);
+        else vcycle(mg, st, 0, mg->r, mg->p);
+        return hipSuccess;
+    };
+    MGCHK(start());
     // The learned factor alone is measured against its own untrained start
     // (block Jacobi) on the assembled FP32 values both are built from: 1,368
     // against 1,648 iterations on 40x8x8.  With the reference blocks' more
@@ -2166,6 +2220,15 @@ int mg_fcg_solve(Multigrid* mg, hipStream_t st, const float* b, float* x, double
         MGCHK(hipGetLastError());
         MGCHK(hipMemcpyAsync(mg->h_sv, mg->sv, SV_N * sizeof(double), hipMemcpyDeviceToHost, st));
         MGCHK(hipStreamSynchronize(st));
+        if (precond == 0 && mg->fine_smoother == 0) {
+            bool formed = false;
+            const int rc = settle_fine_bound(mg, st, &formed);
+            if (rc) return rc;
+            if (formed) {
+                MGCHK(start());
+                continue;
+            }
+        }
         it = (int64_t)mg->h_sv[SV_IT];
         if (mg->h_sv[SV_DONE] != 0.0) break;
         if (ru && mg->h_sv[SV_RR] <= ru->next) {
@@ -2319,6 +2382,12 @@ int mg_vcycle(Multigrid* mg, hipStream_t st, const float* d_b, float* d_x) {
     if (mg->fine_smoother == 0) {
         int rc = fine_bound(mg, st);
         if (rc) return rc;
+        if (mg->fine_pending && !mg->fine_broken) {
+            bool formed = false;
+            MGCHK(hipStreamSynchronize(st));
+            rc = settle_fine_bound(mg, st, &formed);
+            if (rc) return rc;
+        }
     }
     vcycle(mg, st, 0, d_b, d_x);
     return ASEND_OK;

@@ -4,6 +4,7 @@ V-cycle, and MG-preconditioned mixed-precision solves that reach the FP64
 residual the oracle's LDL^T solution sets."""
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 import oracle as O
 from asend3d_amd import api, problems
@@ -255,3 +256,50 @@ def test_autotuner_choices_are_used(ctx):
     u_ref = ctx.static_compliance(p.f, ref)[0]
     assert np.abs(u - u_ref).max() <= 1e-7 * np.abs(u_ref).max()
     ctx.mg_set_smoother(1, 2, 0.1, 1.15)
+
+
+@pytest.mark.parametrize("mesh", ["lattice", "distorted"])
+def test_bound_of_an_indefinite_operator(ctx, mesh):
+    """K - s M with s a little below the least eigenvalue of the 3x3 diagonal
+    blocks' pencil: not positive definite, block-Jacobi lambda_max far above
+    what 20 FP32 steps without their norms hold ((lambda / 2)^20 > 3e38 from
+    167 on).  The smoother still gets its bound: the setup reports no
+    breakdown, the cycle smooths (its result depends on the degree), and a solve whose
+    first iterations came before the bound was known goes on as one after it."""
+    gpu_case(f"block-Jacobi bound of an indefinite operator, {mesh}")
+    dims = (12, 5, 4)
+    p = problems.cantilever(*dims, 12.0, 5.0, 4.0, E=7.0e4, nu=0.3)
+    if mesh == "distorted":  # so little that all blocks come near zero together
+        p = problems.distorted(p, 4, amp=1e-5, nu_range=(0.3, 0.3))
+    problems.upload(ctx, p, rho=np.full(p.mesh.n_el, 1.0))
+    ctx.set_grid(*dims)
+    ctx.mg_set_smoother(1, 2)
+
+    def blocks(c_mass):
+        ctx.assemble(c_mass)
+        rp, cols, vals = ctx.get_matrix()
+        K = sp.csr_matrix((vals, cols, rp), shape=(p.n_dof, p.n_dof)).tocsr()
+        return np.stack([K[3 * r:3 * r + 3, 3 * r:3 * r + 3].toarray() for r in range(p.n_dof // 3)])
+
+    K, KM = blocks(0.0), blocks(1.0)
+    M = KM - K
+    free = np.ones(p.n_dof // 3, bool)
+    free[p.pen_dofs // 3] = False
+    w = np.linalg.eigvals(np.linalg.solve(M[free], K[free])).real
+    # least eigenvalues of the blocks 1e-3 of what they were: lambda_max of 450
+    s = w.min() * (1.0 - 1e-3)
+    f = np.random.default_rng(3).standard_normal(p.n_dof)
+    f[p.pen_dofs] = 0.0
+    o = ctx.opts(api.SOLVE_IR_MIXED, api.PC_MG, tol=1e-9, inner_tol=1e-3, max_it=6, max_outer=1, check_every=2)
+    ctx.assemble(-s)
+    u1, st1 = ctx.solve(f, o)
+    ctx.mg_set_smoother(1, 2)  # raises where the setup has no bound
+    u2, st2 = ctx.solve(f, o)
+    assert st1.iterations == st2.iterations == 6 and np.array_equal(u1, u2)
+    x = {}
+    for degree in (1, 3):
+        ctx.mg_set_smoother(1, degree)
+        x[degree] = ctx.mg_vcycle(f.astype(np.float32))
+        assert np.isfinite(x[degree]).all()
+    assert np.linalg.norm(x[1] - x[3]) >= 1e-3 * np.linalg.norm(x[1])
+    ctx.mg_set_smoother(1, 2)
