@@ -2786,7 +2786,6 @@ int asend_newmark_run(asend_ctx* ctx, int64_t n_steps, const double* f_shape, co
     // is pending; the iterations pause while one is).  A block leaves the loop
     // scalars in the slot it found them in.
     const bool mixed = nm.mixed == ASEND_NM_MIXED || (nm.mixed == ASEND_NM_AUTO && 8 * ctx->nval() > kMixedAutoBytes);
-    const int blk = mixed ? 2 * kMixedRefreshEvery : 4;
     auto iterations = [&](int count) {
         int cur = 0;
         for (int k = 0; k < count; ++k) {
@@ -2799,8 +2798,14 @@ int asend_newmark_run(asend_ctx* ctx, int64_t n_steps, const double* f_shape, co
             }
         }
     };
-    static_assert(kNewmarkBlock % (2 * kMixedRefreshEvery) == 0 && kNewmarkBlock % 4 == 0, "block lengths");
-    static_assert((2 * kMixedRefreshEvery + 2) % 2 == 0, "a mixed block returns to its scalar slot");
+    // every iteration and every refresh slot moves the loop scalars to the other slot
+    constexpr int kShortMixed = 2 * kMixedRefreshEvery, kShortFp64 = 4;
+    static_assert((kShortMixed + kShortMixed / kMixedRefreshEvery) % 2 == 0 &&
+                      (kNewmarkBlock + kNewmarkBlock / kMixedRefreshEvery) % 2 == 0,
+                  "a mixed block returns to its scalar slot");
+    static_assert(kShortFp64 % 2 == 0 && kNewmarkBlock % 2 == 0, "an FP64 block returns to its scalar slot");
+    static_assert(kNewmarkBlock % kMixedRefreshEvery == 0, "a mixed block ends with a refresh slot");
+    const int blk = mixed ? kShortMixed : kShortFp64;
     auto head = [&]() {
         launch_nm_predict(ctx->st, n, ctx->d_u, nm.v, nm.a, nm.dt, nm.c2, nm.w);
         launch_sell3<double>(ctx->st, 0, ctx->fine(), nm.M64, nm.w, nm.q, nullptr, nullptr, nullptr);
