@@ -449,8 +449,8 @@ class Context:
         return out
 
     def cycle_spmv_timing(self, enable):
-        """Start (True) or stop (False) the event timing of the cycle's FP16
-        SpMV launches; stop returns (launches, total_ms)."""
+        """Start (True) or stop (False) the event timing of the cycle's
+        finest-level operator products; stop returns (launches, total_ms)."""
         n = _i64(0)
         ms = _dbl(0)
         self._chk(_lib.asend_cycle_spmv_timing(self.h, ctypes.c_int(1 if enable else 0), ctypes.byref(n),

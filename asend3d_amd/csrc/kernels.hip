@@ -1373,10 +1373,10 @@ __global__ __launch_bounds__(kSellMaxWaves * kWave) void k_sell3h(int n_rows, in
     mode_partials<MODE>(part, partials, cheb);
 }
 
-// Timing of the FP16 cycle SpMV with the residual epilogue (mode 3, the
-// most frequent kernel of the multigrid solve) inside a whole pipeline: while
-// enabled, each launch outside stream capture is bracketed by two events on
-// its own stream; kernel_timer_stop sums their elapsed times.
+// Timing of the cycle's finest products (mode 8, the smoothing steps, and mode 3,
+// the residual, of a cycle of precision 16) inside a whole pipeline: while enabled, each launch outside stream
+// capture is bracketed by two events on its own stream; kernel_timer_stop sums
+// their elapsed times.
 namespace {
 struct CycleTimer {
     bool on = false;
@@ -1435,12 +1435,9 @@ static int sell3h_go(hipStream_t st, const Sell3& A, const __half* val, const fl
     return nblk;
 }
 
-void launch_sell3_h(hipStream_t st, int mode, const Sell3& A, const __half* val, const float* dinv32, const float* x,
-                    float* y, const float* f) {
-    if (mode != 3) {
-        sell3h_go<0>(st, A, val, dinv32, x, y, f, nullptr, ChebStep());
-        return;
-    }
+// go() between two events while the cycle's products are timed
+template <typename F>
+static void timed_product(hipStream_t st, F go) {
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (g_cycle_timer.on) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -1450,8 +1447,17 @@ void launch_sell3_h(hipStream_t st, int mode, const Sell3& A, const __half* val,
             if (e0 && e1) (void)hipEventRecord(e0, st);
         }
     }
-    sell3h_go<3>(st, A, val, dinv32, x, y, f, nullptr, ChebStep());
+    go();
     if (e0 && e1) (void)hipEventRecord(e1, st);
+}
+
+void launch_sell3_h(hipStream_t st, int mode, const Sell3& A, const __half* val, const float* dinv32, const float* x,
+                    float* y, const float* f) {
+    if (mode != 3) {
+        sell3h_go<0>(st, A, val, dinv32, x, y, f, nullptr, ChebStep());
+        return;
+    }
+    timed_product(st, [&]() { sell3h_go<3>(st, A, val, dinv32, x, y, f, nullptr, ChebStep()); });
 }
 
 void launch_power_step(hipStream_t st, const Sell3& A, const float* val, const __half* val16, const float* dinv32,
@@ -1464,8 +1470,8 @@ StepParts launch_cheb_step(hipStream_t st, const Sell3& A, const float* val, con
                            const float* x, const float* b, const ChebStep& C, double* partials, double* fold) {
     StepParts P;
     P.p = partials;
-    P.n = val16 ? sell3h_go<8>(st, A, val16, dinv32, x, nullptr, b, partials, C)
-                : sell3_go<float, 8>(st, A, val, x, nullptr, b, partials, nullptr, C);
+    if (val16) timed_product(st, [&]() { P.n = sell3h_go<8>(st, A, val16, dinv32, x, nullptr, b, partials, C); });
+    else P.n = sell3_go<float, 8>(st, A, val, x, nullptr, b, partials, nullptr, C);
     return C.q ? folded(st, P, 1, fold) : StepParts();
 }
 

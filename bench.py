@@ -310,12 +310,15 @@ def main():
     copy_gbs = 2 * copy_bytes / (ms_copy * 1e-3) / 1e9
     log(f"SpMV fp32 {ms32 * 1e3:.1f} us ({gbs32:.0f} GB/s), fp64 {ms64 * 1e3:.1f} us ({gbs64:.0f} GB/s); "
         f"copy {copy_gbs:.0f} GB/s")
-    # the timed step's leading kernel, timed inside the pipeline: the
-    # multigrid cycle's finest operator product with residual epilogue (y = f - K x),
-    # HIP events around each of its launches on the context stream during one
-    # more step run with graphs off.  On this mesh of translated elements it
-    # comes from the reference blocks: per node 27 int32 neighbours, 8 FP32
-    # weights, x, f and y once each
+    # the timed step's leading kernels, timed inside the pipeline: the
+    # multigrid cycle's finest operator products, 2 x degree a cycle, HIP events
+    # around each of their launches on the context stream during one more step
+    # run with graphs off.  On this mesh of translated elements they come from
+    # the reference blocks: per node 27 int32 neighbours, 8 FP32 weights, x and f
+    # once each; the residual writes y; a block-Jacobi smoothing step (all but one
+    # of a cycle's, where the network has stepped aside) reads the 3x3 inverse and
+    # the direction and writes the direction and the new iterate, a cycle's last
+    # also reads q for a dot product
     cyc = None
     if pc != api.PC_JACOBI:
         ctx.set_graphs(False)
@@ -324,11 +327,18 @@ def main():
         n_cyc, ms_cyc = ctx.cycle_spmv_timing(False)
         ctx.set_graphs(True)
         if n_cyc:
-            cyc_bytes = n_rows * (27 + 8) * 4 + prob.n_dof * 4 * 3
+            table = n_rows * (27 + 8) * 4
+            residual = table + prob.n_dof * 4 * 3
+            step = table + n_rows * 9 * 4 + prob.n_dof * 4 * 5
+            steps = 0 if tuning["learned_active"] else 2 * tuning["cheb_degree"] - 1
+            mean = lambda r, s: None if r is None or s is None else int((r + steps * s) / (1 + steps))
+            cyc_bytes = mean(residual + (prob.n_dof * 4 if steps else 0), step)
             cyc_ms = ms_cyc / n_cyc
+            traffic = lambda key: measured_traffic(f"traffic_bytes_per_launch_{key}", "uni3_c2_pmc.md")
             cyc = {"launches": n_cyc, "avg_ms": cyc_ms, "bytes_per_launch": cyc_bytes,
-                   "achieved": cyc_bytes / (cyc_ms * 1e-3) / 1e9}
-            log(f"cycle product in the pipeline: {n_cyc} launches, {cyc_ms * 1e3:.2f} us each, "
+                   "achieved": cyc_bytes / (cyc_ms * 1e-3) / 1e9, "steps": steps,
+                   "traffic": mean(traffic("residual"), traffic("step"))}
+            log(f"cycle products in the pipeline: {n_cyc} launches, {cyc_ms * 1e3:.2f} us each, "
                 f"{cyc['achieved']:.0f} GB/s")
 
     c2 = (args.nx, args.ny, args.nz) == (200, 40, 40)
@@ -377,9 +387,10 @@ def main():
         "wall_s_timed": wall,
         "roofline": ({"bound": "hbm", "achieved": cyc["achieved"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                       "frac": cyc["achieved"] / HBM_PEAK_GBS,
-                      "traffic": None,
-                      "kernel": "k_uni3<float, 3> cycle product from the reference blocks, y = f - K x (timed "
-                                "inside the pipeline)",
+                      "traffic": cyc["traffic"] if c2 else None,
+                      "kernel": f"cycle products from the reference blocks, mean of {cyc['steps']} smoothing steps "
+                                "(k_uni3<float, 8>) and the residual (k_uni3<float, 3>) a cycle (timed inside the "
+                                "pipeline)",
                       "bytes_per_launch": cyc["bytes_per_launch"], "avg_ms": cyc["avg_ms"],
                       "launches_per_step": cyc["launches"]} if cyc else
                      {"bound": "hbm", "achieved": gbs32, "peak": HBM_PEAK_GBS, "unit": "GB/s",

@@ -326,10 +326,12 @@ int asend_solve(asend_ctx* ctx, const double* rhs, double* x, const asend_solve_
                 asend_solve_stats* stats);
 
 /* Measurement (no reference counterpart): with enable = 1, every launch of
- * the multigrid cycle's FP16 SpMV with residual epilogue that is not being
- * captured into a graph is bracketed by HIP events on its stream; enable = 0
- * stops and returns the number of launches and their summed kernel time.
- * For timing that kernel inside a whole pipeline (run it with graphs off). */
+ * the multigrid cycle's finest-level operator product (a block-Jacobi smoothing
+ * step holds its residual's; the residual before the coarse correction) that is
+ * not being captured into a graph is bracketed by HIP events on its stream;
+ * enable = 0 stops and returns the number of launches (2 x Chebyshev degree a
+ * cycle) and their summed kernel time.  Cycle precision 16 only.
+ * For timing them inside a whole pipeline (run it with graphs off). */
 int asend_cycle_spmv_timing(asend_ctx* ctx, int enable, int64_t* launches, double* total_ms);
 
 /* LDL^T factor of the assembled K_eff restricted to diagonal blocks of
@@ -741,7 +743,8 @@ int asend_mg_set_smoother(asend_ctx* ctx, int kind, int degree, double lo_frac, 
  * reads an FP16 copy of the operator whose rows are scaled by their diagonal
  * (entries O(1) whatever the moduli and penalty), FP32 accumulation, for the
  * smoothing and restriction residuals and the smoother bounds; 32 reads the
- * FP32 operator.  The flexible CG around the cycle keeps its FP32 operator
+ * FP32 operator.  On meshes of translated elements both take the FP32 products
+ * from the reference blocks.  The flexible CG around the cycle keeps its FP32 operator
  * products and the FP64 residual refreshes decide convergence either way. */
 int asend_mg_set_cycle_precision(asend_ctx* ctx, int bits);
 
