@@ -259,15 +259,15 @@ __device__ __forceinline__ void tile_rows_abt(const double* __restrict__ sA, con
 }
 
 // Step k, panel: L_Ik = A_Ik L_kk^-T D_k^-1 for the tiles below the diagonal
-// (blockIdx.x = I - k - 1).
+// (blockIdx.y = I - k - 1).
 //
 // Panel and update are bound by the latency of one tile product per workgroup
 // (a band of 9 tiles gives 9 and 45 of them): both operand tiles are loaded
 // into registers at once (one exposed latency instead of one per loop turn)
 // and multiplied on the matrix cores.
 __global__ __launch_bounds__(kBlock) void k_ldl_panel(LdlDesc d, int k, double* __restrict__ L) {
-    const int blk = blockIdx.y;
-    const int I = k + 1 + blockIdx.x;
+    const int blk = blockIdx.x;
+    const int I = k + 1 + blockIdx.y;
     if (I >= ldl_block_nt(d, blk)) return;
     __shared__ __align__(16) double sA[kLdlTile * kLm];
     __shared__ __align__(16) double sB[kLdlTile * kLm];
@@ -296,7 +296,7 @@ __global__ __launch_bounds__(kBlock) void k_ldl_panel(LdlDesc d, int k, double* 
 }
 
 // Step k, trailing update of the band: A_IJ -= L_Ik D_k L_Jk^T for
-// k < J <= I <= k + wt (blockIdx.x enumerates the pairs row by row).  The
+// k < J <= I <= k + wt (blockIdx.y enumerates the pairs row by row).  The
 // workgroup of the first pair holds the next diagonal tile once updated and
 // factors it at once: one launch and one tile round trip less on the chain
 // from a diagonal tile to the next.
@@ -307,8 +307,8 @@ __global__ __launch_bounds__(kBlock) void k_ldl_panel(LdlDesc d, int k, double* 
 // and update (18) tiles staged one load at a time and multiplied on the VALU.
 __global__ __launch_bounds__(kBlock) void k_ldl_update(LdlDesc d, int k, double* __restrict__ L,
                                                        int32_t* __restrict__ neg) {
-    const int blk = blockIdx.y;
-    const int q = blockIdx.x;
+    const int blk = blockIdx.x;
+    const int q = blockIdx.y;
     int pi = (int)((std::sqrt(8.0 * q + 1.0) - 1.0) * 0.5);
     while ((pi + 1) * (pi + 2) / 2 <= q) ++pi;
     while (pi * (pi + 1) / 2 > q) --pi;
@@ -451,14 +451,16 @@ __device__ __forceinline__ double rows_sum(double (&a)[N]) {
 //   forward  z_s = Li_s y_s, w_s = z_s / d;  y_K -= sum_J L_KJ z_J below
 //   backward x_s = Li_s^T w_s;               w_J -= sum_I L_IJ^T x_I above
 // A workgroup of 4 wavefronts owns 16 rows (columns) of one tile row
-// (column).  Every entry is written by one workgroup per launch and read by
+// (column); the blocks are the grid's x, which takes any number of them (y ends at
+// 65,536: one node a block reaches that on 65,537 nodes).  Every entry is written by one workgroup per launch and read by
 // none of the same launch, so the result is deterministic.
 //
 // Bound by the factor's bytes, read twice, on many blocks and by the launches
 // on few.  One CU streams tiles at only 20-45 GB/s here, so a step is spread
-// over many workgroups: 58 blocks of 720 DOFs take 57 us a solve (5.2 TB/s of
-// factor) against 118 us with one workgroup per block and 331 us with one
-// launch per tile row and substitutions; one block of 31,248 DOFs, band 552,
+// over many workgroups: 58 blocks of 720 DOFs take 45 us a solve (6.6 TB/s of
+// factor; 56 us with the blocks in the grid's y, a block's long and short rows
+// dispatched together) against 118 us with one workgroup per block and 331 us
+// with one launch per tile row and substitutions; one block of 31,248 DOFs, band 552,
 // 1.28 ms in 245 launches against 13.5 ms in 978.
 
 // Rows row0.. (4 of them) of tiles (I, ja..jb - 1) times the vector v (the
@@ -530,11 +532,11 @@ __global__ __launch_bounds__(kBlock) void k_ldl_fwd_diag(LdlDesc d, const double
                                                          const double* __restrict__ y, double* __restrict__ z,
                                                          double* __restrict__ w, const int* __restrict__ done) {
     if (done && *done) return;
-    const int blk = blockIdx.y, nt = ldl_block_nt(d, blk);
-    const int I = sb * S + (blockIdx.x >> 2);
+    const int blk = blockIdx.x, nt = ldl_block_nt(d, blk);
+    const int I = sb * S + (blockIdx.y >> 2);
     if (I >= nt) return;
     const int64_t s = (int64_t)blk * d.bs, m = std::min(d.bs, d.n - s);
-    const int c = threadIdx.x & 63, row0 = 16 * (blockIdx.x & 3) + 4 * (threadIdx.x >> 6);
+    const int c = threadIdx.x & 63, row0 = 16 * (blockIdx.y & 3) + 4 * (threadIdx.x >> 6);
     const double* TI = L + ldl_tile(d, blk, I, I);
     double li[4];
 #pragma unroll
@@ -560,11 +562,11 @@ __global__ __launch_bounds__(kBlock) void k_ldl_fwd_band(LdlDesc d, const double
                                                          const double* __restrict__ z, double* __restrict__ y,
                                                          const int* __restrict__ done) {
     if (done && *done) return;
-    const int blk = blockIdx.y, nt = ldl_block_nt(d, blk);
-    const int K = (sb + 1) * S + (blockIdx.x >> 2);
+    const int blk = blockIdx.x, nt = ldl_block_nt(d, blk);
+    const int K = (sb + 1) * S + (blockIdx.y >> 2);
     if (K >= nt) return;
     const int64_t s = (int64_t)blk * d.bs, m = std::min(d.bs, d.n - s);
-    const int c = threadIdx.x & 63, row0 = 16 * (blockIdx.x & 3) + 4 * (threadIdx.x >> 6);
+    const int c = threadIdx.x & 63, row0 = 16 * (blockIdx.y & 3) + 4 * (threadIdx.x >> 6);
     double acc[4] = {};
     rows_dot(d, L, blk, K, max(sb * S, K - d.wt), (sb + 1) * S, row0, z + s, m, acc);
     const double v = rows_sum<4>(acc);
@@ -577,11 +579,11 @@ __global__ __launch_bounds__(kBlock) void k_ldl_bwd_diag(LdlDesc d, const double
                                                          const double* __restrict__ w, double* __restrict__ x,
                                                          const int* __restrict__ done) {
     if (done && *done) return;
-    const int blk = blockIdx.y, nt = ldl_block_nt(d, blk);
-    const int J = sb * S + (blockIdx.x >> 2);
+    const int blk = blockIdx.x, nt = ldl_block_nt(d, blk);
+    const int J = sb * S + (blockIdx.y >> 2);
     if (J >= nt) return;
     const int64_t s = (int64_t)blk * d.bs, m = std::min(d.bs, d.n - s);
-    const int l = threadIdx.x & 63, c0 = 16 * (blockIdx.x & 3), r0 = 16 * (threadIdx.x >> 6) + (l >> 4);
+    const int l = threadIdx.x & 63, c0 = 16 * (blockIdx.y & 3), r0 = 16 * (threadIdx.x >> 6) + (l >> 4);
     const int col = c0 + (l & 15);
     // the diagonal tile: ones where it holds D
     double a[4], v[4];
@@ -605,11 +607,11 @@ __global__ __launch_bounds__(kBlock) void k_ldl_bwd_band(LdlDesc d, const double
                                                          const double* __restrict__ x, double* __restrict__ w,
                                                          const int* __restrict__ done) {
     if (done && *done) return;
-    const int blk = blockIdx.y, nt = ldl_block_nt(d, blk);
-    const int J = sb * S - 1 - (int)(blockIdx.x >> 2);
+    const int blk = blockIdx.x, nt = ldl_block_nt(d, blk);
+    const int J = sb * S - 1 - (int)(blockIdx.y >> 2);
     if (J < 0 || sb * S >= nt) return;
     const int64_t s = (int64_t)blk * d.bs, m = std::min(d.bs, d.n - s);
-    const int c0 = 16 * (blockIdx.x & 3);
+    const int c0 = 16 * (blockIdx.y & 3);
     const int ib = min(min((sb + 1) * S, nt), J + d.wt + 1);
     const double v = cols_total(cols_dot(d, L, blk, J, sb * S, ib, c0, x + s, m));
     const int64_t g = (int64_t)J * kLdlTile + c0 + threadIdx.x;
@@ -673,8 +675,8 @@ void ldl_factor_launch(hipStream_t st, const LdlDesc& d, double* L, double* tmp,
     for (int k = 0; k < d.nt_full; ++k) {
         const int r = std::min(d.wt, d.nt_full - 1 - k);
         if (r <= 0) continue;
-        hipLaunchKernelGGL(k_ldl_panel, dim3(r, d.n_blocks), dim3(kBlock), 0, st, d, k, L);
-        hipLaunchKernelGGL(k_ldl_update, dim3(r * (r + 1) / 2, d.n_blocks), dim3(kBlock), 0, st, d, k, L, neg);
+        hipLaunchKernelGGL(k_ldl_panel, dim3(d.n_blocks, r), dim3(kBlock), 0, st, d, k, L);
+        hipLaunchKernelGGL(k_ldl_update, dim3(d.n_blocks, r * (r + 1) / 2), dim3(kBlock), 0, st, d, k, L, neg);
     }
     ldl_invert_launch(st, d, L, tmp);
 }
@@ -718,7 +720,7 @@ void ldl_solve_launch(hipStream_t st, const LdlDesc& d, const double* L, const d
     const int S = ldl_super(d);
     const int ns = (d.nt_full + S - 1) / S;
     double *w = work, *y = work + d.n, *z = work + 2 * d.n;
-    const dim3 diag(4 * S, d.n_blocks);
+    const dim3 diag(d.n_blocks, 4 * S);
     if (ns == 1) {
         hipLaunchKernelGGL(k_ldl_fwd_diag, diag, dim3(kBlock), 0, st, d, L, S, 0, b, (double*)nullptr, w, done);
         hipLaunchKernelGGL(k_ldl_bwd_diag, diag, dim3(kBlock), 0, st, d, L, S, 0, w, x, done);
@@ -729,14 +731,14 @@ void ldl_solve_launch(hipStream_t st, const LdlDesc& d, const double* L, const d
         hipLaunchKernelGGL(k_ldl_fwd_diag, diag, dim3(kBlock), 0, st, d, L, S, s, y, z, w, done);
         const int rows = std::min(d.wt, d.nt_full - (s + 1) * S);
         if (rows > 0)
-            hipLaunchKernelGGL(k_ldl_fwd_band, dim3(4 * rows, d.n_blocks), dim3(kBlock), 0, st, d, L, S, s, z, y,
+            hipLaunchKernelGGL(k_ldl_fwd_band, dim3(d.n_blocks, 4 * rows), dim3(kBlock), 0, st, d, L, S, s, z, y,
                                done);
     }
     for (int s = ns - 1; s >= 0; --s) {
         hipLaunchKernelGGL(k_ldl_bwd_diag, diag, dim3(kBlock), 0, st, d, L, S, s, w, x, done);
         const int cols = std::min(d.wt, s * S);
         if (cols > 0)
-            hipLaunchKernelGGL(k_ldl_bwd_band, dim3(4 * cols, d.n_blocks), dim3(kBlock), 0, st, d, L, S, s, x, w,
+            hipLaunchKernelGGL(k_ldl_bwd_band, dim3(d.n_blocks, 4 * cols), dim3(kBlock), 0, st, d, L, S, s, x, w,
                                done);
     }
 }

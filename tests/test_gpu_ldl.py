@@ -73,6 +73,28 @@ def test_super_block_edges(ctx, mesh, blocks):
         assert rel_err(x, x_ref) <= 1e-10, rel_err(x, x_ref)
 
 
+def test_more_blocks_than_a_grid_row_holds(ctx):
+    """One node a block on 68,160 nodes: more blocks than the 65,536 that the
+    second dimension of a launch takes."""
+    gpu_case("ldl 68,160 blocks of one node")
+    p = problems.heterogeneous(70, 31, 29, seed=2, block_dim=48)
+    problems.upload(ctx, p)
+    ctx.assemble()
+    info = ctx.ldl_factor(3)
+    assert info["n_blocks"] == p.n_dof // 3 == 68160 and info["pos_def"] == 1
+    rp, cols, vals = ctx.get_matrix()
+    b = np.random.default_rng(8).standard_normal(p.n_dof)
+    x = ctx.ldl_solve(b)
+    ctx.ldl_release()
+    row = np.repeat(np.arange(p.n_dof), np.diff(rp))
+    d = row // 3 == cols // 3
+    D = np.zeros((p.n_dof // 3, 3, 3))
+    D[row[d] // 3, row[d] % 3, cols[d] % 3] = vals[d]
+    ref = np.linalg.solve(D, b.reshape(-1, 3, 1)).reshape(-1)
+    # condition number of a node's block below 1e6 (penalised DOFs beside free ones)
+    assert (np.abs(x - ref) <= 1e-9 * np.abs(ref.reshape(-1, 3)).max(axis=1).repeat(3)).all()
+
+
 def test_direct_solve_is_exact(ctx):
     p = solid("het-12x6x6 distorted")
     gpu_case("direct solve het-12x6x6 distorted")
