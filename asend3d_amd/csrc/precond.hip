@@ -206,8 +206,7 @@ struct Multigrid {
         const float* val0 = nullptr;  // finest-level operator values
         const float* b = nullptr;
         float* x = nullptr;
-        const float* ls = nullptr;
-        const float* lst = nullptr;
+        Factor factor;  // every array of it that the launches hold
         uint64_t use = 0;
     };
     FcgGraph graphs[4];
@@ -235,6 +234,11 @@ struct Multigrid {
 };
 
 namespace {
+
+bool same_factor(const Factor& a, const Factor& b) {
+    return a.n == b.n && a.n_edge == b.n_edge && a.Ls == b.Ls && a.LsT == b.LsT && a.enb == b.enb && a.erev == b.erev &&
+           a.Ls16 == b.Ls16 && a.LsT16 == b.LsT16 && a.sc16 == b.sc16 && a.scT16 == b.scT16;
+}
 
 // whether the finest products come from the mesh's reference blocks (the
 // captured graphs hold the choice)
@@ -1842,9 +1846,7 @@ int mg_learned_bound_begin(Multigrid* mg, hipStream_t st, const Factor& F, const
     // replay as one graph while the factor storage, the operator and the
     // SpMV geometry stay where they were captured.
     if (mg->use_graphs) {
-        const Factor& P = mg->pw_factor;
-        const bool same = mg->pw_exec && P.n == F.n && P.n_edge == F.n_edge && P.Ls == F.Ls && P.LsT == F.LsT &&
-                          P.enb == F.enb && P.erev == F.erev && mg->pw_val == d_K32 &&
+        const bool same = mg->pw_exec && same_factor(mg->pw_factor, F) && mg->pw_val == d_K32 &&
                           mg->pw_waves == mg->fine.waves_per_block && mg->pw_half == (int)cycle_half(mg) &&
                           mg->pw_uni == fine_uni(mg);
         if (!same) {
@@ -2167,13 +2169,12 @@ int mg_fcg_solve(Multigrid* mg, hipStream_t st, const float* b, float* x, double
     };
     Multigrid::FcgGraph* gr = nullptr;
     if (mg->use_graphs) {
-        const float* ls = mg->has_factor ? mg->factor.Ls : nullptr;
-        const float* lst = mg->has_factor ? mg->factor.LsT : nullptr;
+        const Factor factor = mg->has_factor ? mg->factor : Factor();
         for (auto& g : mg->graphs)
             if (g.exec && g.precond == precond && g.fine_smoother == mg->fine_smoother && g.check == check_every &&
-                g.degree == mg->cheb_degree && g.kind == mg->smoother_kind && g.b == b && g.x == x && g.ls == ls &&
-                g.lst == lst && g.waves == mg->fine.waves_per_block && g.uni == fine_uni(mg) && g.val0 == l0.d_val &&
-                g.half == (int)cycle_half(mg))
+                g.degree == mg->cheb_degree && g.kind == mg->smoother_kind && g.b == b && g.x == x &&
+                same_factor(g.factor, factor) && g.waves == mg->fine.waves_per_block && g.uni == fine_uni(mg) &&
+                g.val0 == l0.d_val && g.half == (int)cycle_half(mg))
                 gr = &g;
         if (!gr) {
             // capture into the least recently used slot
@@ -2204,8 +2205,7 @@ int mg_fcg_solve(Multigrid* mg, hipStream_t st, const float* b, float* x, double
             gr->kind = mg->smoother_kind;
             gr->b = b;
             gr->x = x;
-            gr->ls = ls;
-            gr->lst = lst;
+            gr->factor = factor;
             gr->waves = mg->fine.waves_per_block;
             gr->uni = fine_uni(mg);
             gr->val0 = l0.d_val;

@@ -201,6 +201,36 @@ def test_new_constraints_between_solves(precond):
     old.close()
 
 
+def test_new_network_between_solves():
+    """A network made anew after solves with captured iterations, its arrays in
+    other places (some of the old ones taken by another context's)."""
+    gpu_case("network made anew between solves")
+    dims = (17, 7, 6)
+    p = problems.heterogeneous(*dims, seed=6, sigma_ln=0.7)
+    o = api.Context.opts(api.SOLVE_IR_MIXED, api.PC_LEARNED, tol=1e-9, inner_tol=1e-3, max_it=2000, check_every=3)
+
+    def make(seed):
+        c = api.Context(0)
+        c.learned_init(seed)
+        problems.upload(c, p)
+        c.set_grid(*dims)
+        c.assemble()
+        c.learned_train(4, seed=3)
+        return c
+
+    old = make(1)
+    old.solve(p.f, o)
+    old.learned_init(2)
+    new = make(2)
+    old.learned_train(4, seed=3)
+    for _ in range(2):
+        (u, st), (u_new, st_new) = old.solve(p.f, o), new.solve(p.f, o)
+        assert st.converged and st.fallback_used == 0 and st.iterations == st_new.iterations
+        assert np.array_equal(u, u_new)
+    new.close()
+    old.close()
+
+
 @pytest.mark.parametrize("mode", [api.NM_FP64, api.NM_MIXED])
 def test_new_constraints_between_newmark_runs(mode):
     """The same of Newmark steps, whose captured launches also outlive a change
