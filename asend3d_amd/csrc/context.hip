@@ -1159,40 +1159,6 @@ void uni_set(asend_ctx* ctx, int i, double k_scale, double c_mass, const double*
     }
 }
 
-// Tables of the reference-block products for the slices of a mesh (conn_r:
-// block-row ranks), if its nodes are one lattice: at most one element per
-// local position of a node, and the same node at the same offset of a node
-// from all of its elements.
-bool uni_tables(int64_t n_nodes, int64_t n_el, const std::vector<int32_t>& conn_r, std::vector<int32_t>& nbr,
-                std::vector<int32_t>& el) {
-    static const int pos[8][3] = {{0, 0, 0}, {1, 0, 0}, {1, 1, 0}, {0, 1, 0}, {0, 0, 1}, {1, 0, 1}, {1, 1, 1}, {0, 1, 1}};
-    const int64_t ns = (n_nodes + 63) / 64;
-    nbr.assign(27 * 64 * ns, -1);
-    el.assign(8 * 64 * ns, -1);
-    for (int64_t e = 0; e < n_el; ++e)
-        for (int a = 0; a < 8; ++a) {
-            const int64_t r = conn_r[8 * e + a], s = r >> 6, l = r & 63;
-            int32_t& slot = el[64 * (8 * s + a) + l];
-            if (slot >= 0) return false;
-            slot = (int32_t)e;
-            for (int b = 0; b < 8; ++b) {
-                const int o = (pos[b][0] - pos[a][0] + 1) + 3 * (pos[b][1] - pos[a][1] + 1) +
-                              9 * (pos[b][2] - pos[a][2] + 1);
-                int32_t& c = nbr[64 * (27 * s + o) + l];
-                const int32_t v = conn_r[8 * e + b];
-                if (c >= 0 && c != v) return false;
-                c = v;
-            }
-        }
-    for (int64_t s = 0; s < ns; ++s)
-        for (int o = 0; o < 27; ++o)
-            for (int64_t l = 0; l < 64; ++l) {
-                int32_t& c = nbr[64 * (27 * s + o) + l];
-                if (c < 0) c = (int32_t)std::min(64 * s + l, n_nodes - 1);
-            }
-    return true;
-}
-
 bool all_equal(const double* v, int64_t n) {
     for (int64_t i = 1; i < n; ++i)
         if (v[i] != v[0]) return false;
@@ -1764,20 +1730,30 @@ int asend_upload_mesh(asend_ctx* ctx, int elem_type, int64_t n_mesh_nodes, const
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(ctx->st));
         ctx->uniform_hex = true;
-        std::vector<int32_t> nbr, el;
-        if (uni_tables(n_nodes, n_el, conn_r, nbr, el)) {
-            const size_t ns = (size_t)ctx->n_slices;
-            if ((rc = dalloc(ctx, &ctx->d_uni_nbr, nbr.size())) || (rc = dalloc(ctx, &ctx->d_uni_el, el.size())) ||
-                (rc = dalloc(ctx, &ctx->d_uni_pslot, ns)) || (rc = dalloc(ctx, &ctx->d_uni_pen64, 192 * ns)) ||
-                (rc = dalloc(ctx, &ctx->d_uni_pen32, 192 * ns)))
+        // the reference-block products, if the nodes are one lattice
+        const size_t ns = (size_t)ctx->n_slices;
+        int32_t torn = 0;
+        if ((rc = dalloc(ctx, &ctx->d_uni_nbr, 27 * 64 * ns)) || (rc = dalloc(ctx, &ctx->d_uni_el, 8 * 64 * ns)) ||
+            (rc = dalloc(ctx, &ctx->d_uni_pslot, ns)))
+            return rc;
+        HIPCHK(hipMemsetAsync(ctx->d_uni_pslot, 0, 4, ctx->st));
+        launch_uni_tables(ctx->st, (int)n_nodes, (int)ns, ctx->d_n2e_ptr, ctx->d_n2rec, ctx->d_conn_r, ctx->d_uni_nbr,
+                          ctx->d_uni_el, ctx->d_uni_pslot);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(&torn, ctx->d_uni_pslot, 4, hipMemcpyDeviceToHost, ctx->st));
+        HIPCHK(hipMemsetAsync(ctx->d_uni_pslot, 0xff, ns * 4, ctx->st));  // no penalties
+        HIPCHK(hipStreamSynchronize(ctx->st));
+        if (torn) {
+            dfree(ctx->d_uni_nbr);
+            dfree(ctx->d_uni_el);
+            dfree(ctx->d_uni_pslot);
+        } else {
+            if ((rc = dalloc(ctx, &ctx->d_uni_pen64, 192 * ns)) || (rc = dalloc(ctx, &ctx->d_uni_pen32, 192 * ns)))
                 return rc;
             for (auto& b : ctx->uni_bufs)
                 if ((rc = dalloc(ctx, &b.w64, 512 * ns)) || (rc = dalloc(ctx, &b.w32, 512 * ns)) ||
                     (rc = dalloc(ctx, &b.kh64, kUniCoefs)) || (rc = dalloc(ctx, &b.kh32, kUniCoefs)))
                     return rc;
-            HIPCHK(hipMemcpy(ctx->d_uni_nbr, nbr.data(), nbr.size() * 4, hipMemcpyHostToDevice));
-            HIPCHK(hipMemcpy(ctx->d_uni_el, el.data(), el.size() * 4, hipMemcpyHostToDevice));
-            HIPCHK(hipMemset(ctx->d_uni_pslot, 0xff, ns * 4));  // no penalties
             ctx->e_const = all_equal(E, n_el);
             ctx->e_first = E[0];
             ctx->rho_const = !rho || all_equal(rho, n_el);

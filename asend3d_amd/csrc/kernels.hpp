@@ -136,6 +136,11 @@ void launch_to_f32(hipStream_t st, const double* a, float* b, int64_t n);
 void launch_diag_inv(hipStream_t st, int n_rows, const int32_t* sptr, const int32_t* kdiag, const double* K,
                      double* d64, float* d32);
 
+// Neighbours and elements of a lattice's rows by slice (UniOp::nbr, and the element
+// at each local position, -1 where there is none) from the node -> element lists
+// n2rec (8 e + a); *torn is set where the nodes are not one lattice.
+void launch_uni_tables(hipStream_t st, int n_rows, int n_slices, const int32_t* n2e_ptr, const int32_t* n2rec,
+                       const int32_t* conn_r, int32_t* nbr, int32_t* el, int32_t* torn);
 // Tables of a reference-block operator: weights (scale times E per element,
 // or times 1 where E is null), and kUniCoefs entries: the blocks sK Khat + sM
 // Mhat I and their rows' sums over b (sM sum Mhat_ab), in FP64 and FP32.
