@@ -754,7 +754,11 @@ int residual64(asend_ctx* ctx, const double* f, const double* u, double* r) {
 constexpr int64_t kLearnedInnerBudget = 300;
 constexpr int kNewmarkBlock = 16;  // PCG iterations per long captured block of a Newmark step
 constexpr int kMixedRefreshEvery = 4;  // mixed step solver: iterations between reliable-update slots
-// ASEND_NM_AUTO takes the mixed step solver above this FP64 operator size
+// ASEND_NM_AUTO takes the mixed step solver above this FP64 operator size, 69,000
+// nodes of a lattice.  A step, FP64 / mixed, where the products read the operator
+// (a modulus per element) and where they come from the reference blocks: 44,541
+// nodes 803 / 822 us and 723 / 770 us, 75,625 nodes 1,214 / 1,024 us and
+// 1,189 / 1,111 us.
 constexpr int64_t kMixedAutoBytes = 128ll << 20;
 constexpr int64_t kLearnedPcgBudget = 20000;
 
@@ -3567,7 +3571,9 @@ int asend_autotune(asend_ctx* ctx, const double* rhs, int what, asend_tuning* ou
     int rc;
     if (what & ASEND_TUNE_SPMV) {
         // SpMV workgroup geometry: 1, 2, 4 or 8 slices per workgroup, timed
-        // with HIP events on the context stream (FP32 decides, FP64 reported)
+        // with HIP events on the context stream (FP32 decides, FP64 reported).
+        // It is the assembled values' product: on a mesh of translated elements
+        // only asend_spmv and the learned factor alone use it.
         double best = 1e300;
         int best_w = ctx->spmv_wpb;
         for (int k = 0; k < 4; ++k) {

@@ -1,12 +1,10 @@
 // HIP kernels of the solve path for gfx950 (MI355X).
 //
-// Operator storage: node-block CSR ("BSR") with b x b blocks (b = DOFs per
-// node).  Block row r holds the blocks of the nodes coupled to node r (sorted
-// by node rank); within a block row, values are component-major:
-//   value(block k of row r, component c = b*i + j) = val[b*b*rp[r] + c*nb_r + k]
-// with nb_r = rp[r+1] - rp[r].  A group of G lanes sweeps one block row, so
-// every value load is a unit-stride burst, and the column index is read once
-// per b*b values (4 B per 9 values for b = 3 instead of 4 B per value).
+// Operator storage: 3x3 blocks in sliced ELL (k_sell3): 64-row slices, a lane
+// per block row, its blocks sorted by node rank; slot k of lane l has its column
+// at scol[64 k + l] and component c = 3 i + j of its value at
+// val[64 (9 k + c) + l].  On meshes of translated elements the solves' products
+// come from the reference blocks instead (k_uni3).
 #include <hip/hip_runtime.h>
 
 #include "device_common.hpp"
@@ -984,10 +982,13 @@ __global__ __launch_bounds__(kSellMaxWaves * kWave) void k_sell3(int n_rows, int
 // slice reads each neighbour once instead of 1.6 times but holds all 81
 // values at once (256 registers, one wavefront per SIMD): 52 us against 30 us
 // on 200x40x40 in FP64.  Assembled values against this, p.Kp included:
-//   525 nodes FP64 12.9 / 5.0 us, 44,541 nodes FP64 14.8 / 7.7 us,
-//   337,881 nodes FP64 136 / 29.6 us, FP32 65 / 18 us, cycle (FP16) 38 / 17.7 us,
-// so it is taken wherever the tables exist.  The large ones are bound by the
-// 26 gathers of 24 (12) scattered bytes per lane.
+//   525 nodes FP64 12.9 / 5.3 us, 44,541 nodes FP64 14.8 / 8.6 us,
+//   337,881 nodes FP64 136 / 32.6 us, FP32 66 / 22.3 us, the cycle's residual
+//   (FP16 values) 38 / 20.0 us (kernel traces inside the solves; launched back to
+//   back on the same vectors the last four take 29.6, 18 and 17.7 us),
+// so it is taken wherever the tables exist.  The large ones move 1.04 to 1.07
+// times the bytes they have to, at 1.9 to 3.3 TB/s: they are bound by the L1,
+// whose accesses for the 26 scattered gathers take 83 to 93% of its cycles.
 // ---------------------------------------------------------------------------
 constexpr int kUniWaves = 4;  // wavefronts per slice
 
@@ -1717,7 +1718,7 @@ __global__ __launch_bounds__(kBlock) void k_cg1_update(int64_t n, const T* __res
 
 // Flexible Jacobi PCG (one truncation vector): alpha = p.r / p.q (launch_sell3
 // mode 7), x += alpha p, r -= alpha q, beta = -(Dinv r).q / p.q, then
-// p = Dinv r + beta p (launch_pcg_dir).  Fresh inner products every
+// p = Dinv r + beta p (launch_fpcg_dir).  Fresh inner products every
 // iteration, so a residual replaced by a reliable update needs no repair.
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_fpcg_update(int64_t n, const T* __restrict__ dinv, T* __restrict__ x,

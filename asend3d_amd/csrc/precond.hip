@@ -2128,10 +2128,12 @@ int mg_fcg_solve(Multigrid* mg, hipStream_t st, const float* b, float* x, double
         return hipSuccess;
     };
     MGCHK(start());
-    // The learned factor alone is measured against its own untrained start
-    // (block Jacobi) on the assembled FP32 values both are built from: 1,368
-    // against 1,648 iterations on 40x8x8.  With the reference blocks' more
-    // exact products block Jacobi takes 1,051 and the trained factor 1,107.
+    // The learned factor alone stays on the assembled FP32 values that it is
+    // built from, the operator its gain over block Jacobi (its untrained start)
+    // is stated for: 1,317 against 1,644 iterations on 40x8x8, 46 ms against 60.
+    // It is a gain on these values only: on the reference blocks' more exact
+    // products block Jacobi takes 1,051 iterations and 34 ms, the trained factor
+    // 1,172 and 35.  The multigrid, with either smoother, uses those products.
     Sell3 op = mg->fine;
     if (precond == 1) op.n_uni = 0;
     // the V-cycle's first smoothing step rides on the update, z.q on its last
